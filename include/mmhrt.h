@@ -259,8 +259,9 @@ MMHRT_API int32_t mmhrt_get_timings(mmhrt_ctx ctx, float* times_ms, int32_t n);
 /* Instrumented trace counters of the last render (when enabled with mmhrt_set_option
  * "count_visits"): node visits, sphere tests, rays traced. Also refreshes the options
  * "stack_overflow" (1 if a traversal stack ever exceeded its capacity; 0 expected),
- * "pair_visits" (the node visits that were leaf pairs: two 16-byte spheres read instead of a
- * 64-byte node) and "leaf_fetches" (spheres read for the leaf children of stored nodes). */
+ * "pair_visits" (the node visits that were leaf references: two 16-byte spheres read instead of a
+ * 64-byte node) and "leaf_fetches" (spheres read apart from visits: none by the current kernels).
+ * A visit that a whole wavefront makes together is counted once per active lane. */
 MMHRT_API int32_t mmhrt_get_counters(mmhrt_ctx ctx, uint64_t* node_visits, uint64_t* sphere_tests, uint64_t* rays);
 
 /* ---- batched time series ---------------------------------------------------
@@ -317,7 +318,8 @@ MMHRT_API int32_t mmhrt_denoiser_train_step(mmhrt_ctx ctx, const uint16_t* feats
                                             uint32_t h, uint32_t w, float depth_scale, const float bg[4], float lr,
                                             int32_t apply, float* loss_out, float* grads_out);
 
-/* Tuning knobs (autotuner output): "stack_lds" (LDS stack entries per lane: 8, 16, 24 or 32, default 16),
+/* Tuning knobs (autotuner output): "stack_lds" (LDS words of the traversal stack per lane: 8, 16, 24
+ * or 32, default 16; an entry, a reference and its entry distance, takes two),
  * "tile_w", "tile_h", "persistent" (0/1), "refill" (ballot refill threshold in lanes; -1, the
  * default: 16 for 1-spp frames, 0 otherwise), "blocks_per_cu" (persistent
  * workgroups per CU), "refit_period" (MMHRT_BUILD_AUTO: refits between rebuilds), "build_chunk"

@@ -135,7 +135,7 @@ struct mmhrt_ctx_s {
     mmhrt::DevBuf<uint32_t> counters;  // [0] tile counter, [2..7] visit counters (u64 pairs)
 
     // options
-    int64_t opt_stack_lds = 16;  // 16 leaves the LDS for 7 wavefronts per SIMD
+    int64_t opt_stack_lds = 16;  // LDS words per lane (8 entries): leaves the LDS for 7 wavefronts per SIMD
     int64_t opt_persistent = 1;
     int64_t opt_refill = -1;  // ballot-refill threshold; -1: 16 for 1-spp frames (measured 13% faster), else off
     int64_t opt_count = 0;
@@ -257,8 +257,8 @@ int sort_spheres(mmhrt_ctx_s* c, int bits);
 int build_pkd(mmhrt_ctx_s* c, int bits);
 
 // trace.hip
-constexpr int TRACE_STACK_CAP = 128;                       // traversal stack entries per lane
-constexpr int TRACE_SPILL_PER_LANE = TRACE_STACK_CAP - 8;  // the most any LDS stack depth (>= 8) spills
+constexpr int TRACE_STACK_CAP = 124;                       // traversal stack entries per lane
+constexpr int TRACE_SPILL_PER_LANE = TRACE_STACK_CAP - 4;  // the most any LDS stack depth (>= 4) spills, one word each
 constexpr uint32_t TRACE_CTR_WORDS = 16;                   // tile counter, overflow flag, 5 u64 counters
 struct FrameOutputs {
     float4* color;

@@ -8,11 +8,11 @@
 // reference's one (TEA seed, two LCG draws per sample for the jitter).
 //
 // Traversal: BVH2 with both child boxes in the 64-byte node (four 16-byte loads per visit),
-// ordered front-to-back, leaves tested inline with one 16-byte sphere load; a node over two
-// leaves is not stored and its visit reads the two spheres instead (leaf pairs). The traversal stack
-// keeps its top S entries in LDS (lane-strided, conflict free) and spills deeper entries to a
-// per-lane global region. Closest hit keeps the lowest particle ID among equal t; boxes whose
-// entry distance equals the current best are still visited so that ties resolve the same way
+// ordered front-to-back, the spheres of a leaf reference tested apart from the node visits, two at
+// a time (leaf pairs); the samples of one pixel walk the tree together with scalar loads. The
+// traversal stack keeps its lowest S entries in LDS (lane-strided, conflict free) and spills deeper
+// ones to a per-lane global region. Closest hit keeps the lowest particle ID among equal t; boxes
+// whose entry distance equals the current best are still visited so that ties resolve the same way
 // whatever the visiting order. AO rays stop at the first occluder (any hit).
 #include <float.h>
 
@@ -52,27 +52,44 @@ struct TraceArgs {
     uint32_t tl_log2;        // log2 of the treelet size
 };
 
+// Reference of no node: the bottom of a stack. Not a leaf reference, whose k is below 2^31 - 1.
+constexpr int32_t REF_NONE = INT32_MIN;
+
+// Traversal stack of one lane: (reference, entry distance of its box), the lowest S entries in
+// LDS, lane-interleaved. Deeper entries spill their reference alone to the lane's global words
+// and come back with an entry distance below every ray's (they are visited without the test).
 template <int S>
 struct LaneStack {
-    int32_t* lds;  // element k at lds[k * TB]
+    int2* lds;  // element k at lds[k * TB]
     int32_t* spill;
     uint32_t stride;
     int sp;
     uint32_t* overflow;
-    __device__ __forceinline__ void push(int32_t v) {
-        if (sp < S) {
-            lds[sp * TB] = v;
+    __device__ __forceinline__ void push(int32_t ref, float tn) {
+        if (__builtin_expect(sp < S, 1)) {
+            lds[sp * TB] = make_int2(ref, __float_as_int(tn));
         } else if (sp < STACK_CAP) {
-            spill[(size_t)(sp - S) * stride] = v;
+            spill[(size_t)(sp - S) * stride] = ref;
         } else {
             *overflow = 1u;  // cannot happen for a valid LBVH; recorded, entry dropped
             return;
         }
         ++sp;
     }
-    __device__ __forceinline__ int32_t pop() {
+    // the top entry (the stack is not empty)
+    __device__ __forceinline__ int2 take() {
         --sp;
-        return sp < S ? lds[sp * TB] : spill[(size_t)(sp - S) * stride];
+        int2 e = lds[(sp < S ? sp : S - 1) * TB];
+        if (__builtin_expect(sp >= S, 0)) e = make_int2(spill[(size_t)(sp - S) * stride], (int)0xff800000u);
+        return e;
+    }
+    // the topmost reference whose box starts no farther than t_best; REF_NONE when there is none
+    __device__ __forceinline__ int32_t pop(float t_best) {
+        while (sp > 0) {
+            const int2 e = take();
+            if (__int_as_float(e.y) <= t_best) return e.x;
+        }
+        return REF_NONE;
     }
 };
 
@@ -109,65 +126,89 @@ struct Count {
     uint64_t visits = 0, tests = 0, rays = 0, pair_visits = 0, leaf_fetches = 0;
 };
 
-// The fetch of one visit. node >= 0: an internal node (four 16-byte loads). node < 0: the leaf
-// pair ~node, ~node + 1, which the build does not store: its two spheres are read in the same
-// four loads (each twice; the second reads hit the same cache lines) and turned in place into
-// the node they stand for: child boxes the leaves' boxes (centre -+ radius, as the build
-// computes them), children the two leaves. Waves without a pair skip that branch. PAIRS = false:
-// the tree has none (built with leaf pairs off) and a visit is the node fetch alone.
-struct Visit {
-    float4 a, b, c;
-    int4 d;
-};
-template <bool COUNT, bool PAIRS>
-__device__ __forceinline__ Visit fetch(const TraceArgs& A, int32_t node, Count& cnt) {
-    const bool pair = PAIRS && node < 0;
-    const float4* q = pair ? A.leaf_sph + ~node : reinterpret_cast<const float4*>(A.nodes + node);
-    const float4* q23 = pair ? q : q + 2;
-    Visit v;
-    v.a = q[0];
-    v.b = q[1];
-    v.c = q23[0];
-    v.d = reinterpret_cast<const int4*>(q23)[1];
-    if (COUNT) {
-        cnt.visits++;
-        if (pair) cnt.pair_visits++;
-    }
-    if (pair) {
-        const float4 s0 = v.c, s1 = make_float4(__int_as_float(v.d.x), __int_as_float(v.d.y),
-                                                __int_as_float(v.d.z), __int_as_float(v.d.w));
-        v.a = make_float4(s0.x - s0.w, s0.y - s0.w, s0.z - s0.w, s0.x + s0.w);
-        v.b = make_float4(s0.y + s0.w, s0.z + s0.w, s1.x - s1.w, s1.y - s1.w);
-        v.c = make_float4(s1.z - s1.w, s1.x + s1.w, s1.y + s1.w, s1.z + s1.w);
-        v.d = make_int4(node, node - 1, 0, 1);  // ~l, ~(l + 1)
-    }
-    return v;
+// Traversal of the LBVH by one lane, in two alternating phases. The inner phase visits stored
+// nodes (64 bytes, both child boxes); a lane that reaches a leaf reference puts it aside and goes
+// on with the next node from its stack, and the phase ends when every lane has one aside or is
+// out of nodes. The leaf phase then tests the spheres put aside. Testing the spheres inside the
+// visits instead made nearly every visit of a wavefront run the whole sphere test (two square
+// roots and divisions) for the few lanes that had reached a leaf.
+// Every leaf reference ~k stands for the two spheres k and k + 1, one 32-byte read, whether the
+// node over them was left out of the tree (a leaf pair) or ~k is a single leaf: one more sphere
+// tested changes no result, since the result is that over all spheres, whatever was visited (the
+// least t, ties to the lowest particle id; for an any-hit ray whether there is a hit at all).
+// A stack entry keeps its box's entry distance, and one that lies beyond the best hit when its
+// turn comes is dropped without a fetch.
+
+// One visit: both child boxes against the ray; the near child becomes the node, a far one that is
+// hit too goes to the stack; with neither, the next from the stack.
+template <int S, bool COUNT>
+__device__ __forceinline__ void visit(const TraceArgs& A, const RayPre& r, float tmin, float t_best, int32_t& node,
+                                      LaneStack<S>& st, Count& cnt) {
+    const float4* q = reinterpret_cast<const float4*>(A.nodes + node);
+    const float4 a = q[0], b = q[1], c = q[2];
+    const int2 d = *reinterpret_cast<const int2*>(q + 3);
+    if (COUNT) cnt.visits++;
+    const float tn0 = slab(r, a.x, a.y, a.z, a.w, b.x, b.y, tmin, t_best);
+    const float tn1 = slab(r, b.z, b.w, c.x, c.y, c.z, c.w, tmin, t_best);
+    const bool first0 = tn0 <= tn1;
+    const float tnear = first0 ? tn0 : tn1, tfar = first0 ? tn1 : tn0;
+    node = first0 ? d.x : d.y;
+    if (tfar != INFINITY)
+        st.push(first0 ? d.y : d.x, tfar);
+    else if (tnear == INFINITY)
+        node = st.pop(t_best);
 }
 
-// One node visit of a closest-hit ray (state: node, stack, t_best, best leaf). Returns true when
-// the ray is finished. A closest-hit trace is this step repeated from the root.
-template <int S, bool COUNT, bool PAIRS = true>
-__device__ __forceinline__ bool step_closest(const TraceArgs& A, const RayPre& r, float tmin, float tmax, float& t_best,
-                                             int& best, int32_t& node, LaneStack<S>& st, Count& cnt) {
-    const bool pair_visit = PAIRS && node < 0;
-    const Visit v = fetch<COUNT, PAIRS>(A, node, cnt);
-    float tn0 = slab(r, v.a.x, v.a.y, v.a.z, v.a.w, v.b.x, v.b.y, tmin, t_best);
-    float tn1 = slab(r, v.b.z, v.b.w, v.c.x, v.c.y, v.c.z, v.c.w, tmin, t_best);
-    const int32_t ch0 = v.d.x, ch1 = v.d.y;
-    // a leaf child (ref < 0 without its pair flag: bit 0 / bit 1 of d.z) is tested here; a leaf
-    // pair child is descended into like an internal node. Both leaf spheres are fetched before
-    // either is tested: one memory round trip (for a pair's own two, cache hits).
-    const bool lf0 = tn0 != INFINITY && ch0 < 0 && !(PAIRS && (v.d.z & 1));
-    const bool lf1 = tn1 != INFINITY && ch1 < 0 && !(PAIRS && (v.d.z & 2));
-    float4 sp0 = make_float4(0.f, 0.f, 0.f, 0.f), sp1 = sp0;
-    if (lf0) sp0 = A.leaf_sph[~ch0];
-    if (lf1) sp1 = A.leaf_sph[~ch1];
-    if (COUNT && !pair_visit) cnt.leaf_fetches += (lf0 ? 1 : 0) + (lf1 ? 1 : 0);
-    // the hit is the least t, ties going to the least particle ID, whatever the test order
-    auto test = [&](int leaf, float4 sp) {
-        float t = sphere_t(r.o, r.d, sp, tmin, tmax);
-        if (COUNT) cnt.tests++;
+// The part of sphere_t before its square root: false when that sphere reports no hit. (With b < 0
+// q = b -+ sqrt(delta) is negative and min(c / q, q) too, whatever c is: no report.)
+__device__ __forceinline__ bool sphere_near(const RayPre& r, float4 s, V3& oc, float& b, float& delta) {
+    oc = V3{r.o.x - s.x, r.o.y - s.y, r.o.z - s.z};
+    b = dot(neg(oc), r.d);
+    const V3 tmp = V3{oc.x + b * r.d.x, oc.y + b * r.d.y, oc.z + b * r.d.z};
+    delta = s.w * s.w - dot(tmp, tmp);
+    return !(delta < 0.0f) && !(b < 0.0f);
+}
+// The rest of it.
+__device__ __forceinline__ float sphere_far(V3 oc, float rr, float b, float delta, float tmin, float tmax) {
+    const float c = dot(oc, oc) - rr;
+    const float q = b + __builtin_copysignf(__builtin_sqrtf(delta), b);
+    const float t = fminf(c / q, q);
+    if (t < 0.0f) return -1.0f;
+    return (t > tmin && t < tmax) ? t : -1.0f;
+}
+
+// The spheres k and k + 1 of leaf reference ~k. Most spheres fail the first part of the test, so
+// the second part runs once for whichever sphere passes, and again only for a lane where both do.
+// Closest hit (any false): t_best and best are updated. any: returns true at a hit of a sphere
+// other than leaf `skip` (best and t_best stay).
+template <bool COUNT>
+__device__ __forceinline__ bool test_leaf(const TraceArgs& A, const RayPre& r, float tmin, float tmax, int32_t ref,
+                                          int skip, bool any, float& t_best, int& best, Count& cnt) {
+    const int k0 = ~ref;
+    const int k1 = (uint32_t)k0 + 1u < A.n_sph ? k0 + 1 : k0;
+    const float4 s0 = A.leaf_sph[k0], s1 = A.leaf_sph[k1];
+    if (COUNT) {
+        cnt.visits++;
+        cnt.pair_visits++;
+        cnt.tests += 2;
+    }
+    V3 oc0, oc1;
+    float b0, b1, e0, e1;
+    bool p0 = sphere_near(r, s0, oc0, b0, e0);
+    bool p1 = sphere_near(r, s1, oc1, b1, e1);
+    p0 = p0 && k0 != skip;
+    p1 = p1 && k1 != skip;
+    while (p0 || p1) {
+        const int leaf = p0 ? k0 : k1;
+        const float w = p0 ? s0.w : s1.w;
+        const float t = sphere_far(V3{p0 ? oc0.x : oc1.x, p0 ? oc0.y : oc1.y, p0 ? oc0.z : oc1.z}, w * w, p0 ? b0 : b1,
+                                   p0 ? e0 : e1, tmin, tmax);
+        if (p0)
+            p0 = false;
+        else
+            p1 = false;
         if (t >= 0.0f) {
+            if (any) return true;
             if (t < t_best) {
                 t_best = t;
                 best = leaf;
@@ -175,159 +216,177 @@ __device__ __forceinline__ bool step_closest(const TraceArgs& A, const RayPre& r
                 best = leaf;
             }
         }
-    };
-    if (lf0) {
-        test(~ch0, sp0);
-        tn0 = INFINITY;
-    }
-    if (lf1) {
-        test(~ch1, sp1);
-        tn1 = INFINITY;
-    }
-    bool h0 = tn0 <= t_best, h1 = tn1 <= t_best;
-    if (h0 && h1) {
-        bool first0 = tn0 <= tn1;
-        st.push(first0 ? ch1 : ch0);
-        node = first0 ? ch0 : ch1;
-    } else if (h0) {
-        node = ch0;
-    } else if (h1) {
-        node = ch1;
-    } else {
-        if (st.sp == 0) return true;
-        node = st.pop();
     }
     return false;
 }
 
-// One node visit of an any-hit ray ignoring leaf `skip`: 0 = continue, 1 = finished without a
-// hit, 2 = occluded. Nodes, leaves and leaf pairs as in step_closest.
-template <int S, bool COUNT, bool PAIRS = true>
-__device__ __forceinline__ int step_any(const TraceArgs& A, const RayPre& r, float tmin, float tmax, int skip,
-                                        int32_t& node, LaneStack<S>& st, Count& cnt) {
-    const bool pair_visit = PAIRS && node < 0;
-    const Visit v = fetch<COUNT, PAIRS>(A, node, cnt);
-    float tn0 = slab(r, v.a.x, v.a.y, v.a.z, v.a.w, v.b.x, v.b.y, tmin, tmax);
-    float tn1 = slab(r, v.b.z, v.b.w, v.c.x, v.c.y, v.c.z, v.c.w, tmin, tmax);
-    const int32_t ch0 = v.d.x, ch1 = v.d.y;
-    bool h0 = tn0 != INFINITY, h1 = tn1 != INFINITY;
-    const bool leaf0 = ch0 < 0 && !(PAIRS && (v.d.z & 1)), leaf1 = ch1 < 0 && !(PAIRS && (v.d.z & 2));
-    const bool lf0 = h0 && leaf0 && ~ch0 != skip, lf1 = h1 && leaf1 && ~ch1 != skip;
-    float4 sp0 = make_float4(0.f, 0.f, 0.f, 0.f), sp1 = sp0;
-    if (lf0) sp0 = A.leaf_sph[~ch0];
-    if (lf1) sp1 = A.leaf_sph[~ch1];
-    if (COUNT && !pair_visit) cnt.leaf_fetches += (lf0 ? 1 : 0) + (lf1 ? 1 : 0);
-    if (h0 && leaf0) {
-        if (lf0) {
-            if (COUNT) cnt.tests++;
-            if (sphere_t(r.o, r.d, sp0, tmin, tmax) >= 0.0f) return 2;
+// The inner phase: visits until at most 3/8 of the lanes that began it still look for a leaf to put
+// aside. A lane with a second leaf waits, and where leaves are rare (clusters of sub-pixel spheres)
+// the wait for the last lanes is long: 60M clustered spheres at 4K, 1 sample, 6.82 ms when the phase
+// ran until no lane looked for one, 5.83, 5.71, 5.81 and 6.09 ms at 1/4, 1/2, 3/4 and 15/16 of the
+// lanes (1M uniform spheres: 0.50 ms, then 0.46, 0.45, 0.47, 0.53).
+template <int S, bool COUNT>
+__device__ __forceinline__ void inner_phase(const TraceArgs& A, const RayPre& r, float tmin, float t_best,
+                                            int32_t& node, int32_t& leaf, LaneStack<S>& st, Count& cnt) {
+    const int few = (int)__popcll(__ballot(node >= 0)) * 3 / 8;
+    while (node >= 0) {
+        visit<S, COUNT>(A, r, tmin, t_best, node, st, cnt);
+        if (node < 0 && leaf == REF_NONE && node != REF_NONE) {
+            leaf = node;
+            node = st.pop(t_best);
         }
-        h0 = false;
+        if ((int)__popcll(__ballot(leaf == REF_NONE)) <= few) break;
     }
-    if (h1 && leaf1) {
-        if (lf1) {
-            if (COUNT) cnt.tests++;
-            if (sphere_t(r.o, r.d, sp1, tmin, tmax) >= 0.0f) return 2;
-        }
-        h1 = false;
-    }
-    if (h0 && h1) {
-        bool first0 = tn0 <= tn1;
-        st.push(first0 ? ch1 : ch0);
-        node = first0 ? ch0 : ch1;
-    } else if (h0) {
-        node = ch0;
-    } else if (h1) {
-        node = ch1;
-    } else {
-        if (st.sp == 0) return 1;
-        node = st.pop();
-    }
-    return 0;
-}
-
-// One node visit of either kind of ray, for wavefronts that hold both: a closest-hit ray (ao
-// false; t_best its current bound, as in step_closest) or an any-hit ray (ao true; t_best holds
-// its tmax and is never lowered, leaf `skip` is ignored, as in step_any). Both kinds run one
-// instruction stream, where a lane-divergent choice between the two steps ran both bodies with
-// half the lanes masked off. The arithmetic, the visit order and the tie rule are those of the
-// two steps, so the results are bit-identical. Returns 0 to continue, 1 when the ray is finished
-// (for any-hit: without a hit), 2 for an any-hit ray's hit.
-template <int S, bool COUNT, bool PAIRS = true>
-__device__ __forceinline__ int step_mixed(const TraceArgs& A, const RayPre& r, float tmin, float tmax, float& t_best,
-                                          int& best, int32_t& node, LaneStack<S>& st, Count& cnt, int skip, bool ao) {
-    const bool pair_visit = PAIRS && node < 0;
-    const Visit v = fetch<COUNT, PAIRS>(A, node, cnt);
-    float tn0 = slab(r, v.a.x, v.a.y, v.a.z, v.a.w, v.b.x, v.b.y, tmin, t_best);
-    float tn1 = slab(r, v.b.z, v.b.w, v.c.x, v.c.y, v.c.z, v.c.w, tmin, t_best);
-    const int32_t ch0 = v.d.x, ch1 = v.d.y;
-    const bool leaf0 = ch0 < 0 && !(PAIRS && (v.d.z & 1)), leaf1 = ch1 < 0 && !(PAIRS && (v.d.z & 2));
-    const bool lf0 = tn0 != INFINITY && leaf0 && ~ch0 != skip, lf1 = tn1 != INFINITY && leaf1 && ~ch1 != skip;
-    float4 sp0 = make_float4(0.f, 0.f, 0.f, 0.f), sp1 = sp0;
-    if (lf0) sp0 = A.leaf_sph[~ch0];
-    if (lf1) sp1 = A.leaf_sph[~ch1];
-    if (COUNT && !pair_visit) cnt.leaf_fetches += (lf0 ? 1 : 0) + (lf1 ? 1 : 0);
-    bool hit = false;
-    auto test = [&](int leaf, float4 sp) {
-        const float t = sphere_t(r.o, r.d, sp, tmin, tmax);
-        if (COUNT) cnt.tests++;
-        if (t >= 0.0f) {
-            if (ao) {
-                hit = true;
-            } else if (t < t_best) {
-                t_best = t;
-                best = leaf;
-            } else if (t == t_best && best >= 0 && A.leaf_id[leaf] < A.leaf_id[best]) {
-                best = leaf;
-            }
-        }
-    };
-    if (lf0) test(~ch0, sp0);
-    if (hit) return 2;
-    if (lf1) test(~ch1, sp1);
-    if (hit) return 2;
-    // leaf children are never descended (a skipped leaf neither)
-    if (leaf0) tn0 = INFINITY;
-    if (leaf1) tn1 = INFINITY;
-    const bool h0 = tn0 <= t_best, h1 = tn1 <= t_best;
-    if (h0 && h1) {
-        const bool first0 = tn0 <= tn1;
-        st.push(first0 ? ch1 : ch0);
-        node = first0 ? ch0 : ch1;
-    } else if (h0) {
-        node = ch0;
-    } else if (h1) {
-        node = ch1;
-    } else {
-        if (st.sp == 0) return 1;
-        node = st.pop();
-    }
-    return 0;
 }
 
 // Closest hit: returns the leaf index of the nearest reported intersection (or -1) and its t.
-template <int S, bool COUNT, bool PAIRS = true>
+template <int S, bool COUNT>
 __device__ int trace_closest(const TraceArgs& A, const RayPre& r, float tmin, float tmax, float& t_best,
                              LaneStack<S>& st, Count& cnt) {
     int best = -1;
     t_best = tmax;
-    int32_t node = 0;
+    int32_t node = 0, leaf = REF_NONE;
     st.sp = 0;
-    while (!step_closest<S, COUNT, PAIRS>(A, r, tmin, tmax, t_best, best, node, st, cnt)) {
+    while (node != REF_NONE) {
+        inner_phase<S, COUNT>(A, r, tmin, t_best, node, leaf, st, cnt);
+        while (leaf != REF_NONE) {
+            test_leaf<COUNT>(A, r, tmin, tmax, leaf, -1, false, t_best, best, cnt);
+            leaf = REF_NONE;
+            if (node < 0 && node != REF_NONE) {
+                leaf = node;
+                node = st.pop(t_best);
+            }
+        }
     }
     return best;
 }
 
 // Any hit in (tmin, tmax) ignoring leaf `skip`.
-template <int S, bool COUNT, bool PAIRS = true>
+template <int S, bool COUNT>
 __device__ bool trace_any(const TraceArgs& A, const RayPre& r, float tmin, float tmax, int skip, LaneStack<S>& st,
                           Count& cnt) {
-    int32_t node = 0;
+    int32_t node = 0, leaf = REF_NONE;
     st.sp = 0;
-    int res;
-    while ((res = step_any<S, COUNT, PAIRS>(A, r, tmin, tmax, skip, node, st, cnt)) == 0) {
+    float tb = tmax;
+    int best = -1;
+    while (node != REF_NONE) {
+        inner_phase<S, COUNT>(A, r, tmin, tmax, node, leaf, st, cnt);
+        while (leaf != REF_NONE) {
+            if (test_leaf<COUNT>(A, r, tmin, tmax, leaf, skip, true, tb, best, cnt)) return true;
+            leaf = REF_NONE;
+            if (node < 0 && node != REF_NONE) {
+                leaf = node;
+                node = st.pop(tmax);
+            }
+        }
     }
-    return res == 2;
+    return false;
+}
+
+// Node and sphere words read at a wavefront-uniform address: through the constant address space, so
+// that they arrive in scalar registers (the structure is written by earlier kernels only).
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+typedef const __attribute__((address_space(4))) f32x4* const_f32x4;
+typedef const __attribute__((address_space(4))) i32x4* const_i32x4;
+
+// Closest hit of a whole wavefront whose rays lie in one octant of directions, as the samples of a
+// pixel do: all lanes walk the same nodes together (a node is visited while any lane's ray meets
+// its box before its best hit). The node and its spheres are scalar loads, the stack holds one
+// reference with each lane's own entry distance, and since the sign of every direction component
+// is the same in all lanes, the near and far planes of a box are picked by scalar selects: a visit
+// takes 6 multiply-adds and 5 compares per box, against 6 and 11 lane by lane, and no lane waits
+// for another's sphere test. Every lane's result is that of trace_closest. Lanes need not all be
+// active (sx, sy, sz: the negative direction components).
+template <int S, bool COUNT>
+__device__ __forceinline__ int trace_closest_packet(const TraceArgs& A, const RayPre& r, float tmin, float tmax,
+                                                    bool sx, bool sy, bool sz, float& t_best, LaneStack<S>& st,
+                                                    Count& cnt) {
+    const V3 on = V3{sx ? r.oih.x : r.oil.x, sy ? r.oih.y : r.oil.y, sz ? r.oih.z : r.oil.z};
+    const V3 of = V3{sx ? r.oil.x : r.oih.x, sy ? r.oil.y : r.oih.y, sz ? r.oil.z : r.oih.z};
+    int best = -1;
+    t_best = tmax;
+    int32_t node = 0;
+    int sp = 0;
+    auto slab_oct = [&](float lx, float ly, float lz, float hx, float hy, float hz) -> float {
+        const float xn = __builtin_fmaf(sx ? hx : lx, r.inv.x, -on.x), xf = __builtin_fmaf(sx ? lx : hx, r.inv.x, -of.x);
+        const float yn = __builtin_fmaf(sy ? hy : ly, r.inv.y, -on.y), yf = __builtin_fmaf(sy ? ly : hy, r.inv.y, -of.y);
+        const float zn = __builtin_fmaf(sz ? hz : lz, r.inv.z, -on.z), zf = __builtin_fmaf(sz ? lz : hz, r.inv.z, -of.z);
+        const float tn = fmaxf(fmaxf(xn, yn), fmaxf(zn, tmin));
+        const float tf = fminf(fminf(xf, yf), fminf(zf, t_best));
+        return tn <= tf ? tn : INFINITY;
+    };
+    for (;;) {
+        bool pop = true;
+        if (node >= 0) {
+            const_f32x4 q = (const_f32x4)(uintptr_t)(A.nodes + node);
+            const f32x4 a = q[0], b = q[1], c = q[2];
+            const i32x4 d = *(const_i32x4)(q + 3);
+            if (COUNT) cnt.visits++;
+            const float tn0 = slab_oct(a.x, a.y, a.z, a.w, b.x, b.y);
+            const float tn1 = slab_oct(b.z, b.w, c.x, c.y, c.z, c.w);
+            const uint64_t m0 = __ballot(tn0 != INFINITY), m1 = __ballot(tn1 != INFINITY);
+            if (m0 && m1) {
+                // the child that is nearer for more of the lanes first
+                const bool first0 = 2 * __popcll(__ballot(tn0 <= tn1 && tn0 != INFINITY)) >= __popcll(m0 | m1);
+                st.sp = sp;
+                st.push(first0 ? d.y : d.x, first0 ? tn1 : tn0);
+                sp = st.sp;
+                node = first0 ? d.x : d.y;
+                pop = false;
+            } else if (m0 | m1) {
+                node = m0 ? d.x : d.y;
+                pop = false;
+            }
+        } else {
+            const int k0 = ~node;
+            const int k1 = (uint32_t)k0 + 1u < A.n_sph ? k0 + 1 : k0;
+            if (COUNT) {
+                cnt.visits++;
+                cnt.pair_visits++;
+                cnt.tests += 2;
+            }
+            const f32x4 v0 = *(const_f32x4)(uintptr_t)(A.leaf_sph + k0), v1 = *(const_f32x4)(uintptr_t)(A.leaf_sph + k1);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const f32x4 v = j ? v1 : v0;
+                const int leaf = j ? k1 : k0;
+                V3 oc;
+                float b, e;
+                if (!sphere_near(r, make_float4(v.x, v.y, v.z, v.w), oc, b, e)) continue;
+                const float t = sphere_far(oc, v.w * v.w, b, e, tmin, tmax);
+                if (t >= 0.0f) {
+                    if (t < t_best) {
+                        t_best = t;
+                        best = leaf;
+                    } else if (t == t_best && best >= 0 && A.leaf_id[leaf] < A.leaf_id[best]) {
+                        best = leaf;
+                    }
+                }
+            }
+        }
+        while (pop) {
+            if (sp == 0) return best;
+            st.sp = sp;
+            const int2 e = st.take();
+            --sp;
+            if (!__ballot(__int_as_float(e.y) <= t_best)) continue;
+            node = __builtin_amdgcn_readfirstlane(e.x);
+            pop = false;
+        }
+    }
+}
+
+// The closest hit of the active lanes' rays: together where they share an octant of directions,
+// else lane by lane.
+template <int S, bool COUNT>
+__device__ __forceinline__ int trace_closest_group(const TraceArgs& A, const RayPre& r, float tmin, float tmax,
+                                                   float& t_best, LaneStack<S>& st, Count& cnt) {
+    const uint64_t act = __ballot(true);
+    const uint64_t bx = __ballot(r.inv.x < 0.0f), by = __ballot(r.inv.y < 0.0f), bz = __ballot(r.inv.z < 0.0f);
+    if ((bx == 0 || bx == act) && (by == 0 || by == act) && (bz == 0 || bz == act))
+        return trace_closest_packet<S, COUNT>(A, r, tmin, tmax, bx != 0, by != 0, bz != 0, t_best, st, cnt);
+    return trace_closest<S, COUNT>(A, r, tmin, tmax, t_best, st, cnt);
 }
 
 // Slab test of one child box returning the entry distance (+inf when missed) and the exit.
@@ -384,8 +443,7 @@ __device__ int trace_tl(const TraceArgs& A, const RayPre& r, float tmin, float t
                 const bool first0 = tn0 <= tn1;
                 const int32_t rn = first0 ? r0 : r1, rf = first0 ? r1 : r0;
                 const float tnf = first0 ? tn1 : tn0;
-                if (rf < 0) st.push(__float_as_int(tnf));
-                st.push(rf);
+                st.push(rf, tnf);
                 node = rn;
                 t0 = first0 ? tn0 : tn1;
                 t1 = first0 ? tf0 : tf1;
@@ -445,8 +503,7 @@ __device__ int trace_tl(const TraceArgs& A, const RayPre& r, float tmin, float t
             const bool need_n = nc < m && t0 <= n_t1;
             const bool need_f = fc < m && f_t0 <= lim;
             if (need_n && need_f) {
-                st.push(__float_as_int(f_t0));
-                st.push(~(int32_t)(bs + fc));
+                st.push(~(int32_t)(bs + fc), f_t0);
                 node = ~(int32_t)(bs + nc);
                 t1 = n_t1;
             } else if (need_n) {
@@ -463,15 +520,11 @@ __device__ int trace_tl(const TraceArgs& A, const RayPre& r, float tmin, float t
         if (pop) {
             for (;;) {
                 if (st.sp == 0) return ANY ? 0 : best;
-                const int32_t v = st.pop();
-                if (v >= 0) {
-                    node = v;
-                    break;
-                }
-                const float a0 = __int_as_float(st.pop());
+                const int2 e = st.take();
+                const float a0 = __int_as_float(e.y);
                 if (a0 <= t_best) {
-                    node = v;
-                    t0 = a0;
+                    node = e.x;
+                    t0 = fmaxf(a0, 0.0f);  // (a spilled entry carries no distance)
                     t1 = t_best;
                     break;
                 }
@@ -481,20 +534,20 @@ __device__ int trace_tl(const TraceArgs& A, const RayPre& r, float tmin, float t
 }
 
 // The structure a kernel traverses: TL = treelet P-k-d trees, else the LBVH.
-template <int S, bool COUNT, bool PAIRS, bool TL>
+template <int S, bool COUNT, bool TL>
 __device__ __forceinline__ int trace_closest_x(const TraceArgs& A, const RayPre& r, float tmin, float tmax,
                                                float& t_best, LaneStack<S>& st, Count& cnt) {
     if (TL) return trace_tl<S, COUNT, false>(A, r, tmin, tmax, -1, t_best, st, cnt);
-    return trace_closest<S, COUNT, PAIRS>(A, r, tmin, tmax, t_best, st, cnt);
+    return trace_closest<S, COUNT>(A, r, tmin, tmax, t_best, st, cnt);
 }
-template <int S, bool COUNT, bool PAIRS, bool TL>
+template <int S, bool COUNT, bool TL>
 __device__ __forceinline__ bool trace_any_x(const TraceArgs& A, const RayPre& r, float tmin, float tmax, int skip,
                                             LaneStack<S>& st, Count& cnt) {
     if (TL) {
         float tb;
         return trace_tl<S, COUNT, true>(A, r, tmin, tmax, skip, tb, st, cnt) != 0;
     }
-    return trace_any<S, COUNT, PAIRS>(A, r, tmin, tmax, skip, st, cnt);
+    return trace_any<S, COUNT>(A, r, tmin, tmax, skip, st, cnt);
 }
 
 // Diffuse bounce direction of raygen.cu:71-77,149-152: rejection sample in the unit cube,
@@ -589,7 +642,7 @@ __device__ void shade_pixel(const TraceArgs& A, uint32_t px, uint32_t py, float 
         RayPre r = prep(o, d, pad);
         float t;
         if (COUNT) cnt.rays++;
-        int leaf = trace_closest_x<S, COUNT, true, TL>(A, r, 1e-6f, 1e20f, t, st, cnt);
+        int leaf = trace_closest_x<S, COUNT, TL>(A, r, 1e-6f, 1e20f, t, st, cnt);
         float4 sc;
         float ray_depth = FLT_MAX;
         if (leaf < 0) {
@@ -611,7 +664,7 @@ __device__ void shade_pixel(const TraceArgs& A, uint32_t px, uint32_t py, float 
                 V3 ad = ao_direction(N, aseed, s, f.spp);
                 RayPre ra = prep(P, ad, pad);
                 if (COUNT) cnt.rays++;
-                bool occ = trace_any_x<S, COUNT, true, TL>(A, ra, 0.0f, f.ao_distance, leaf, st, cnt);
+                bool occ = trace_any_x<S, COUNT, TL>(A, ra, 0.0f, f.ao_distance, leaf, st, cnt);
                 float V = occ ? 0.0f : 1.0f;
                 sc = make_float4(alb.x * V, alb.y * V, alb.z * V, 1.0f);
                 vis_sum += V;
@@ -633,7 +686,7 @@ __device__ void shade_pixel(const TraceArgs& A, uint32_t px, uint32_t py, float 
                     RayPre rb = prep(so, sd, pad);
                     float tb;
                     if (COUNT) cnt.rays++;
-                    int lb = trace_closest_x<S, COUNT, true, TL>(A, rb, 1e-3f, 1e8f, tb, st, cnt);
+                    int lb = trace_closest_x<S, COUNT, TL>(A, rb, 1e-3f, 1e8f, tb, st, cnt);
                     if (lb < 0) {
                         res = make_float4(cc.x * 0.8f, cc.y * 0.8f, cc.z * 0.8f, 1.0f);
                         break;
@@ -673,11 +726,12 @@ __device__ void shade_pixel(const TraceArgs& A, uint32_t px, uint32_t py, float 
     write_pixel(A, opix, col, depth, best_t, best_leaf, aux, vis_sum);
 }
 
-// Lane per pixel, samples in a loop (every sample count). Held to 72 VGPRs (7 wavefronts per SIMD
-// instead of 4): 64-spp AO 64.3 -> 57.7 ms, 1-spp AO 1.22 -> 1.14 ms.
+// Lane per pixel, samples in a loop (every sample count). Held to 72 VGPRs (7 wavefronts per SIMD),
+// which the fetch latency needs. With the two-phase traversal a frame of 4-bounce paths (1M spheres,
+// 801x600, 1 sample) went from 1.65 to 0.71 ms.
 template <int S, int MODE, bool COUNT, bool STEAL, bool TL = false>
 __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(7, 8))) void k_trace(TraceArgs A) {
-    __shared__ int32_t lds_stack[S * TB];
+    __shared__ int2 lds_stack[S * TB];
     const uint32_t gtid = blockIdx.x * TB + threadIdx.x;
     LaneStack<S> st{lds_stack + threadIdx.x, A.spill + gtid, A.spill_stride, 0, A.ctr + 1};
     Count cnt;
@@ -716,7 +770,7 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(7, 8))) void
 // One sample of a Lambert (MODE 0) or AO (MODE 1) pixel, the arithmetic of shade_pixel: the
 // sample colour, its depth contribution, the hit (t, leaf), the visibility and, for the
 // features, albedo and normal.
-template <int S, int MODE, bool COUNT, bool PAIRS, bool TL = false>
+template <int S, int MODE, bool COUNT, bool TL = false>
 __device__ __forceinline__ void shade_sample(const TraceArgs& A, uint32_t px, uint32_t py, uint32_t pix, uint32_t s,
                                              float jx, float jy, float pad, LaneStack<S>& st, Count& cnt,
                                              float4& sc, float& ray_depth, float& t, int& leaf, float& V,
@@ -726,7 +780,10 @@ __device__ __forceinline__ void shade_sample(const TraceArgs& A, uint32_t px, ui
     primary_ray(f, px, py, jx, jy, o, d);
     RayPre r = prep(o, d, pad);
     if (COUNT) cnt.rays++;
-    leaf = trace_closest_x<S, COUNT, PAIRS, TL>(A, r, 1e-6f, 1e20f, t, st, cnt);
+    if (TL)
+        leaf = trace_closest_x<S, COUNT, TL>(A, r, 1e-6f, 1e20f, t, st, cnt);
+    else
+        leaf = trace_closest_group<S, COUNT>(A, r, 1e-6f, 1e20f, t, st, cnt);
     ray_depth = FLT_MAX;
     V = 0.0f;
     if (leaf < 0) {
@@ -751,7 +808,7 @@ __device__ __forceinline__ void shade_sample(const TraceArgs& A, uint32_t px, ui
         V3 ad = ao_direction(N, aseed, s, f.spp);
         RayPre ra = prep(P, ad, pad);
         if (COUNT) cnt.rays++;
-        bool occ = trace_any_x<S, COUNT, PAIRS, TL>(A, ra, 0.0f, f.ao_distance, leaf, st, cnt);
+        bool occ = trace_any_x<S, COUNT, TL>(A, ra, 0.0f, f.ao_distance, leaf, st, cnt);
         V = occ ? 0.0f : 1.0f;
         sc = make_float4(alb.x * V, alb.y * V, alb.z * V, 1.0f);
     } else {
@@ -767,13 +824,13 @@ __device__ __forceinline__ void shade_sample(const TraceArgs& A, uint32_t px, ui
 // Sample s of a pixel draws its jitter from the pixel's stream advanced by 2s steps
 // (lcg_skip), and the group folds its samples into the pixel in sample order (colour sums,
 // first strictly nearer hit, visibility, sample-0 features), so every output is bit-identical
-// to the lane-per-pixel kernels. Held to 72 VGPRs (7 wavefronts per SIMD instead of 4, a few
-// registers spilled): 64-spp AO 33.8 -> 30.6 ms, Lambert 22.9 -> 20.8 ms (5 wavefronts: 32.6 and
-// 21.2 ms, 6: 31.1 and 21.3, 8: 30.8 and 21.0).
-template <int S, int MODE, bool COUNT, bool PAIRS, bool TL = false>
+// to the lane-per-pixel kernels. The primary rays of a pass take one packet walk, the AO rays the
+// two-phase traversal lane by lane; 50M FCC spheres at 1080p, 64-spp AO: 31.5 -> 18.4 ms (bound by
+// vector ALU issue before; 16 spp of 3M spheres at 1000x621: 3.66 -> 1.97 ms). Held to 72 VGPRs (7
+// wavefronts per SIMD, a few registers spilled) like the other lane kernels.
+template <int S, int MODE, bool COUNT, bool TL = false>
 __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(7, 8))) void k_trace_sl(TraceArgs A) {
-    __shared__ int32_t lds_stack[S * TB];
-    __shared__ float4 lds_col[TB];  // the wavefront's sample colours of one round
+    __shared__ int2 lds_stack[S * TB];
     const uint32_t gtid = blockIdx.x * TB + threadIdx.x;
     LaneStack<S> st{lds_stack + threadIdx.x, A.spill + gtid, A.spill_stride, 0, A.ctr + 1};
     Count cnt;
@@ -815,7 +872,7 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(7, 8))) void
                     uint32_t seed = lcg_skip(seed0, 2u * s);
                     float jx = rnd(seed);
                     float jy = rnd(seed);
-                    shade_sample<S, MODE, COUNT, PAIRS, TL>(A, px, py, pix, s, jx, jy, pad, st, cnt, sc, ray_depth,
+                    shade_sample<S, MODE, COUNT, TL>(A, px, py, pix, s, jx, jy, pad, st, cnt, sc, ray_depth,
                                                             t, leaf, V, alb, N);
                 }
                 // visibility is 0 or 1 per sample, so its sum is exact in any order: the count of
@@ -842,18 +899,20 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(7, 8))) void
                     best_leaf = rl;
                 }
                 // colours are summed in sample order by the group's first lane (the one that
-                // writes the pixel), from the wavefront's slice of LDS
-                float4* wcol = lds_col + (threadIdx.x - lane);
-                wcol[lane] = sc;
+                // writes the pixel), through the first two stack rows of the wavefront's lanes (no
+                // ray is under way here)
+                int2* wcol = lds_stack + (threadIdx.x - lane);
+                wcol[lane] = make_int2(__float_as_int(sc.x), __float_as_int(sc.y));
+                wcol[TB + lane] = make_int2(__float_as_int(sc.z), __float_as_int(sc.w));
                 __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
                 __builtin_amdgcn_wave_barrier();
                 if (sl == 0) {
                     for (uint32_t i = 0; i < L; ++i) {
-                        const float4 c = wcol[base + i];
-                        col.x += c.x;
-                        col.y += c.y;
-                        col.z += c.z;
-                        col.w += c.w;
+                        const int2 c = wcol[base + i], d = wcol[TB + base + i];
+                        col.x += __int_as_float(c.x);
+                        col.y += __int_as_float(c.y);
+                        col.z += __int_as_float(d.x);
+                        col.w += __int_as_float(d.y);
                     }
                 }
                 __builtin_amdgcn_wave_barrier();
@@ -895,14 +954,12 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(7, 8))) void
 // random streams are those of k_trace, so the results are bit-identical.
 enum : int { L_IDLE = 0, L_NEED = 1, L_PRIM = 2, L_AO = 3, L_PRIM_DONE = 4, L_AO_DONE = 5, L_OFF = 6 };
 
-// Held to 5 wavefronts per SIMD (at most 102 VGPRs; it takes 95 and spills nothing). With one step
-// for both kinds of ray the kernel is shorter, and the 1-spp frame's trace went from 1.02 ms at 7
-// wavefronts (72 VGPRs and 96 bytes of spills per lane) to 0.92 ms (6 wavefronts, 60 bytes of
-// spills: 0.91 ms). Before that step, 7 wavefronts had been the fastest (5: 1.07, 7: 1.04 ms).
+// Held to 5 wavefronts per SIMD (at most 102 VGPRs; it takes 96 and spills nothing). Primary and AO
+// rays, which a refilled wavefront holds at once, run one instruction stream.
 template <int S, int MODE, bool COUNT>
 __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(5, 8))) void k_trace_refill(TraceArgs A,
                                                                                                 uint32_t refill) {
-    __shared__ int32_t lds_stack[S * TB];
+    __shared__ int2 lds_stack[S * TB];
     const uint32_t gtid = blockIdx.x * TB + threadIdx.x;
     LaneStack<S> st{lds_stack + threadIdx.x, A.spill + gtid, A.spill_stride, 0, A.ctr + 1};
     Count cnt;
@@ -926,10 +983,8 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(5, 8))) void
     RayPre r;
     float tmin = 0.f, tmax = 0.f, t_best = 0.f;
     int best = -1, skip = -1;
-    int32_t node = 0;
+    int32_t node = 0, leaf = REF_NONE;
     float4 alb = make_float4(0.f, 0.f, 0.f, 0.f);
-    float prim_t = 0.f;
-    int prim_leaf = -1;
     for (;;) {
         // 1. idle lanes take pixels (work index -> 8x8 tile order inside the window)
         uint64_t idle = __ballot(state == L_IDLE);
@@ -983,19 +1038,24 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(5, 8))) void
         uint64_t act = __ballot(state == L_PRIM || state == L_AO);
         uint64_t live = __ballot(state != L_OFF);
         if (!live) break;
-        // 3. traversal: one node visit per active lane per iteration
+        // 3. traversal: per iteration one inner phase and one leaf phase of the active lanes,
+        // primary and AO lanes together (an any-hit ray's bound t_best stays at its tmax)
         while (act) {
-            if (state == L_PRIM || state == L_AO) {  // one step for both kinds (primary and AO lanes mix here)
+            if (state == L_PRIM || state == L_AO) {
                 const bool ao = state == L_AO;
-                const int res = step_mixed<S, COUNT>(A, r, tmin, tmax, t_best, best, node, st, cnt, ao ? skip : -1, ao);
-                if (res) {
-                    if (ao) {
-                        state = L_AO_DONE;
-                        best = res;  // 2 = occluded
-                    } else {
-                        state = L_PRIM_DONE;
+                inner_phase<S, COUNT>(A, r, tmin, t_best, node, leaf, st, cnt);
+                while (leaf != REF_NONE) {
+                    const bool occ = test_leaf<COUNT>(A, r, tmin, tmax, leaf, ao ? skip : -1, ao, t_best, best, cnt);
+                    leaf = REF_NONE;
+                    if (occ) {
+                        best = 2;
+                        node = REF_NONE;
+                    } else if (node < 0 && node != REF_NONE) {
+                        leaf = node;
+                        node = st.pop(t_best);
                     }
                 }
+                if (node == REF_NONE) state = ao ? L_AO_DONE : L_PRIM_DONE;
             }
             act = __ballot(state == L_PRIM || state == L_AO);
             if ((uint32_t)__popcll(act) < refill) break;
@@ -1029,13 +1089,12 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(5, 8))) void
                 if (MODE == 1) {
                     uint32_t aseed = tea16(pix, 0xA0000000u + f.frame_idx * 4096u + s);
                     V3 ad = ao_direction(N, aseed, s, f.spp);
-                    prim_t = t;
-                    prim_leaf = best;
                     r = prep(Pp, ad, pad);
                     tmin = 0.0f;
                     tmax = f.ao_distance;
                     t_best = tmax;  // an any-hit ray's bound in step_mixed
                     skip = best;
+                    best = -1;
                     node = 0;
                     st.sp = 0;
                     if (COUNT) cnt.rays++;
@@ -1051,8 +1110,6 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(5, 8))) void
             col.x += alb.x * V; col.y += alb.y * V; col.z += alb.z * V; col.w += 1.0f;
             vis_sum += V;
             sample_done = true;
-            (void)prim_t;
-            (void)prim_leaf;
         }
         if (sample_done) {
             if (++s < f.spp) {
@@ -1097,35 +1154,26 @@ void launch1(const TraceArgs& A, unsigned grid, bool steal, bool count, int mode
         launch2<S, 0>(A, grid, steal, count, s);
 }
 
-template <int S, bool PAIRS>
-void launch_sl_p(const TraceArgs& A, unsigned grid, bool count, int mode, hipStream_t s) {
+template <int S>
+void launch_sl(const TraceArgs& A, unsigned grid, bool count, int mode, hipStream_t s) {
     if (mode == 1) {
         if (count)
-            hipLaunchKernelGGL((k_trace_sl<S, 1, true, PAIRS>), dim3(grid), dim3(TB), 0, s, A);
+            hipLaunchKernelGGL((k_trace_sl<S, 1, true>), dim3(grid), dim3(TB), 0, s, A);
         else
-            hipLaunchKernelGGL((k_trace_sl<S, 1, false, PAIRS>), dim3(grid), dim3(TB), 0, s, A);
+            hipLaunchKernelGGL((k_trace_sl<S, 1, false>), dim3(grid), dim3(TB), 0, s, A);
     } else {
         if (count)
-            hipLaunchKernelGGL((k_trace_sl<S, 0, true, PAIRS>), dim3(grid), dim3(TB), 0, s, A);
+            hipLaunchKernelGGL((k_trace_sl<S, 0, true>), dim3(grid), dim3(TB), 0, s, A);
         else
-            hipLaunchKernelGGL((k_trace_sl<S, 0, false, PAIRS>), dim3(grid), dim3(TB), 0, s, A);
+            hipLaunchKernelGGL((k_trace_sl<S, 0, false>), dim3(grid), dim3(TB), 0, s, A);
     }
-}
-// The sample-lanes kernel is the one whose rays are coherent enough for the cost of the
-// leaf-pair branch to show: a tree built without pairs gets the variant without it.
-template <int S>
-void launch_sl(const TraceArgs& A, unsigned grid, bool count, int mode, bool pairs, hipStream_t s) {
-    if (pairs)
-        launch_sl_p<S, true>(A, grid, count, mode, s);
-    else
-        launch_sl_p<S, false>(A, grid, count, mode, s);
 }
 
 // Kernels over the treelet P-k-d trees.
 template <int MODE, bool COUNT>
 void launch_tl_m(const TraceArgs& A, unsigned grid, bool sl, hipStream_t s) {
     if (sl && MODE != 2)
-        hipLaunchKernelGGL((k_trace_sl<16, MODE == 2 ? 0 : MODE, COUNT, false, true>), dim3(grid), dim3(TB), 0, s, A);
+        hipLaunchKernelGGL((k_trace_sl<16, MODE == 2 ? 0 : MODE, COUNT, true>), dim3(grid), dim3(TB), 0, s, A);
     else
         hipLaunchKernelGGL((k_trace<16, MODE, COUNT, true, true>), dim3(grid), dim3(TB), 0, s, A);
 }
@@ -1158,13 +1206,12 @@ void launch_refill(const TraceArgs& A, unsigned grid, uint32_t refill, bool coun
 // in its constants, share one persistent launch. The global tile index runs over the concatenated
 // tiles of the jobs (prefix[j] = first tile of job j); each wavefront steals tiles and shades them
 // with its job's constants and output buffers.
-// Held to 72 VGPRs (7 wavefronts per SIMD instead of 4) like the single-frame kernels: the batched
-// series (python bench.py --config series) went from 149.0 to 135.7 ms per launch.
+// Held to 72 VGPRs (7 wavefronts per SIMD) like the single-frame kernels.
 template <int S, int MODE, bool TL = false>
 __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(7, 8))) void k_trace_batch(const TraceArgs* __restrict__ jobs,
                                                     const uint32_t* __restrict__ prefix, uint32_t n_jobs,
                                                     uint32_t* ctr) {
-    __shared__ int32_t lds_stack[S * TB];
+    __shared__ int2 lds_stack[S * TB];
     const uint32_t gtid = blockIdx.x * TB + threadIdx.x;
     LaneStack<S> st{lds_stack + threadIdx.x, jobs[0].spill + gtid, jobs[0].spill_stride, 0, ctr + 1};
     Count cnt;
@@ -1219,10 +1266,10 @@ void launch_trace_batch(mmhrt_ctx_s* c, const void* jobs, const uint32_t* prefix
     else                                                                                                    \
         hipLaunchKernelGGL((k_trace_batch<SV, 0>), dim3(grid), dim3(TB), 0, c->stream, J, prefix, n_jobs, ctr);
     switch (S) {
-    case 8: MMHRT_BATCH(8) break;
-    case 24: MMHRT_BATCH(24) break;
-    case 32: MMHRT_BATCH(32) break;
-    default: MMHRT_BATCH(16) break;
+    case 8: MMHRT_BATCH(4) break;
+    case 24: MMHRT_BATCH(12) break;
+    case 32: MMHRT_BATCH(16) break;
+    default: MMHRT_BATCH(8) break;
     }
 #undef MMHRT_BATCH
 }
@@ -1291,24 +1338,24 @@ void dispatch_trace(mmhrt_ctx_s* c, const TraceArgs& A, unsigned grid, bool coun
     }
     if (c->opt_sample_lanes != 0 && refill == 0 && fc.mode != 2 && sl_shape) {
         switch (S) {
-        case 8: launch_sl<8>(A, grid, count, fc.mode, c->bvh_pairs, c->stream); break;
-        case 24: launch_sl<24>(A, grid, count, fc.mode, c->bvh_pairs, c->stream); break;
-        case 32: launch_sl<32>(A, grid, count, fc.mode, c->bvh_pairs, c->stream); break;
-        default: launch_sl<16>(A, grid, count, fc.mode, c->bvh_pairs, c->stream); break;
+        case 8: launch_sl<4>(A, grid, count, fc.mode, c->stream); break;
+        case 24: launch_sl<12>(A, grid, count, fc.mode, c->stream); break;
+        case 32: launch_sl<16>(A, grid, count, fc.mode, c->stream); break;
+        default: launch_sl<8>(A, grid, count, fc.mode, c->stream); break;
         }
     } else if (refill > 0 && fc.mode != 2) {
         switch (S) {
-        case 8: launch_refill<8>(A, grid, refill, count, fc.mode, c->stream); break;
-        case 24: launch_refill<24>(A, grid, refill, count, fc.mode, c->stream); break;
-        case 32: launch_refill<32>(A, grid, refill, count, fc.mode, c->stream); break;
-        default: launch_refill<16>(A, grid, refill, count, fc.mode, c->stream); break;
+        case 8: launch_refill<4>(A, grid, refill, count, fc.mode, c->stream); break;
+        case 24: launch_refill<12>(A, grid, refill, count, fc.mode, c->stream); break;
+        case 32: launch_refill<16>(A, grid, refill, count, fc.mode, c->stream); break;
+        default: launch_refill<8>(A, grid, refill, count, fc.mode, c->stream); break;
         }
     } else {
         switch (S) {
-        case 8: launch1<8>(A, grid, steal, count, fc.mode, c->stream); break;
-        case 24: launch1<24>(A, grid, steal, count, fc.mode, c->stream); break;
-        case 32: launch1<32>(A, grid, steal, count, fc.mode, c->stream); break;
-        default: launch1<16>(A, grid, steal, count, fc.mode, c->stream); break;
+        case 8: launch1<4>(A, grid, steal, count, fc.mode, c->stream); break;
+        case 24: launch1<12>(A, grid, steal, count, fc.mode, c->stream); break;
+        case 32: launch1<16>(A, grid, steal, count, fc.mode, c->stream); break;
+        default: launch1<8>(A, grid, steal, count, fc.mode, c->stream); break;
         }
     }
 }
