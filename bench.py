@@ -69,10 +69,10 @@ def trace_kernel_label(r, spp, mode):
 # AO frame with the feature buffer.
 ABLATION = {
     "64spp": [
-        ("sample lanes, work stealing, LDS stack 16 (library default), 8x8 tiles", {"stack_lds": 16, "refill": 0}),
-        ("LDS stack 8 entries", {"stack_lds": 8, "refill": 0}),
-        ("LDS stack 24 entries", {"stack_lds": 24, "refill": 0}),
-        ("LDS stack 32 entries", {"stack_lds": 32, "refill": 0}),
+        ("sample lanes, work stealing, LDS stack 16 words (library default), 8x8 tiles", {"stack_lds": 16, "refill": 0}),
+        ("LDS stack 8 words", {"stack_lds": 8, "refill": 0}),
+        ("LDS stack 24 words", {"stack_lds": 24, "refill": 0}),
+        ("LDS stack 32 words", {"stack_lds": 32, "refill": 0}),
         ("4x16 tiles", {"stack_lds": 16, "refill": 0, "tile_w": 4}),
         ("lane per pixel (samples in a loop)", {"stack_lds": 16, "refill": 0, "sample_lanes": 0}),
         ("lane per pixel, static tile order (no work stealing)",
@@ -84,12 +84,13 @@ ABLATION = {
          {"stack_lds": 16, "refill": 0, "leaf_pairs": 1}),
     ],
     "1spp": [
-        ("lane per pixel, work stealing, LDS stack 16, 8x8 tiles, no compaction", {"stack_lds": 16, "refill": 0}),
+        ("lane per pixel, work stealing, LDS stack 16 words, 8x8 tiles, no compaction (library default)",
+         {"stack_lds": 16, "refill": 0}),
         ("static tile order (no work stealing)", {"stack_lds": 16, "refill": 0, "persistent": 0}),
-        ("ballot compaction (refill at 16 idle lanes; library default)", {"stack_lds": 16, "refill": 16}),
+        ("ballot compaction (refill at 16 idle lanes)", {"stack_lds": 16, "refill": 16}),
         ("ballot compaction (refill at 32 idle lanes)", {"stack_lds": 16, "refill": 32}),
-        ("LDS stack 8 entries", {"stack_lds": 8, "refill": 0}),
-        ("LDS stack 32 entries", {"stack_lds": 32, "refill": 0}),
+        ("LDS stack 8 words", {"stack_lds": 8, "refill": 0}),
+        ("LDS stack 32 words", {"stack_lds": 32, "refill": 0}),
         ("4 workgroups per CU", {"stack_lds": 16, "refill": 0, "blocks_per_cu": 4}),
         ("tree without leaf pairs", {"stack_lds": 16, "refill": 0, "leaf_pairs": 0}),
     ],

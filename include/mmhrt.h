@@ -320,9 +320,9 @@ MMHRT_API int32_t mmhrt_denoiser_train_step(mmhrt_ctx ctx, const uint16_t* feats
 
 /* Tuning knobs (autotuner output): "stack_lds" (LDS words of the traversal stack per lane: 8, 16, 24
  * or 32, default 16; an entry, a reference and its entry distance, takes two),
- * "tile_w", "tile_h", "persistent" (0/1), "refill" (ballot refill threshold in lanes; -1, the
- * default: 16 for 1-spp frames, 0 otherwise), "blocks_per_cu" (persistent
- * workgroups per CU), "refit_period" (MMHRT_BUILD_AUTO: refits between rebuilds), "build_chunk"
+ * "tile_w", "tile_h", "persistent" (0/1), "refill" (ballot refill threshold in lanes; below 1,
+ * the default: off), "blocks_per_cu" (persistent
+ * workgroups per CU, at most as many as fit), "refit_period" (MMHRT_BUILD_AUTO: refits between rebuilds), "build_chunk"
  * (leaves per LBVH chunk workgroup: 1024, 512 or 256), "build_ls" (level-synchronous chunk
  * pass, default 1; 0: one climbing thread per leaf), "build_grid" (test hook: at most this many
  * persistent chunk workgroups, 0 = as many as fit), "sort_ri" (radix sort keys per thread per

@@ -158,7 +158,7 @@ int32_t mmhrt_render_batch(mmhrt_ctx c, const mmhrt_job* jobs, uint32_t n_jobs, 
     if ((e = ensure(c, c->bt_t, total_px, "batch t"))) return e;
     if ((e = ensure(c, c->bt_id, total_px, "batch id"))) return e;
     if ((e = ensure(c, c->bt_rgba8, total_px, "batch rgba8"))) return e;
-    if ((e = ensure(c, c->batch_ctr, launches.size() * 16, "batch counters"))) return e;
+    if ((e = ensure(c, c->batch_ctr, launches.size() * TRACE_CTR_WORDS, "batch counters"))) return e;
     const size_t js = batch_job_size();
     if ((e = ensure(c, c->batch_jobs, js * n_jobs, "batch jobs"))) return e;
     // The builds read the timestep slices and their count; the context's own spheres, count and
@@ -265,7 +265,7 @@ int32_t mmhrt_render_batch(mmhrt_ctx c, const mmhrt_job* jobs, uint32_t n_jobs, 
     auto launch = [&](size_t li) {
         const Launch& L = launches[li];
         launch_trace_batch(c, c->batch_jobs.p + js * L.first, c->batch_prefix.p + L.prefix, L.count,
-                           c->batch_ctr.p + 16 * li, L.mode, tl);
+                           c->batch_ctr.p + (size_t)TRACE_CTR_WORDS * li, L.mode, tl);
     };
     auto issue = [&]() -> int {
         size_t li = 0;

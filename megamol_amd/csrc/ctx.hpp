@@ -132,12 +132,12 @@ struct mmhrt_ctx_s {
     mmhrt::DevBuf<uint32_t> fb_rgba8;
     mmhrt::DevBuf<__half> fb_aux;
     mmhrt::DevBuf<int32_t> spill;
-    mmhrt::DevBuf<uint32_t> counters;  // [0] tile counter, [2..7] visit counters (u64 pairs)
+    mmhrt::DevBuf<uint32_t> counters;  // TRACE_CTR_WORDS: overflow flag, visit counters (u64 pairs), work queues
 
     // options
     int64_t opt_stack_lds = 16;  // LDS words per lane (8 entries): leaves the LDS for 7 wavefronts per SIMD
     int64_t opt_persistent = 1;
-    int64_t opt_refill = -1;  // ballot-refill threshold; -1: 16 for 1-spp frames (measured 13% faster), else off
+    int64_t opt_refill = -1;  // ballot-refill threshold; below 1: off (the lane-per-pixel kernels)
     int64_t opt_count = 0;
     int64_t opt_blocks_per_cu = 8;
     int64_t opt_tile_w = 8, opt_tile_h = 8;
@@ -257,9 +257,12 @@ int sort_spheres(mmhrt_ctx_s* c, int bits);
 int build_pkd(mmhrt_ctx_s* c, int bits);
 
 // trace.hip
-constexpr int TRACE_STACK_CAP = 124;                       // traversal stack entries per lane
-constexpr int TRACE_SPILL_PER_LANE = TRACE_STACK_CAP - 4;  // the most any LDS stack depth (>= 4) spills, one word each
-constexpr uint32_t TRACE_CTR_WORDS = 16;                   // tile counter, overflow flag, 5 u64 counters
+// Spilled traversal stack words per lane: with at least 4 entries in LDS, room for an LBVH's height
+// (at most 63 + 31) and, at two words each, for a treelet tree's (at most 23 + 10).
+constexpr int TRACE_SPILL_PER_LANE = 120;
+constexpr uint32_t TRACE_QUEUE = 32;                       // first word of the 8 work queue counters
+constexpr uint32_t TRACE_QUEUE_STRIDE = 32;                // words between them (a cache line each)
+constexpr uint32_t TRACE_CTR_WORDS = TRACE_QUEUE + 8 * TRACE_QUEUE_STRIDE;  // overflow flag, 5 u64 counters, queues
 struct FrameOutputs {
     float4* color;
     float* depth;

@@ -2,7 +2,7 @@
 //
 // For callers that cannot allocate device memory (work under HIP graph capture, tight serving
 // loops, harnesses that forbid hipMalloc): the frame goes to device buffers the caller owns, and
-// the trace's scratch (the tile counter, overflow flag and instrumentation words, and the
+// the trace's scratch (the work queue counters, overflow flag and instrumentation words, and the
 // traversal stacks that do not fit in LDS) lives in `scratch`, a file-scope device array of fixed
 // size that every GPU holds for the life of the process. Host code never passes the array's name
 // to a kernel (on the host it is only a stand-in symbol): its device address is looked up per

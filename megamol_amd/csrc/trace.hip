@@ -2,10 +2,10 @@
 // (plugins/optix_hpg/src/optix/AbstractRenderer.cpp:106, cuda_resources/raygen.cu:79-278) and the
 // intersection / closest-hit programs (cuda_resources/sphere.cuh:43-57, 94-131).
 //
-// Launch shape: a persistent grid (blocks_per_cu x CUs blocks of 256 threads). Each wavefront
-// takes 8x8-pixel tiles from a global atomic counter (work stealing) until none are left; a
-// lane owns one pixel and loops over its samples in order, so the per-pixel random stream is the
-// reference's one (TEA seed, two LCG draws per sample for the jitter).
+// Launch shape: a persistent grid (at most blocks_per_cu x CUs blocks of 256 threads). Each wavefront
+// takes 8x8-pixel tiles from work queues until none are left; a lane owns one pixel and loops over
+// its samples in order, so the per-pixel random stream is the reference's one (TEA seed, two LCG
+// draws per sample for the jitter).
 //
 // Traversal: BVH2 with both child boxes in the 64-byte node (four 16-byte loads per visit),
 // ordered front-to-back, the spheres of a leaf reference tested apart from the node visits, two at
@@ -25,7 +25,6 @@ namespace mmhrt {
 namespace {
 
 constexpr int TB = 256;                  // threads per block
-constexpr int STACK_CAP = TRACE_STACK_CAP;  // LDS + spill entries per lane (LBVH height <= 63 + 31)
 
 struct TraceArgs {
     const Node* nodes;
@@ -35,8 +34,9 @@ struct TraceArgs {
     const SceneInfo* info;
     int32_t* spill;
     uint32_t spill_stride;  // lanes in the grid
-    uint32_t* ctr;          // [0] tile counter, [1] overflow flag, [2..11] u64 counters
+    uint32_t* ctr;          // [1] overflow flag, [2..11] u64 counters, from TRACE_QUEUE on the work queues
     uint32_t n_tiles, tiles_x;
+    uint32_t sub_log2;      // k_trace_sl: a unit of work is 1 / (1 << sub_log2) of a tile's passes
     uint32_t tw_log2;  // pixel tile = (1 << tw_log2) x (64 >> tw_log2), one wavefront
     float4* out_col;
     float* out_depth;
@@ -52,26 +52,89 @@ struct TraceArgs {
     uint32_t tl_log2;        // log2 of the treelet size
 };
 
+// The units of work of a launch (tiles, or parts of them), dealt in 8 contiguous bands, one queue
+// per band. A wavefront's first unit is fixed by its number, later ones come from the counter of its
+// own band's queue (workgroups go to the 8 XCDs in turn, so a band stays with one XCD's L2), and when
+// that is used up from the other bands. Every taken unit used to be one atomic on one counter, and
+// those run one after the other, about 10 ns each: 8192 wavefronts that each find out that nothing is
+// left took 90 us by themselves (a 320x240 frame traced in 188 us, in 99 us with fixed tiles), and the
+// refills of a 1080p frame 0.5 ms. All lanes of the wavefront call grab() together.
+struct WorkQueue {
+    uint32_t* q;      // counter of queue k at q[k * TRACE_QUEUE_STRIDE]: units taken beyond the fixed first ones
+    uint32_t total;   // units
+    uint32_t per;     // units per band
+    uint32_t k;       // the queue this wavefront takes from
+    bool first;
+    __device__ __forceinline__ WorkQueue(uint32_t* ctr, uint32_t units)
+        : q(ctr + TRACE_QUEUE), total(units), per((units + 7u) / 8u), k(blockIdx.x & 7u), first(true) {}
+    __device__ __forceinline__ uint32_t size(uint32_t b) const {
+        const uint32_t lo = b * per;
+        return lo >= total ? 0u : (total - lo < per ? total - lo : per);
+    }
+    // wavefronts whose own queue is b: those of the workgroups b, b + 8, ...
+    __device__ __forceinline__ uint32_t owners(uint32_t b) const {
+        return (gridDim.x + 7u - b) / 8u * (TB / 64);
+    }
+    // the next unit, or 0xffffffff when all are taken
+    __device__ __forceinline__ uint32_t grab() {
+        if (first) {
+            first = false;
+            const uint32_t w = (blockIdx.x >> 3) * (TB / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+            if (w < size(k)) return k * per + w;
+        } else {
+            const uint32_t u = take(k);
+            if (u != 0xffffffffu) return u;
+        }
+        for (;;) {  // another queue that has units left, the nearest one on; reads first, they do not queue up
+            const uint32_t lane = __lane_id();
+            const uint32_t b = (k + lane) & 7u;
+            bool left = false;
+            if (lane < 8u)
+                left = owners(b) + __hip_atomic_load(q + b * TRACE_QUEUE_STRIDE, __ATOMIC_RELAXED,
+                                                     __HIP_MEMORY_SCOPE_AGENT) < size(b);
+            const uint64_t m = __ballot(left);
+            if (!m) return 0xffffffffu;
+            k = (k + (uint32_t)__ffsll((unsigned long long)m) - 1u) & 7u;
+            const uint32_t u = take(k);
+            if (u != 0xffffffffu) return u;
+        }
+    }
+    __device__ __forceinline__ uint32_t take(uint32_t b) {
+        uint32_t u = 0;
+        if (__lane_id() == 0) u = atomicAdd(q + b * TRACE_QUEUE_STRIDE, 1u);
+        u = __builtin_amdgcn_readfirstlane(u) + owners(b);
+        return u < size(b) ? b * per + u : 0xffffffffu;
+    }
+};
+
 // Reference of no node: the bottom of a stack. Not a leaf reference, whose k is below 2^31 - 1.
 constexpr int32_t REF_NONE = INT32_MIN;
 
-// Traversal stack of one lane: (reference, entry distance of its box), the lowest S entries in
+// Traversal stack of one lane: (reference, entry distance of its box), the lowest N entries in
 // LDS, lane-interleaved. Deeper entries spill their reference alone to the lane's global words
 // and come back with an entry distance below every ray's (they are visited without the test).
+// With SPILL_DIST in S they spill both words: for the treelets' shallow trees (at most 22 top levels
+// and 10 inside a treelet) the lane's words hold them, and an LDS stack of 8 entries instead of 16
+// keeps two more wavefronts per SIMD.
+constexpr int SPILL_DIST = 256;
 template <int S>
 struct LaneStack {
+    static constexpr int N = S & (SPILL_DIST - 1);
+    static constexpr int W = S & SPILL_DIST ? 2 : 1;                // words per spilled entry
+    static constexpr int CAP = N + TRACE_SPILL_PER_LANE / W;
     int2* lds;  // element k at lds[k * TB]
     int32_t* spill;
     uint32_t stride;
     int sp;
     uint32_t* overflow;
     __device__ __forceinline__ void push(int32_t ref, float tn) {
-        if (__builtin_expect(sp < S, 1)) {
+        if (__builtin_expect(sp < N, 1)) {
             lds[sp * TB] = make_int2(ref, __float_as_int(tn));
-        } else if (sp < STACK_CAP) {
-            spill[(size_t)(sp - S) * stride] = ref;
+        } else if (sp < CAP) {
+            spill[(size_t)(W * (sp - N)) * stride] = ref;
+            if (W == 2) spill[(size_t)(W * (sp - N) + 1) * stride] = __float_as_int(tn);
         } else {
-            *overflow = 1u;  // cannot happen for a valid LBVH; recorded, entry dropped
+            *overflow = 1u;  // cannot happen for a valid tree; recorded, entry dropped
             return;
         }
         ++sp;
@@ -79,8 +142,11 @@ struct LaneStack {
     // the top entry (the stack is not empty)
     __device__ __forceinline__ int2 take() {
         --sp;
-        int2 e = lds[(sp < S ? sp : S - 1) * TB];
-        if (__builtin_expect(sp >= S, 0)) e = make_int2(spill[(size_t)(sp - S) * stride], (int)0xff800000u);
+        int2 e = lds[(sp < N ? sp : N - 1) * TB];
+        if (__builtin_expect(sp >= N, 0)) {
+            e.x = spill[(size_t)(W * (sp - N)) * stride];
+            e.y = W == 2 ? spill[(size_t)(W * (sp - N) + 1) * stride] : (int)0xff800000u;
+        }
         return e;
     }
     // the topmost reference whose box starts no farther than t_best; REF_NONE when there is none
@@ -524,7 +590,7 @@ __device__ int trace_tl(const TraceArgs& A, const RayPre& r, float tmin, float t
                 const float a0 = __int_as_float(e.y);
                 if (a0 <= t_best) {
                     node = e.x;
-                    t0 = fmaxf(a0, 0.0f);  // (a spilled entry carries no distance)
+                    t0 = a0;
                     t1 = t_best;
                     break;
                 }
@@ -728,10 +794,13 @@ __device__ void shade_pixel(const TraceArgs& A, uint32_t px, uint32_t py, float 
 
 // Lane per pixel, samples in a loop (every sample count). Held to 72 VGPRs (7 wavefronts per SIMD),
 // which the fetch latency needs. With the two-phase traversal a frame of 4-bounce paths (1M spheres,
-// 801x600, 1 sample) went from 1.65 to 0.71 ms.
+// 801x600, 1 sample) went from 1.65 to 0.71 ms, with the work queues to 0.61 ms. At 1 sample it now
+// beats the refill kernel, which had been the default there (50M spheres, 1080p AO: 0.88 against 0.70
+// ms; 60M clustered at 4K: 6.7 against 5.7; 10k spheres at 320x240: 92 against 80 us): bound by the
+// vector memory unit's address rate (busy 60-90 %), then by VALU issue (50-70 %).
 template <int S, int MODE, bool COUNT, bool STEAL, bool TL = false>
 __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(7, 8))) void k_trace(TraceArgs A) {
-    __shared__ int2 lds_stack[S * TB];
+    __shared__ int2 lds_stack[LaneStack<S>::N * TB];
     const uint32_t gtid = blockIdx.x * TB + threadIdx.x;
     LaneStack<S> st{lds_stack + threadIdx.x, A.spill + gtid, A.spill_stride, 0, A.ctr + 1};
     Count cnt;
@@ -742,15 +811,9 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(7, 8))) void
     const uint32_t lane = __lane_id();
     const uint32_t gwave = gtid >> 6;
     const uint32_t nwaves = (gridDim.x * TB) >> 6;
+    WorkQueue wq(A.ctr, A.n_tiles);
     for (uint32_t it = 0;; ++it) {
-        uint32_t tile;
-        if (STEAL) {
-            uint32_t t0 = 0;
-            if (lane == 0) t0 = atomicAdd(A.ctr, 1u);
-            tile = __shfl(t0, 0, 64);
-        } else {
-            tile = gwave + it * nwaves;
-        }
+        const uint32_t tile = STEAL ? wq.grab() : gwave + it * nwaves;
         if (tile >= A.n_tiles) break;
         uint32_t tx = tile % A.tiles_x, ty = tile / A.tiles_x;
         const uint32_t tw = 1u << A.tw_log2, th = 64u >> A.tw_log2;
@@ -830,7 +893,7 @@ __device__ __forceinline__ void shade_sample(const TraceArgs& A, uint32_t px, ui
 // wavefronts per SIMD, a few registers spilled) like the other lane kernels.
 template <int S, int MODE, bool COUNT, bool TL = false>
 __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(7, 8))) void k_trace_sl(TraceArgs A) {
-    __shared__ int2 lds_stack[S * TB];
+    __shared__ int2 lds_stack[LaneStack<S>::N * TB];
     const uint32_t gtid = blockIdx.x * TB + threadIdx.x;
     LaneStack<S> st{lds_stack + threadIdx.x, A.spill + gtid, A.spill_stride, 0, A.ctr + 1};
     Count cnt;
@@ -844,13 +907,14 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(7, 8))) void
     const uint32_t g = lane / L, sl = lane % L;
     const uint32_t base = g * L;  // first lane of this lane's pixel group
     const uint32_t tw = 1u << A.tw_log2, th = 64u >> A.tw_log2;
+    const uint32_t passes = L >> A.sub_log2;  // of a unit (a tile has 64 / G = L)
+    WorkQueue wq(A.ctr, A.n_tiles << A.sub_log2);
     for (;;) {
-        uint32_t t0 = 0;
-        if (lane == 0) t0 = atomicAdd(A.ctr, 1u);
-        const uint32_t tile = __shfl(t0, 0, 64);
-        if (tile >= A.n_tiles) break;
+        const uint32_t unit = wq.grab();
+        if (unit == 0xffffffffu) break;
+        const uint32_t tile = unit >> A.sub_log2, q0 = (unit - (tile << A.sub_log2)) * passes;
         const uint32_t tx = tile % A.tiles_x, ty = tile / A.tiles_x;
-        for (uint32_t q = 0; q < 64u / G; ++q) {
+        for (uint32_t q = q0; q < q0 + passes; ++q) {
             const uint32_t tp = q * G + g;  // pixel of this group inside the tile
             const uint32_t px = f.win_x0 + tx * tw + (tp & (tw - 1)), py = f.win_y0 + ty * th + (tp >> A.tw_log2);
             const bool valid = px < f.win_x0 + f.win_w && py < f.win_y0 + f.win_h;
@@ -955,11 +1019,12 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(7, 8))) void
 enum : int { L_IDLE = 0, L_NEED = 1, L_PRIM = 2, L_AO = 3, L_PRIM_DONE = 4, L_AO_DONE = 5, L_OFF = 6 };
 
 // Held to 5 wavefronts per SIMD (at most 102 VGPRs; it takes 96 and spills nothing). Primary and AO
-// rays, which a refilled wavefront holds at once, run one instruction stream.
+// rays, which a refilled wavefront holds at once, run one instruction stream. Off unless the option
+// asks for it (figures at k_trace).
 template <int S, int MODE, bool COUNT>
 __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(5, 8))) void k_trace_refill(TraceArgs A,
                                                                                                 uint32_t refill) {
-    __shared__ int2 lds_stack[S * TB];
+    __shared__ int2 lds_stack[LaneStack<S>::N * TB];
     const uint32_t gtid = blockIdx.x * TB + threadIdx.x;
     LaneStack<S> st{lds_stack + threadIdx.x, A.spill + gtid, A.spill_stride, 0, A.ctr + 1};
     Count cnt;
@@ -968,8 +1033,8 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(5, 8))) void
     const float pad = (fmaxf(f.pad, amax) + amax) * (1.0f / 131072.0f);
     const uint32_t lane = __lane_id();
     const uint32_t tw = 1u << A.tw_log2, th = 64u >> A.tw_log2;
-    const uint32_t tiles_x = (f.win_w + tw - 1) / tw;
-    const uint32_t total_work = ((f.win_h + th - 1) / th) * tiles_x * 64u;  // work indices: whole tiles
+    WorkQueue wq(A.ctr, A.n_tiles);
+    uint32_t tile = 0, used = 64u;  // the wavefront's tile and how many of its pixels are taken
     int state = L_IDLE;
     bool exhausted = false;
     // pixel state
@@ -986,21 +1051,23 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(5, 8))) void
     int32_t node = 0, leaf = REF_NONE;
     float4 alb = make_float4(0.f, 0.f, 0.f, 0.f);
     for (;;) {
-        // 1. idle lanes take pixels (work index -> 8x8 tile order inside the window)
+        // 1. idle lanes take the next pixels of the wavefront's tile, and of a new one when it is used up
         uint64_t idle = __ballot(state == L_IDLE);
-        if (idle && !exhausted) {
-            int leader = __ffsll((unsigned long long)idle) - 1;
-            uint32_t base = 0;
-            if ((int)lane == leader) base = atomicAdd(A.ctr, (uint32_t)__popcll(idle));
-            base = __shfl(base, leader, 64);
-            if (base + (uint32_t)__popcll(idle) >= total_work) exhausted = true;
+        while (idle && !exhausted) {
+            if (used == 64u) {
+                tile = wq.grab();
+                used = 0;
+                if (tile == 0xffffffffu) {
+                    exhausted = true;
+                    break;
+                }
+            }
             if (state == L_IDLE) {
-                uint32_t w = base + (uint32_t)__popcll(idle & ((1ull << lane) - 1ull));
-                uint32_t tile = w >> 6, k = w & 63u;
-                uint32_t tx = tile % tiles_x, ty = tile / tiles_x;
-                uint32_t lx = tx * tw + (k & (tw - 1)), ly = ty * th + (k >> A.tw_log2);
-                // tiles past the window edge map to no pixel; the lane simply asks again
-                if (w < total_work && lx < f.win_w && ly < f.win_h) {
+                const uint32_t k = used + (uint32_t)__popcll(idle & ((1ull << lane) - 1ull));
+                const uint32_t tx = tile % A.tiles_x, ty = tile / A.tiles_x;
+                const uint32_t lx = tx * tw + (k & (tw - 1)), ly = ty * th + (k >> A.tw_log2);
+                // places past the window edge map to no pixel; the lane simply asks again
+                if (k < 64u && lx < f.win_w && ly < f.win_h) {
                     px = f.win_x0 + lx;
                     py = f.win_y0 + ly;
                     pix = py * f.width + px;
@@ -1013,10 +1080,11 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(5, 8))) void
                     vis_sum = 0.0f;
                     aux6 = 0.f;
                     state = L_NEED;
-                } else if (w >= total_work) {
-                    state = L_OFF;
                 }
             }
+            const uint32_t n = (uint32_t)__popcll(idle);
+            used = used + n < 64u ? used + n : 64u;
+            idle = __ballot(state == L_IDLE);
         }
         if (exhausted && state == L_IDLE) state = L_OFF;
         // 2. new primary rays
@@ -1130,75 +1198,98 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(5, 8))) void
     }
 }
 
+// Where and how large a trace launch is: at most `blocks` workgroups on a device of `cus` CUs.
+struct Grid {
+    unsigned blocks, cus;
+    hipStream_t stream;
+};
+
+// A persistent launch of kernel K, of no more workgroups than are resident at once: a workgroup that
+// started only when another had left would find the queues empty but for its wavefronts' own first
+// units, and trace those after everything else (1M spheres, 1 sample: 0.48 -> 0.57 ms).
+template <auto K, typename... Args>
+void launch_resident(const Grid& g, Args... args) {
+    static const unsigned per_cu = [] {
+        int n = 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, K, TB, 0) != hipSuccess || n < 1) {
+            (void)hipGetLastError();
+            n = 1;
+        }
+        return (unsigned)n;
+    }();
+    hipLaunchKernelGGL(K, dim3(std::min(g.blocks, per_cu * g.cus)), dim3(TB), 0, g.stream, args...);
+}
+
 template <int S, int MODE, bool COUNT>
-void launch3(const TraceArgs& A, unsigned grid, bool steal, hipStream_t s) {
+void launch3(const TraceArgs& A, const Grid& g, bool steal) {
     if (steal)
-        hipLaunchKernelGGL((k_trace<S, MODE, COUNT, true>), dim3(grid), dim3(TB), 0, s, A);
+        launch_resident<k_trace<S, MODE, COUNT, true>>(g, A);
     else
-        hipLaunchKernelGGL((k_trace<S, MODE, COUNT, false>), dim3(grid), dim3(TB), 0, s, A);
+        launch_resident<k_trace<S, MODE, COUNT, false>>(g, A);
 }
 template <int S, int MODE>
-void launch2(const TraceArgs& A, unsigned grid, bool steal, bool count, hipStream_t s) {
+void launch2(const TraceArgs& A, const Grid& g, bool steal, bool count) {
     if (count)
-        launch3<S, MODE, true>(A, grid, steal, s);
+        launch3<S, MODE, true>(A, g, steal);
     else
-        launch3<S, MODE, false>(A, grid, steal, s);
+        launch3<S, MODE, false>(A, g, steal);
 }
 template <int S>
-void launch1(const TraceArgs& A, unsigned grid, bool steal, bool count, int mode, hipStream_t s) {
+void launch1(const TraceArgs& A, const Grid& g, bool steal, bool count, int mode) {
     if (mode == 1)
-        launch2<S, 1>(A, grid, steal, count, s);
+        launch2<S, 1>(A, g, steal, count);
     else if (mode == 2)
-        launch2<S, 2>(A, grid, steal, count, s);
+        launch2<S, 2>(A, g, steal, count);
     else
-        launch2<S, 0>(A, grid, steal, count, s);
+        launch2<S, 0>(A, g, steal, count);
 }
 
 template <int S>
-void launch_sl(const TraceArgs& A, unsigned grid, bool count, int mode, hipStream_t s) {
+void launch_sl(const TraceArgs& A, const Grid& g, bool count, int mode) {
     if (mode == 1) {
         if (count)
-            hipLaunchKernelGGL((k_trace_sl<S, 1, true>), dim3(grid), dim3(TB), 0, s, A);
+            launch_resident<k_trace_sl<S, 1, true>>(g, A);
         else
-            hipLaunchKernelGGL((k_trace_sl<S, 1, false>), dim3(grid), dim3(TB), 0, s, A);
+            launch_resident<k_trace_sl<S, 1, false>>(g, A);
     } else {
         if (count)
-            hipLaunchKernelGGL((k_trace_sl<S, 0, true>), dim3(grid), dim3(TB), 0, s, A);
+            launch_resident<k_trace_sl<S, 0, true>>(g, A);
         else
-            hipLaunchKernelGGL((k_trace_sl<S, 0, false>), dim3(grid), dim3(TB), 0, s, A);
+            launch_resident<k_trace_sl<S, 0, false>>(g, A);
     }
 }
 
 // Kernels over the treelet P-k-d trees.
+constexpr int TL_STACK = 8 + SPILL_DIST;
 template <int MODE, bool COUNT>
-void launch_tl_m(const TraceArgs& A, unsigned grid, bool sl, hipStream_t s) {
+void launch_tl_m(const TraceArgs& A, const Grid& g, bool sl) {
     if (sl && MODE != 2)
-        hipLaunchKernelGGL((k_trace_sl<16, MODE == 2 ? 0 : MODE, COUNT, true>), dim3(grid), dim3(TB), 0, s, A);
+        launch_resident<k_trace_sl<TL_STACK, MODE == 2 ? 0 : MODE, COUNT, true>>(g, A);
     else
-        hipLaunchKernelGGL((k_trace<16, MODE, COUNT, true, true>), dim3(grid), dim3(TB), 0, s, A);
+        launch_resident<k_trace<TL_STACK, MODE, COUNT, true, true>>(g, A);
 }
-void launch_tl(const TraceArgs& A, unsigned grid, bool sl, bool count, int mode, hipStream_t s) {
+void launch_tl(const TraceArgs& A, const Grid& g, bool sl, bool count, int mode) {
     if (mode == 1) {
-        if (count) launch_tl_m<1, true>(A, grid, sl, s); else launch_tl_m<1, false>(A, grid, sl, s);
+        if (count) launch_tl_m<1, true>(A, g, sl); else launch_tl_m<1, false>(A, g, sl);
     } else if (mode == 2) {
-        if (count) launch_tl_m<2, true>(A, grid, false, s); else launch_tl_m<2, false>(A, grid, false, s);
+        if (count) launch_tl_m<2, true>(A, g, false); else launch_tl_m<2, false>(A, g, false);
     } else {
-        if (count) launch_tl_m<0, true>(A, grid, sl, s); else launch_tl_m<0, false>(A, grid, sl, s);
+        if (count) launch_tl_m<0, true>(A, g, sl); else launch_tl_m<0, false>(A, g, sl);
     }
 }
 
 template <int S>
-void launch_refill(const TraceArgs& A, unsigned grid, uint32_t refill, bool count, int mode, hipStream_t s) {
+void launch_refill(const TraceArgs& A, const Grid& g, uint32_t refill, bool count, int mode) {
     if (mode == 1) {
         if (count)
-            hipLaunchKernelGGL((k_trace_refill<S, 1, true>), dim3(grid), dim3(TB), 0, s, A, refill);
+            launch_resident<k_trace_refill<S, 1, true>>(g, A, refill);
         else
-            hipLaunchKernelGGL((k_trace_refill<S, 1, false>), dim3(grid), dim3(TB), 0, s, A, refill);
+            launch_resident<k_trace_refill<S, 1, false>>(g, A, refill);
     } else {
         if (count)
-            hipLaunchKernelGGL((k_trace_refill<S, 0, true>), dim3(grid), dim3(TB), 0, s, A, refill);
+            launch_resident<k_trace_refill<S, 0, true>>(g, A, refill);
         else
-            hipLaunchKernelGGL((k_trace_refill<S, 0, false>), dim3(grid), dim3(TB), 0, s, A, refill);
+            launch_resident<k_trace_refill<S, 0, false>>(g, A, refill);
     }
 }
 
@@ -1211,17 +1302,15 @@ template <int S, int MODE, bool TL = false>
 __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(7, 8))) void k_trace_batch(const TraceArgs* __restrict__ jobs,
                                                     const uint32_t* __restrict__ prefix, uint32_t n_jobs,
                                                     uint32_t* ctr) {
-    __shared__ int2 lds_stack[S * TB];
+    __shared__ int2 lds_stack[LaneStack<S>::N * TB];
     const uint32_t gtid = blockIdx.x * TB + threadIdx.x;
     LaneStack<S> st{lds_stack + threadIdx.x, jobs[0].spill + gtid, jobs[0].spill_stride, 0, ctr + 1};
     Count cnt;
     const uint32_t lane = __lane_id();
-    const uint32_t total = prefix[n_jobs];
+    WorkQueue wq(ctr, prefix[n_jobs]);
     for (;;) {
-        uint32_t t0 = 0;
-        if (lane == 0) t0 = atomicAdd(ctr, 1u);
-        const uint32_t tile = __shfl(t0, 0, 64);
-        if (tile >= total) break;
+        const uint32_t tile = wq.grab();
+        if (tile == 0xffffffffu) break;
         // the job holding the tile: the last j with prefix[j] <= tile (binary search: a launch
         // over a whole series holds hundreds of jobs)
         uint32_t j = 0, hi = n_jobs - 1;
@@ -1249,22 +1338,22 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(7, 8))) void
 // One batched launch over jobs that share the mode.
 void launch_trace_batch(mmhrt_ctx_s* c, const void* jobs, const uint32_t* prefix, uint32_t n_jobs, uint32_t* ctr,
                         int mode, bool treelets) {
-    unsigned grid = (unsigned)std::max<int64_t>(1, c->cu_count * c->opt_blocks_per_cu);
+    const Grid g{(unsigned)std::max<int64_t>(1, c->cu_count * c->opt_blocks_per_cu), (unsigned)c->cu_count, c->stream};
     const TraceArgs* J = static_cast<const TraceArgs*>(jobs);
     int S = (int)c->opt_stack_lds;
-    launch_fill_u32(c->stream, ctr, 0u, 16);
-    if (treelets) {  // treelet P-k-d trees: 16-entry LDS stacks
+    launch_fill_u32(c->stream, ctr, 0u, TRACE_CTR_WORDS);
+    if (treelets) {  // treelet P-k-d trees
         if (mode == 1)
-            hipLaunchKernelGGL((k_trace_batch<16, 1, true>), dim3(grid), dim3(TB), 0, c->stream, J, prefix, n_jobs, ctr);
+            launch_resident<k_trace_batch<TL_STACK, 1, true>>(g, J, prefix, n_jobs, ctr);
         else
-            hipLaunchKernelGGL((k_trace_batch<16, 0, true>), dim3(grid), dim3(TB), 0, c->stream, J, prefix, n_jobs, ctr);
+            launch_resident<k_trace_batch<TL_STACK, 0, true>>(g, J, prefix, n_jobs, ctr);
         return;
     }
-#define MMHRT_BATCH(SV)                                                                                     \
-    if (mode == 1)                                                                                          \
-        hipLaunchKernelGGL((k_trace_batch<SV, 1>), dim3(grid), dim3(TB), 0, c->stream, J, prefix, n_jobs, ctr); \
-    else                                                                                                    \
-        hipLaunchKernelGGL((k_trace_batch<SV, 0>), dim3(grid), dim3(TB), 0, c->stream, J, prefix, n_jobs, ctr);
+#define MMHRT_BATCH(SV)                                                     \
+    if (mode == 1)                                                          \
+        launch_resident<k_trace_batch<SV, 1>>(g, J, prefix, n_jobs, ctr);   \
+    else                                                                    \
+        launch_resident<k_trace_batch<SV, 0>>(g, J, prefix, n_jobs, ctr);
     switch (S) {
     case 8: MMHRT_BATCH(4) break;
     case 24: MMHRT_BATCH(12) break;
@@ -1302,6 +1391,7 @@ int batch_fill_job(mmhrt_ctx_s* c, const FrameConsts& fc, size_t out_offset, voi
     A.n_sph = (uint32_t)c->n;
     A.tl_log2 = 0;
     while ((1u << A.tl_log2) < c->pkd_M) ++A.tl_log2;
+    A.sub_log2 = 0;
     A.fc = fc;
     A.fc.want_aux = 0;
     A.fc.accumulate = 0;
@@ -1318,44 +1408,57 @@ uint32_t tile_log2(int64_t tw) {
 }
 
 namespace {
+// Units of work the sample-lanes kernel wants per wavefront. 64-spp AO of 50M spheres at 1080p: 18.4 ms
+// in whole tiles, 15.4, 14.4, 13.8 and 13.8 ms at 4, 8, 16 and 32 (16 spp of 3M spheres at 1000x621:
+// 1.97 ms, then 1.38, 1.35, 1.42, 1.43): the last tiles of 64 passes each ran on an idle device.
+constexpr uint64_t SUB_UNITS = 16;
+
 // Kernel choice for one frame (the same for both entry points): sample-parallel lanes for Lambert
 // and AO with spp a power of two up to 64 or a multiple of 64, the ballot-refill kernel when a
 // refill threshold is set, else the lane-per-pixel kernel.
-void dispatch_trace(mmhrt_ctx_s* c, const TraceArgs& A, unsigned grid, bool count) {
+void dispatch_trace(mmhrt_ctx_s* c, TraceArgs& A, unsigned grid, bool count) {
     const FrameConsts& fc = A.fc;
     int S = (int)c->opt_stack_lds;
     if (S != 8 && S != 16 && S != 24 && S != 32) S = 16;
     bool steal = c->opt_persistent != 0;
-    const int64_t rq = c->opt_refill < 0 ? (fc.spp == 1 ? 16 : 0) : c->opt_refill;
+    const int64_t rq = c->opt_refill;
     uint32_t refill = (uint32_t)std::max<int64_t>(0, std::min<int64_t>(64, rq));
     const bool sl_shape = fc.spp > 1 && ((fc.spp >= 64 && fc.spp % 64 == 0) || (fc.spp < 64 && 64 % fc.spp == 0));
+    const bool sl = c->opt_sample_lanes != 0 && fc.mode != 2 && sl_shape && (c->accel == 1 || refill == 0);
+    // the sample-lanes kernel divides its tiles (min(spp, 64) passes each) until every wavefront
+    // of the full grid has SUB_UNITS units, and no launch has more wavefronts than units
+    if (sl)
+        while ((1u << A.sub_log2) < std::min(fc.spp, 64u) &&
+               ((uint64_t)A.n_tiles << A.sub_log2) < SUB_UNITS * grid * (TB / 64))
+            ++A.sub_log2;
+    const uint64_t need = (((uint64_t)A.n_tiles << A.sub_log2) + TB / 64 - 1) / (TB / 64);
+    const Grid g{(unsigned)std::min<uint64_t>(grid, need), (unsigned)c->cu_count, c->stream};
     if (c->accel == 1) {
         // treelet P-k-d trees: the sample-lanes kernel where the samples fill the lanes, else
-        // lane per pixel with work stealing (16-entry LDS stacks)
-        const bool sl = c->opt_sample_lanes != 0 && fc.mode != 2 && sl_shape;
-        launch_tl(A, grid, sl, count, fc.mode, c->stream);
+        // lane per pixel with work stealing
+        launch_tl(A, g, sl, count, fc.mode);
         return;
     }
-    if (c->opt_sample_lanes != 0 && refill == 0 && fc.mode != 2 && sl_shape) {
+    if (sl) {
         switch (S) {
-        case 8: launch_sl<4>(A, grid, count, fc.mode, c->stream); break;
-        case 24: launch_sl<12>(A, grid, count, fc.mode, c->stream); break;
-        case 32: launch_sl<16>(A, grid, count, fc.mode, c->stream); break;
-        default: launch_sl<8>(A, grid, count, fc.mode, c->stream); break;
+        case 8: launch_sl<4>(A, g, count, fc.mode); break;
+        case 24: launch_sl<12>(A, g, count, fc.mode); break;
+        case 32: launch_sl<16>(A, g, count, fc.mode); break;
+        default: launch_sl<8>(A, g, count, fc.mode); break;
         }
     } else if (refill > 0 && fc.mode != 2) {
         switch (S) {
-        case 8: launch_refill<4>(A, grid, refill, count, fc.mode, c->stream); break;
-        case 24: launch_refill<12>(A, grid, refill, count, fc.mode, c->stream); break;
-        case 32: launch_refill<16>(A, grid, refill, count, fc.mode, c->stream); break;
-        default: launch_refill<8>(A, grid, refill, count, fc.mode, c->stream); break;
+        case 8: launch_refill<4>(A, g, refill, count, fc.mode); break;
+        case 24: launch_refill<12>(A, g, refill, count, fc.mode); break;
+        case 32: launch_refill<16>(A, g, refill, count, fc.mode); break;
+        default: launch_refill<8>(A, g, refill, count, fc.mode); break;
         }
     } else {
         switch (S) {
-        case 8: launch1<4>(A, grid, steal, count, fc.mode, c->stream); break;
-        case 24: launch1<12>(A, grid, steal, count, fc.mode, c->stream); break;
-        case 32: launch1<16>(A, grid, steal, count, fc.mode, c->stream); break;
-        default: launch1<8>(A, grid, steal, count, fc.mode, c->stream); break;
+        case 8: launch1<4>(A, g, steal, count, fc.mode); break;
+        case 24: launch1<12>(A, g, steal, count, fc.mode); break;
+        case 32: launch1<16>(A, g, steal, count, fc.mode); break;
+        default: launch1<8>(A, g, steal, count, fc.mode); break;
         }
     }
 }
@@ -1375,6 +1478,7 @@ void fill_scene_args(mmhrt_ctx_s* c, const FrameConsts& fc, TraceArgs& A) {
     A.tw_log2 = tile_log2(c->opt_tile_w);
     A.tiles_x = (fc.win_w + (1u << A.tw_log2) - 1) >> A.tw_log2;
     A.n_tiles = A.tiles_x * ((fc.win_h + (64u >> A.tw_log2) - 1) / (64u >> A.tw_log2));
+    A.sub_log2 = 0;
     A.fc = fc;
 }
 

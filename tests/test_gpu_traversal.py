@@ -77,3 +77,22 @@ def test_deep_tree_small_stack(gpu_renderer, spp, refill):
         assert gpu_renderer.get_option("stack_overflow") == 0
     finally:
         gpu_renderer.set_option("count_visits", 0)
+
+
+@pytest.mark.parametrize("w,h", [(1, 1), (8, 8), (9, 1), (3, 70), (130, 67)])
+@pytest.mark.parametrize("blocks", [8, 1])
+def test_work_queues(gpu_renderer, w, h, blocks):
+    """Every pixel is rendered whatever the number of tiles is beside the 8 queues and the
+    wavefronts: fewer tiles than queues, tiles divided into units (64 samples), all wavefronts' first
+    units and many more."""
+    xyzr, rgba = scenes.random_spheres(1500, seed=3, rmin=0.02, rmax=0.06)
+    cam = look_at((0.5, 0.5, 2.0), (0.5, 0.5, 0.5), (0, 1, 0), 40.0, w / h, 0.1, 10.0)
+    try:
+        gpu_renderer.set_option("blocks_per_cu", blocks)
+        for spp in (1, 2, 64) if w * h < 2000 else (1, 2):
+            for refill in (0, 16):
+                p = params(w, h, spp=spp, mode=L.MODE_AO, ao_distance=0.3)
+                check(gpu_renderer, xyzr, rgba, cam, p, f"queues {w}x{h} spp {spp} refill {refill} blocks {blocks}",
+                      refill=refill)
+    finally:
+        gpu_renderer.set_option("blocks_per_cu", 8)
