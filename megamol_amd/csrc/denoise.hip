@@ -796,95 +796,150 @@ __global__ __launch_bounds__(256) void k_conv_bwd_data(ConvBwdArgs a) {
 }
 
 // ------------------------------------------------------------------ backward weights
-// dW[t][ci][co] += sum_p X[p + o_t, ci] * G[p, co] over this block's pixel range; one wave per
-// (tap, 16 input channels) and pixel split; K of the MFMA runs over 16 pixels at a time.
+// dW[t][ci][co] += sum_p X[p + o_t, ci] * G[p, co] and db[co] += sum_p G[p, co], G = dY * (Y > 0
+// if relu), with K of v_mfma_f32_16x16x32_bf16 running over 32 pixels of a row. A wavefront takes 16
+// input channels, NB * 16 output channels and all 9 taps (so 9 * NB accumulators) over `rows` output
+// rows of a 32-pixel column strip, and walks down the input rows: per row it stages 34 input pixels
+// and 32 gradient pixels in its own LDS slice as they lie in memory (channels together) and reads
+// them back with pixels along k (the transposing LDS read: 4 pixels of one channel per lane, from any
+// pixel on, which is what the taps' column offsets need). An input row's three fragments (dx) meet the
+// gradients of the rows above, at and below it, whose fragments stay in registers for three rows. The
+// next row's global loads are in flight meanwhile. No barrier: a wavefront's LDS accesses execute in
+// issue order. The bias gradient is one more product per row, with ones as A, in the wavefronts of the
+// first input channels.
+// The kernel before gathered both operands two bytes at a time, once per tap, for one MFMA per 16
+// pixels: 5.4 ms for the 15 layers of a 16 x 128 x 128 batch, and 1.0 ms for the bias kernel beside it.
+__device__ __forceinline__ bf16x8 lds_tr8(const uint16_t* s) {
+    typedef short s16x4 __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) s16x4* lds_s16x4;
+    union {
+        s16x4 h[2];
+        bf16x8 v;
+    } f;
+    f.h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(s));
+    f.h[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(s + 4 * 16));
+    return f.v;
+}
+
+// g where the bf16 in y is above 0 (and no NaN), else 0, for the two values of a word
+__device__ __forceinline__ uint32_t mask_bf16x2(uint32_t g, uint32_t y) {
+    const uint32_t lo = ((y - 1u) & 0xffffu) < 0x7f80u ? 0xffffu : 0u;
+    const uint32_t hi = (((y >> 16) - 1u) & 0xffffu) < 0x7f80u ? 0xffff0000u : 0u;
+    return g & (lo | hi);
+}
+
+constexpr int BW_PX = 32;  // pixels of a strip
 template <int NB>
-__global__ __launch_bounds__(64) void k_conv_bwd_weight(ConvWgtArgs a) {
-    const int lane = __lane_id();
-    const int CC = (a.C1 + a.C2) / 16;
-    const int CC1 = a.C1 / 16;
-    const int t = blockIdx.x / CC, cc = blockIdx.x % CC;
-    const int NBT = a.CO / 16;
-    const int nb0 = blockIdx.z * NB;
-    const int dy = t / 3 - 1, dx = t % 3 - 1;
-    const long P = (long)a.B * a.H * a.W;
-    const long per = (P + gridDim.y - 1) / gridDim.y;
-    const long p0 = (long)blockIdx.y * per;
-    const long p1 = p0 + per < P ? p0 + per : P;
-    f32x4 acc[NB];
+__global__ __launch_bounds__(256) void k_conv_bwd_weight(ConvWgtArgs a, int strips, int segs, int rows) {
+    constexpr int XP = 36 * 16, GP = BW_PX * 16;  // LDS halfs of the input row (34 pixels used) and of one gradient block
+    __shared__ __align__(16) uint16_t lds[4][XP + NB * GP];
+    const int lane = __lane_id(), wave = threadIdx.x >> 6;
+    const long item = (long)blockIdx.x * 4 + wave;
+    if (item >= (long)a.B * strips * segs) return;
+    const int seg = (int)(item % segs), x0 = (int)(item / segs % strips) * BW_PX, b = (int)(item / segs / strips);
+    const int y0 = seg * rows, y1 = y0 + rows < a.H ? y0 + rows : a.H;
+    const int cc = blockIdx.y, CC1 = a.C1 / 16;
+    const int co0 = blockIdx.z * NB * 16;
+    const int q = lane >> 4, lr = lane & 15;
+    uint16_t* sx = lds[wave];
+    uint16_t* sg = sx + XP;
+    // this lane's pieces of 8 channels: pixel lane / 2, half lane & 1 (and for the input row lanes 0-3
+    // also of pixels 32 and 33)
+    const int pp = lane >> 1, ph = (lane & 1) * 8;
+    auto load_x = [&](int r, int px) -> uint4 {
+        const int xx = x0 + px - 1;
+        uint4 v = make_uint4(0u, 0u, 0u, 0u);
+        if (r >= 0 && r < a.H && xx >= 0 && xx < a.W && px < BW_PX + 2) {
+            const uint16_t* s = cc < CC1 ? a.X1 + (((size_t)b * a.H + r) * a.W + xx) * a.C1 + cc * 16
+                                         : a.X2 + (((size_t)b * (a.H >> 1) + (r >> 1)) * (a.W >> 1) + (xx >> 1)) * a.C2 +
+                                               (cc - CC1) * 16;
+            v = *reinterpret_cast<const uint4*>(s + ph);
+        }
+        return v;
+    };
+    uint4 xq0, xq1, gq[NB], yq[NB];
+    auto load_row = [&](int r) {  // input row r and gradient row r + 1
+        xq0 = load_x(r, pp);
+        xq1 = make_uint4(0u, 0u, 0u, 0u);
+        if (lane < 4) xq1 = load_x(r, BW_PX + pp);
+        const int y = r + 1, x = x0 + pp;
+        const bool in = y >= y0 && y < y1 && x < a.W;
+        const size_t o = (((size_t)b * a.H + y) * a.W + x) * a.CO + co0 + ph;
 #pragma unroll
-    for (int j = 0; j < NB; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int kq = lane >> 4, lr = lane & 15;
-    for (long base = p0; base < p1; base += 16) {
-        Frag fa;
-        Frag fg[NB];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            long p = base + kq * 4 + e;
-            uint16_t xv = 0;
-            bool in = p < p1;
-            int b = 0, y = 0, x = 0;
+        for (int j = 0; j < NB; ++j) {
+            gq[j] = make_uint4(0u, 0u, 0u, 0u);
+            yq[j] = gq[j];
             if (in) {
-                x = (int)(p % a.W);
-                long r = p / a.W;
-                y = (int)(r % a.H);
-                b = (int)(r / a.H);
-                int yy = y + dy, xx = x + dx;
-                if (yy >= 0 && yy < a.H && xx >= 0 && xx < a.W) {
-                    if (cc < CC1)
-                        xv = a.X1[(((size_t)b * a.H + yy) * a.W + xx) * a.C1 + cc * 16 + lr];
-                    else
-                        xv = a.X2[(((size_t)b * (a.H >> 1) + (yy >> 1)) * (a.W >> 1) + (xx >> 1)) * a.C2 +
-                                  (cc - CC1) * 16 + lr];
-                }
-            }
-            fa.h[e] = xv;
-#pragma unroll
-            for (int j = 0; j < NB; ++j) {
-                int nb = nb0 + j;
-                uint16_t gv = 0;
-                if (in && nb < NBT) {
-                    size_t o = (size_t)p * a.CO + nb * 16 + lr;
-                    gv = a.dY[o];
-                    if (a.relu && !(bf2f(a.Y[o]) > 0.0f)) gv = 0;
-                }
-                fg[j].h[e] = gv;
+                gq[j] = *reinterpret_cast<const uint4*>(a.dY + o + j * 16);
+                if (a.relu) yq[j] = *reinterpret_cast<const uint4*>(a.Y + o + j * 16);
             }
         }
-        // A = X^T (rows: 16 input channels, k: 16 pixels), B = G (k: 16 pixels, columns: 16 outputs)
+    };
+    f32x4 acc[9][NB], accb[NB];
+    bf16x8 gm[NB], g0[NB], gp[NB];  // gradients of the rows above, at and below the input row
+    bf16x8 ones;
 #pragma unroll
-        for (int j = 0; j < NB; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(fa.v, fg[j].v, acc[j], 0, 0, 0);
+    for (int e = 0; e < 8; ++e) ones[e] = (__bf16)1.0f;
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+#pragma unroll
+        for (int t = 0; t < 9; ++t) acc[t][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        accb[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int e = 0; e < 8; ++e) g0[j][e] = gp[j][e] = (__bf16)0.0f;
     }
-    // result rows = input channels 4*kq+e, column = output channel lr
+    load_row(y0 - 1);
+    for (int r = y0 - 1; r <= y1; ++r) {
+        *reinterpret_cast<uint4*>(sx + pp * 16 + ph) = xq0;
+        if (lane < 4) *reinterpret_cast<uint4*>(sx + (BW_PX + pp) * 16 + ph) = xq1;
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+            uint4 g = gq[j];
+            if (a.relu)
+                g = make_uint4(mask_bf16x2(g.x, yq[j].x), mask_bf16x2(g.y, yq[j].y), mask_bf16x2(g.z, yq[j].z),
+                               mask_bf16x2(g.w, yq[j].w));
+            *reinterpret_cast<uint4*>(sg + j * GP + pp * 16 + ph) = g;
+        }
+        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+        if (r < y1) load_row(r + 1);
+        // fragments: lane (q, lr) takes channel lr of pixels 8q .. 8q + 7, each 16-lane group reading
+        // 4 pixels x 16 channels at once
+        const int fo = (8 * q + (lr >> 2)) * 16 + 4 * (lr & 3);
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+            gm[j] = g0[j];
+            g0[j] = gp[j];
+            gp[j] = lds_tr8(sg + j * GP + fo);
+        }
+        if (r >= 0 && r < a.H) {
+#pragma unroll
+            for (int dx = 0; dx < 3; ++dx) {
+                const bf16x8 x = lds_tr8(sx + fo + dx * 16);
+#pragma unroll
+                for (int j = 0; j < NB; ++j) {
+                    acc[dx][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, gp[j], acc[dx][j], 0, 0, 0);
+                    acc[3 + dx][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, g0[j], acc[3 + dx][j], 0, 0, 0);
+                    acc[6 + dx][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, gm[j], acc[6 + dx][j], 0, 0, 0);
+                }
+            }
+        }
+        if (cc == 0) {
+#pragma unroll
+            for (int j = 0; j < NB; ++j) accb[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, gp[j], accb[j], 0, 0, 0);
+        }
+        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    }
+    // result rows = input channels 4q + e, column = output channel lr
     const int CI = a.C1 + a.C2;
 #pragma unroll
     for (int j = 0; j < NB; ++j) {
-        int nb = nb0 + j;
-        if (nb >= NBT) break;
+        const int co = co0 + j * 16 + lr;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            int ci = cc * 16 + kq * 4 + e;
-            atomicAdd(a.dW + ((size_t)t * CI + ci) * a.CO + nb * 16 + lr, acc[j][e]);
-        }
+        for (int t = 0; t < 9; ++t)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) atomicAdd(a.dW + ((size_t)t * CI + cc * 16 + q * 4 + e) * a.CO + co, acc[t][j][e]);
+        if (cc == 0 && q == 0) atomicAdd(a.db + co, accb[j][0]);
     }
-}
-
-// bias gradient: db[co] = sum_p G[p, co]
-__global__ __launch_bounds__(256) void k_bias_grad(const uint16_t* __restrict__ dY, const uint16_t* __restrict__ Y,
-                                                   int relu, long P, int CO, float* db) {
-    int co = blockIdx.y;
-    float s = 0.0f;
-    for (long p = (long)blockIdx.x * blockDim.x + threadIdx.x; p < P; p += (long)gridDim.x * blockDim.x) {
-        size_t o = (size_t)p * CO + co;
-        float g = bf2f(dY[o]);
-        if (relu && !(bf2f(Y[o]) > 0.0f)) g = 0.0f;
-        s += g;
-    }
-    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-    __shared__ float ws[4];
-    if (__lane_id() == 0) ws[threadIdx.x >> 6] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) atomicAdd(db + co, ws[0] + ws[1] + ws[2] + ws[3]);
 }
 
 // ------------------------------------------------------------------ pooling / concat split
@@ -1341,20 +1396,26 @@ static void conv_bwd_data(hipStream_t s, const ConvBwdArgs& a) {
     }
 }
 
-static void conv_bwd_weight(hipStream_t s, const ConvWgtArgs& a, int cu) {
-    int CC = (a.C1 + a.C2) / 16;
-    int NBT = a.CO / 16;
-    int nb = NBT <= 6 ? NBT : 4;
-    long P = (long)a.B * a.H * a.W;
-    int splits = (int)std::max<long>(1, std::min<long>((long)cu * 8 / (9 * CC), (P + 1023) / 1024));
-    dim3 g(9 * CC, splits, (NBT + nb - 1) / nb);
+// Wavefronts of a weight-gradient launch: fewer leave CUs idle, more spend their time on the sums they
+// add to memory (whole training step of a 16 x 128 x 128 batch at 8192, 4096, 2048, 1024, 512, 256:
+// 3.07, 2.98, 2.58, 2.26-2.41, 2.24, 2.46 ms; 8.24 ms with the kernel before).
+constexpr long BW_WAVES = 1024;
+static void conv_bwd_weight(hipStream_t s, const ConvWgtArgs& a) {
+    const int CC = (a.C1 + a.C2) / 16;
+    // output channel blocks of a wavefront: 3 or 2 (every width but the 16-channel output is a
+    // multiple of 48 or 32)
+    const int nb = a.CO % 48 == 0 ? 3 : (a.CO % 32 == 0 ? 2 : 1);
+    const int groups = a.CO / 16 / nb, strips = (a.W + BW_PX - 1) / BW_PX;
+    // rows of a wavefront: as many as leave BW_WAVES wavefronts (each one adds 9 * 16 * 16 * nb sums to
+    // memory at its end), and at least 4 (it reads two input rows more than it has)
+    const long per_row = (long)a.B * strips * CC * groups;
+    const int rows = (int)std::max<long>(4, std::min<long>(a.H, (per_row * a.H + BW_WAVES - 1) / BW_WAVES));
+    const int segs = (a.H + rows - 1) / rows;
+    const dim3 g((unsigned)(((long)a.B * strips * segs + 3) / 4), CC, groups);
     switch (nb) {
-    case 1: hipLaunchKernelGGL(k_conv_bwd_weight<1>, g, dim3(64), 0, s, a); break;
-    case 2: hipLaunchKernelGGL(k_conv_bwd_weight<2>, g, dim3(64), 0, s, a); break;
-    case 3: hipLaunchKernelGGL(k_conv_bwd_weight<3>, g, dim3(64), 0, s, a); break;
-    case 4: hipLaunchKernelGGL(k_conv_bwd_weight<4>, g, dim3(64), 0, s, a); break;
-    case 5: hipLaunchKernelGGL(k_conv_bwd_weight<5>, g, dim3(64), 0, s, a); break;
-    default: hipLaunchKernelGGL(k_conv_bwd_weight<6>, g, dim3(64), 0, s, a); break;
+    case 1: hipLaunchKernelGGL(k_conv_bwd_weight<1>, g, dim3(256), 0, s, a, strips, segs, rows); break;
+    case 2: hipLaunchKernelGGL(k_conv_bwd_weight<2>, g, dim3(256), 0, s, a, strips, segs, rows); break;
+    default: hipLaunchKernelGGL(k_conv_bwd_weight<3>, g, dim3(256), 0, s, a, strips, segs, rows); break;
     }
 }
 
@@ -1492,7 +1553,7 @@ void Denoiser::forward(hipStream_t s, int B, int Hp, int Wp) {
 
 // Backward pass. dOut (bf16 [B,Hp,Wp,16]) must be in the first P0*16 halfs of gbuf; weight and
 // bias gradients are accumulated into `grads` (zero it first).
-void Denoiser::backward(hipStream_t s, int B, int Hp, int Wp, int cu) {
+void Denoiser::backward(hipStream_t s, int B, int Hp, int Wp) {
     int Hs[4] = {Hp, Hp / 2, Hp / 4, Hp / 8}, Ws[4] = {Wp, Wp / 2, Wp / 4, Wp / 8};
     size_t P0 = (size_t)B * Hp * Wp;
     const int lvl[kNumLayers] = {0, 0, 1, 1, 2, 2, 3, 3, 2, 2, 1, 1, 0, 0, 0};
@@ -1532,10 +1593,8 @@ void Denoiser::backward(hipStream_t s, int B, int Hp, int Wp, int cu) {
         ConvWgtArgs wa{};
         wa.X1 = in1[l]; wa.X2 = in2[l]; wa.C1 = L.c1; wa.C2 = L.c2; wa.CO = L.co;
         wa.B = B; wa.H = H; wa.W = W; wa.dY = cur; wa.Y = Y; wa.relu = L.relu; wa.dW = grads.p + poff[l];
-        conv_bwd_weight(s, wa, cu);
-        long P = (long)B * H * W;
-        hipLaunchKernelGGL(k_bias_grad, dim3((unsigned)std::min<long>(nblk(P), 256), L.co), dim3(256), 0, s, cur, Y,
-                           L.relu, P, L.co, grads.p + poff[l] + 9ull * CI * L.co);
+        wa.db = grads.p + poff[l] + 9ull * CI * L.co;
+        conv_bwd_weight(s, wa);
         if (l == 0) break;
         uint16_t* dx = free_tmp(cur, nullptr);
         ConvBwdArgs ba{};
@@ -1722,7 +1781,7 @@ int32_t mmhrt_denoiser_train_step(mmhrt_ctx c, const uint16_t* feats, const floa
         return e;
     size_t n = mmhrt::dn::param_count();
     mmhrt::dn::zero(s, d.grads.p, (long)n);
-    d.backward(s, (int)b, ceil8((int)h), ceil8((int)w), c->cu_count);
+    d.backward(s, (int)b, ceil8((int)h), ceil8((int)w));
     if (grads_out) {
         he = hipMemcpyAsync(grads_out, d.grads.p, n * 4, hipMemcpyDeviceToHost, s);
         if (he != hipSuccess) return mmhrt::hip_fail(c, he, "train_step grads");

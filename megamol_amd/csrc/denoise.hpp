@@ -55,6 +55,7 @@ struct ConvWgtArgs {
     const uint16_t* Y;
     int relu;
     float* dW;
+    float* db;
 };
 
 struct Denoiser {
@@ -80,7 +81,7 @@ struct Denoiser {
     int ensure_acts(mmhrt_ctx_s* c, int B, int Hp, int Wp, bool train);
     void relayout(hipStream_t s);
     void forward(hipStream_t s, int B, int Hp, int Wp);
-    void backward(hipStream_t s, int B, int Hp, int Wp, int cu);
+    void backward(hipStream_t s, int B, int Hp, int Wp);
     void release_all();
 };
 

@@ -93,6 +93,30 @@ def test_gradients_match_reference(dnz):
     assert np.array_equal(dnz.get_params(), p), "apply=0 must not update the parameters"
 
 
+@pytest.mark.parametrize("shape", [(1, 8, 8), (2, 9, 33), (1, 40, 24), (3, 16, 72), (1, 130, 40)])
+def test_gradients_at_strip_edges(dnz, shape):
+    """Weight and bias gradients where the 32-pixel strips and the row segments of the gradient
+    kernels end: images of one strip and less, widths past a multiple of 32, padded sizes, rows that
+    are divided among wavefronts. Bounds as in the test above."""
+    case(f"denoiser gradients {shape}")
+    b, h, w = shape
+    feats = random_features(b, h, w, seed=h + w)
+    target = np.random.default_rng(4).random((b, h, w, 3)).astype(np.float32)
+    p = (dnz.p0 + np.random.default_rng(6).normal(size=dnz.p0.shape).astype(np.float32) * 0.02).astype(np.float32)
+    dnz.set_params(p)
+    loss, g = dnz.train_step(feats, target, 2.0, lr=0.0, apply=False, want_grads=True)
+    rloss, rg, _ = R.loss_and_grads(p, feats, target, 2.0, "float32", round_bf16=True)
+    _, eg, _ = R.loss_and_grads(p, feats, target, 2.0, "float64", round_bf16=False)
+    assert abs(loss - rloss) <= 2e-2 * rloss
+    o = 0
+    for name, c1, c2, co, _ in D.LAYERS:
+        n = 9 * (c1 + c2) * co + co
+        gg, rr, ee = g[o:o + n], rg[o:o + n], eg[o:o + n]
+        o += n
+        assert rel(gg, ee) < max(1.2 * rel(rr, ee), 1e-3), (name, rel(gg, ee), rel(rr, ee))
+        assert rel(gg, rr) < 2e-2, (name, rel(gg, rr))
+
+
 def test_frame_path_equals_feature_path(gpu_renderer):
     """mmhrt_denoise on a rendered frame (its features packed into the network input on the device
     in one pass, colours composed into the framebuffer) gives the same colours, bit for bit, as
