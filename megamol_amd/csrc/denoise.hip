@@ -733,21 +733,22 @@ __device__ __forceinline__ uint32_t mask_bf16x2(uint32_t g, uint32_t y) {
 // dXc[p, ci] = sum_t sum_co G[p - o_t, co] * W[t][ci][co], G = dY * (Y > 0 if relu).
 // dXc is [B,H,W,CI] bf16 (full-resolution concatenated input gradient).
 // Wb: weights in fragment order [tap][co/16][ci/16][ci%16][co%16].
-// A workgroup computes 16 blocks of 16 pixels (64 x 4, 32 x 8 or 16 x 16 pixels, as the image's width
-// wastes least) against NB * 16 input channels; it stages the masked gradient of those pixels and a
-// one-pixel border once in LDS, all CO = 16 KC channels of it, and each wavefront takes 4 blocks. A
+// A workgroup computes 4 NI blocks of 16 pixels (for NI = 4 64 x 4, 32 x 8 or 16 x 16 pixels, as the
+// image's size wastes least) against NB * 16 input channels; it stages the masked gradient of those
+// pixels and a one-pixel border once in LDS, all CO = 16 KC channels of it, and each wavefront takes NI
+// blocks. A
 // pixel's channels are padded to an odd multiple of 32 bytes, so that the 16 pixels of a fragment
 // read lie in different banks. The weights are the MFMA's A operand, so that a lane's results are 4
 // adjacent channels of one pixel. The order of the sum (taps, then 16 channels at a time) is that of
 // the kernel before, which fetched and masked every fragment from global memory once per tap, one
-// output row per wavefront, and stored two bytes at a time: 0.93 -> 0.2 ms for the 14 layers of a
+// output row per wavefront, and stored two bytes at a time: 0.93 -> 0.28 ms for the 14 layers of a
 // 16 x 128 x 128 batch.
-constexpr int BD_PX = 6 * 66;  // pixels of the largest staged tile (64 x 4 and its border)
-template <int KC, int NB>
+template <int KC, int NB, int NI>
 __global__ __launch_bounds__(256) void k_conv_bwd_data(ConvBwdArgs a, int pbl, int tiles_x, int tiles_y) {
     constexpr int SP = 16 * KC + (KC % 2 ? 0 : 16);  // halfs per staged pixel
-    __shared__ __align__(16) uint16_t lds[BD_PX * SP];
-    const int TW = 16 << pbl, TH = 16 >> pbl, LW = TW + 2;
+    constexpr int PX = NI == 4 ? 6 * 66 : 3 * 66;  // the largest staged tile: 64 x NI and its border
+    __shared__ __align__(16) uint16_t lds[PX * SP];
+    const int TW = 16 << pbl, TH = (4 * NI) >> pbl, LW = TW + 2;
     const int tile = (int)blockIdx.x;
     const int tx = tile % tiles_x, ty = tile / tiles_x % tiles_y, b = tile / (tiles_x * tiles_y);
     const int nb0 = blockIdx.y * NB, NBT = a.CI / 16;
@@ -771,40 +772,40 @@ __global__ __launch_bounds__(256) void k_conv_bwd_data(ConvBwdArgs a, int pbl, i
     __syncthreads();
     const int lane = __lane_id(), wave = threadIdx.x >> 6;
     const int q = lane >> 4, lr = lane & 15;
-    int src[4];  // staged place of the lane's pixel in each block, channel 4q
+    int src[NI];  // staged place of the lane's pixel in each block, channel 4q
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int k = wave * 4 + i;
+    for (int i = 0; i < NI; ++i) {
+        const int k = wave * NI + i;
         src[i] = (((k >> pbl) + 1) * LW + (k & ((1 << pbl) - 1)) * 16 + lr + 1) * SP + q * 4;
     }
     const uint16_t* wt[NB];
 #pragma unroll
     for (int j = 0; j < NB; ++j) wt[j] = a.Wt + ((size_t)(nb0 + j < NBT ? nb0 + j : NBT - 1) * 16 + lr) * 16 + q * 4;
     const size_t wstep = (size_t)NBT * 256;  // weights of one tap and 16 channels
-    f32x4 acc[4][NB];
+    f32x4 acc[NI][NB];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < NI; ++i)
 #pragma unroll
         for (int j = 0; j < NB; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     for (int t = 0; t < 9; ++t) {
         const int off = -((t / 3 - 1) * LW + t % 3 - 1) * SP;
 #pragma unroll
         for (int kc = 0; kc < KC; ++kc) {
-            Frag fg[4], fw[NB];
+            Frag fg[NI], fw[NB];
 #pragma unroll
             for (int j = 0; j < NB; ++j) fw[j].u = *reinterpret_cast<const uint2*>(wt[j] + (size_t)(t * KC + kc) * wstep);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) fg[i].u = *reinterpret_cast<const uint2*>(lds + src[i] + off + kc * 16);
+            for (int i = 0; i < NI; ++i) fg[i].u = *reinterpret_cast<const uint2*>(lds + src[i] + off + kc * 16);
 #pragma unroll
             for (int j = 0; j < NB; ++j)
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
+                for (int i = 0; i < NI; ++i)
                     acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(fw[j].v, fg[i].v, acc[i][j], 0, 0, 0);
         }
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int k = wave * 4 + i;
+    for (int i = 0; i < NI; ++i) {
+        const int k = wave * NI + i;
         const int y = ty * TH + (k >> pbl), x = tx * TW + (k & ((1 << pbl) - 1)) * 16 + lr;
         if (y >= a.H || x >= a.W) continue;
         uint16_t* d = a.dX + (((size_t)b * a.H + y) * a.W + x) * a.CI + q * 4;
@@ -847,16 +848,23 @@ constexpr int BW_PX = 32;  // pixels of a strip
 template <int NB>
 __global__ __launch_bounds__(256) void k_conv_bwd_weight(ConvWgtArgs a, int strips, int segs, int rows) {
     constexpr int XP = 36 * 16, GP = BW_PX * 16;  // LDS halfs of the input row (34 pixels used) and of one gradient block
-    __shared__ __align__(16) uint16_t lds[4][XP + NB * GP];
+    constexpr int SUMS = (9 * NB + 1) * 256;  // a wavefront's sums: [9 taps x NB and, in 16 * NB of the last 256, bias]
+    union Lds {
+        uint16_t stage[4][XP + NB * GP];
+        float sum[SUMS];
+    };
+    __shared__ __align__(16) Lds u;
     const int lane = __lane_id(), wave = threadIdx.x >> 6;
-    const long item = (long)blockIdx.x * 4 + wave;
-    if (item >= (long)a.B * strips * segs) return;
+    const long items = (long)a.B * strips * segs;
+    long item = (long)blockIdx.x * 4 + wave;
+    const bool some = item < items;
+    if (!some) item = items - 1;  // (a wavefront past the last item adds nothing)
     const int seg = (int)(item % segs), x0 = (int)(item / segs % strips) * BW_PX, b = (int)(item / segs / strips);
     const int y0 = seg * rows, y1 = y0 + rows < a.H ? y0 + rows : a.H;
     const int cc = blockIdx.y, CC1 = a.C1 / 16;
     const int co0 = blockIdx.z * NB * 16;
     const int q = lane >> 4, lr = lane & 15;
-    uint16_t* sx = lds[wave];
+    uint16_t* sx = u.stage[wave];
     uint16_t* sg = sx + XP;
     // this lane's pieces of 8 channels: pixel lane / 2, half lane & 1 (and for the input row lanes 0-3
     // also of pixels 32 and 33)
@@ -903,8 +911,8 @@ __global__ __launch_bounds__(256) void k_conv_bwd_weight(ConvWgtArgs a, int stri
 #pragma unroll
         for (int e = 0; e < 8; ++e) g0[j][e] = gp[j][e] = (__bf16)0.0f;
     }
-    load_row(y0 - 1);
-    for (int r = y0 - 1; r <= y1; ++r) {
+    if (some) load_row(y0 - 1);
+    for (int r = y0 - 1; some && r <= y1; ++r) {
         *reinterpret_cast<uint4*>(sx + pp * 16 + ph) = xq0;
         if (lane < 4) *reinterpret_cast<uint4*>(sx + (BW_PX + pp) * 16 + ph) = xq1;
 #pragma unroll
@@ -944,17 +952,34 @@ __global__ __launch_bounds__(256) void k_conv_bwd_weight(ConvWgtArgs a, int stri
         }
         __atomic_signal_fence(__ATOMIC_SEQ_CST);
     }
-    // result rows = input channels 4q + e, column = output channel lr
-    const int CI = a.C1 + a.C2;
-#pragma unroll
-    for (int j = 0; j < NB; ++j) {
-        const int co = co0 + j * 16 + lr;
+    // the four wavefronts' sums are added in LDS, one after the other, and leave as one set of atomics.
+    // Result rows = input channels 4q + e, column = output channel lr.
+    for (int w = 0; w < 4; ++w) {
+        __syncthreads();  // the first one also ends the staging
+        if (wave != w) continue;
 #pragma unroll
         for (int t = 0; t < 9; ++t)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) atomicAdd(a.dW + ((size_t)t * CI + cc * 16 + q * 4 + e) * a.CO + co, acc[t][j][e]);
-        if (cc == 0 && q == 0) atomicAdd(a.db + co, accb[j][0]);
+            for (int j = 0; j < NB; ++j)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    float* d = u.sum + (t * NB + j) * 256 + (q * 4 + e) * 16 + lr;
+                    *d = w ? *d + acc[t][j][e] : acc[t][j][e];
+                }
+        if (cc == 0 && q == 0)
+#pragma unroll
+            for (int j = 0; j < NB; ++j) {
+                float* d = u.sum + 9 * NB * 256 + j * 16 + lr;
+                *d = w ? *d + accb[j][0] : accb[j][0];
+            }
     }
+    __syncthreads();
+    const int CI = a.C1 + a.C2;
+    for (int i = threadIdx.x; i < 9 * NB * 256; i += 256) {
+        const int t = i / (NB * 256), j = i / 256 % NB, ci = i / 16 % 16, co = i % 16;
+        atomicAdd(a.dW + ((size_t)t * CI + cc * 16 + ci) * a.CO + co0 + j * 16 + co, u.sum[i]);
+    }
+    if (cc == 0 && threadIdx.x < 16 * NB) atomicAdd(a.db + co0 + threadIdx.x, u.sum[9 * NB * 256 + threadIdx.x]);
 }
 
 // ------------------------------------------------------------------ pooling / concat split
@@ -1410,42 +1435,56 @@ static void conv_fwd(hipStream_t s, const ConvArgs& a, bool k32, int shape) {
     }
 }
 
-template <int KC>
+// Below this many workgroups of 16 blocks the data gradients take 4 blocks per workgroup (training step
+// of a 16 x 128 x 128 batch at 0, 256, 512, 1024: 1.72, 1.53, 1.53, 1.53 ms).
+constexpr long BD_FEW = 512;
+template <int KC, int NI>
 static void launch_bwd_data(hipStream_t s, const ConvBwdArgs& a, int nb, int pbl, int tx, int ty, dim3 g) {
     switch (nb) {
-    case 2: hipLaunchKernelGGL((k_conv_bwd_data<KC, 2>), g, dim3(256), 0, s, a, pbl, tx, ty); break;
-    case 3: hipLaunchKernelGGL((k_conv_bwd_data<KC, 3>), g, dim3(256), 0, s, a, pbl, tx, ty); break;
-    case 4: hipLaunchKernelGGL((k_conv_bwd_data<KC, 4>), g, dim3(256), 0, s, a, pbl, tx, ty); break;
-    default: hipLaunchKernelGGL((k_conv_bwd_data<KC, 5>), g, dim3(256), 0, s, a, pbl, tx, ty); break;
+    case 2: hipLaunchKernelGGL((k_conv_bwd_data<KC, 2, NI>), g, dim3(256), 0, s, a, pbl, tx, ty); break;
+    case 3: hipLaunchKernelGGL((k_conv_bwd_data<KC, 3, NI>), g, dim3(256), 0, s, a, pbl, tx, ty); break;
+    case 4: hipLaunchKernelGGL((k_conv_bwd_data<KC, 4, NI>), g, dim3(256), 0, s, a, pbl, tx, ty); break;
+    default: hipLaunchKernelGGL((k_conv_bwd_data<KC, 5, NI>), g, dim3(256), 0, s, a, pbl, tx, ty); break;
+    }
+}
+template <int NI>
+static void conv_bwd_data_t(hipStream_t s, const ConvBwdArgs& a, int nb, int groups) {
+    // tile shape: the one whose tiles cover the image with the fewest pixels, the widest on a tie
+    int pbl = 2;
+    auto area = [&](int l) {
+        const long w = 16 << l, h = (4 * NI) >> l;
+        return (a.W + w - 1) / w * w * ((a.H + h - 1) / h * h);
+    };
+    for (int l = 1; l >= 0; --l)
+        if (area(l) < area(pbl)) pbl = l;
+    const int th = (4 * NI) >> pbl;
+    const int tx = (a.W + (16 << pbl) - 1) / (16 << pbl), ty = (a.H + th - 1) / th;
+    const dim3 g((unsigned)((long)a.B * tx * ty), groups);
+    switch (a.CO / 16) {
+    case 1: launch_bwd_data<1, NI>(s, a, nb, pbl, tx, ty, g); break;
+    case 2: launch_bwd_data<2, NI>(s, a, nb, pbl, tx, ty, g); break;
+    case 3: launch_bwd_data<3, NI>(s, a, nb, pbl, tx, ty, g); break;
+    case 4: launch_bwd_data<4, NI>(s, a, nb, pbl, tx, ty, g); break;
+    default: launch_bwd_data<6, NI>(s, a, nb, pbl, tx, ty, g); break;
     }
 }
 static void conv_bwd_data(hipStream_t s, const ConvBwdArgs& a) {
     const int NBT = a.CI / 16;
     // input-channel blocks of a workgroup: all of them up to 5, else in equal groups (6: 3 + 3, 7: 4 + 3,
     // 10: 5 + 5)
-    const int nb = NBT <= 5 ? std::max(NBT, 2) : (NBT + 1) / 2;
-    // tile shape: the one whose tiles cover the image with the fewest pixels, the widest on a tie
-    int pbl = 2;
-    auto area = [&](int l) {
-        const long w = 16 << l, h = 16 >> l;
-        return (a.W + w - 1) / w * w * ((a.H + h - 1) / h * h);
-    };
-    for (int l = 1; l >= 0; --l)
-        if (area(l) < area(pbl)) pbl = l;
-    const int tx = (a.W + (16 << pbl) - 1) / (16 << pbl), ty = (a.H + (16 >> pbl) - 1) / (16 >> pbl);
-    const dim3 g((unsigned)((long)a.B * tx * ty), (NBT + nb - 1) / nb);
-    switch (a.CO / 16) {
-    case 1: launch_bwd_data<1>(s, a, nb, pbl, tx, ty, g); break;
-    case 2: launch_bwd_data<2>(s, a, nb, pbl, tx, ty, g); break;
-    case 3: launch_bwd_data<3>(s, a, nb, pbl, tx, ty, g); break;
-    case 4: launch_bwd_data<4>(s, a, nb, pbl, tx, ty, g); break;
-    default: launch_bwd_data<6>(s, a, nb, pbl, tx, ty, g); break;
-    }
+    int nb = NBT <= 5 ? std::max(NBT, 2) : (NBT + 1) / 2;
+    int groups = (NBT + nb - 1) / nb;
+    // one block per wavefront, and 2 channel blocks per workgroup, where 4 would leave CUs without
+    // work (fewer than BD_FEW workgroups): the coarse levels of a batch of crops
+    const long wgs = (long)a.B * a.H * a.W / 256 * groups;
+    if (wgs >= BD_FEW) return conv_bwd_data_t<4>(s, a, nb, groups);
+    nb = 2;
+    conv_bwd_data_t<1>(s, a, nb, (NBT + nb - 1) / nb);
 }
 
-// Wavefronts of a weight-gradient launch: fewer leave CUs idle, more spend their time on the sums they
-// add to memory (whole training step of a 16 x 128 x 128 batch at 8192, 4096, 2048, 1024, 512, 256:
-// 3.07, 2.98, 2.58, 2.26-2.41, 2.24, 2.46 ms; 8.24 ms with the kernel before).
+// Wavefronts of a weight-gradient launch: fewer leave CUs idle, more spend their time on the sums that
+// each four of them add to memory (training step of a 16 x 128 x 128 batch at 8192, 4096, 2048, 1024,
+// 768, 512: 1.58, 1.53, 1.45, 1.40, 1.37, 1.47 ms; with every wavefront's sums as atomics 1.71 at 1024).
 constexpr long BW_WAVES = 1024;
 static void conv_bwd_weight(hipStream_t s, const ConvWgtArgs& a) {
     const int CC = (a.C1 + a.C2) / 16;

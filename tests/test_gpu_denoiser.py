@@ -117,6 +117,22 @@ def test_gradients_at_strip_edges(dnz, shape):
         assert rel(gg, rr) < 2e-2, (name, rel(gg, rr))
 
 
+@pytest.mark.parametrize("h,w", [(128, 128), (136, 120)])
+def test_gradients_of_a_large_batch(dnz, h, w):
+    """8 copies of one image have its gradients: the loss is a mean, and an eighth scales every bf16
+    gradient exactly, so only the order of the fp32 sums over 8 x more pixels differs (2^-24 times the
+    square root of 140,000 terms). The large batch takes the data-gradient kernel's 16-block tiles, the
+    single image its 4-block ones."""
+    case(f"denoiser gradients, 8 copies of {h}x{w}")
+    feats = random_features(1, h, w, seed=h + w)
+    target = np.random.default_rng(8).random((1, h, w, 3)).astype(np.float32)
+    dnz.set_params(dnz.p0)
+    l1, g1 = dnz.train_step(feats, target, 2.0, lr=0.0, apply=False, want_grads=True)
+    l8, g8 = dnz.train_step(np.repeat(feats, 8, 0), np.repeat(target, 8, 0), 2.0, lr=0.0, apply=False, want_grads=True)
+    assert abs(l8 - l1) <= 3e-5 * l1
+    assert rel(g8, g1) < 3e-5, rel(g8, g1)
+
+
 def test_frame_path_equals_feature_path(gpu_renderer):
     """mmhrt_denoise on a rendered frame (its features packed into the network input on the device
     in one pass, colours composed into the framebuffer) gives the same colours, bit for bit, as
