@@ -225,6 +225,13 @@ MMHRT_API int32_t mmhrt_get_device_framebuffer(mmhrt_ctx ctx, mmhrt_device_frame
 MMHRT_API int32_t mmhrt_render_noalloc(mmhrt_ctx ctx, const mmhrt_camera* cam, const mmhrt_render_params* params,
                                        const mmhrt_device_framebuffer* out);
 
+/* Page-locked host memory for the calls' host outputs, from a pool of the process (freed blocks are
+ * kept, up to 256 MB, until the last context is destroyed). A copy into it runs at the link's rate
+ * and needs no staging and no page faults. At most 1 GB is handed out at a time (then MMHRT_E_OOM: use
+ * ordinary memory). Thread-safe; a block may outlive every context. */
+MMHRT_API int32_t mmhrt_host_alloc(uint64_t bytes, void** out);
+MMHRT_API int32_t mmhrt_host_free(void* p);
+
 /* Wait for all queued work on the context's stream. */
 MMHRT_API int32_t mmhrt_sync(mmhrt_ctx ctx);
 

@@ -3,8 +3,11 @@
 #include <string.h>
 
 #include <algorithm>
+#include <map>
+#include <mutex>
 #include <new>
 #include <string>
+#include <unordered_map>
 #include <vector>
 
 #include "../../include/mmhrt.h"
@@ -106,11 +109,93 @@ int check_ctx(mmhrt_ctx c) {
     if (e != hipSuccess) return hip_fail(c, e, "hipSetDevice");
     return MMHRT_OK;
 }
+
+namespace {
+// Page-locked host blocks (mmhrt_host_alloc), in sizes of 4 steps per power of two so that frames of
+// about the same size share them. The pool is never torn down with the process: the runtime may be
+// gone by then.
+struct HostPool {
+    static constexpr uint64_t KEEP = 256ull << 20, OUT = 1ull << 30;
+    std::mutex mu;
+    std::multimap<uint64_t, void*> idle;
+    std::unordered_map<void*, uint64_t> out;
+    uint64_t idle_bytes = 0, out_bytes = 0;
+    int contexts = 0;
+};
+HostPool& host_pool() {
+    static HostPool* p = new HostPool();
+    return *p;
+}
+uint64_t host_block_size(uint64_t n) {
+    uint64_t step = 1u << 14;
+    while (step * 8 < n) step *= 2;
+    return (n + step - 1) / step * step;
+}
+void host_pool_contexts(int d) {
+    HostPool& h = host_pool();
+    std::lock_guard<std::mutex> lk(h.mu);
+    h.contexts += d;
+    if (h.contexts > 0) return;
+    for (auto& b : h.idle) (void)hipHostFree(b.second);
+    h.idle.clear();
+    h.idle_bytes = 0;
+}
+}  // namespace
 }  // namespace mmhrt
 
 using namespace mmhrt;
 
 extern "C" {
+
+int32_t mmhrt_host_alloc(uint64_t bytes, void** out) {
+    if (!out || bytes == 0) return MMHRT_E_INVALID;
+    *out = nullptr;
+    if (bytes > HostPool::OUT) return MMHRT_E_OOM;
+    const uint64_t n = host_block_size(bytes);
+    HostPool& h = host_pool();
+    std::lock_guard<std::mutex> lk(h.mu);
+    if (h.contexts == 0 || h.out_bytes + n > HostPool::OUT) return MMHRT_E_OOM;
+    void* p = nullptr;
+    auto it = h.idle.find(n);
+    if (it != h.idle.end()) {
+        p = it->second;
+        h.idle.erase(it);
+        h.idle_bytes -= n;
+    } else if (hipHostMalloc(&p, n, hipHostMallocPortable) != hipSuccess) {
+        (void)hipGetLastError();
+        return MMHRT_E_OOM;
+    }
+    try {
+        h.out.emplace(p, n);
+    } catch (const std::bad_alloc&) {
+        (void)hipHostFree(p);
+        return MMHRT_E_OOM;
+    }
+    h.out_bytes += n;
+    *out = p;
+    return MMHRT_OK;
+}
+
+int32_t mmhrt_host_free(void* p) {
+    HostPool& h = host_pool();
+    std::lock_guard<std::mutex> lk(h.mu);
+    auto it = h.out.find(p);
+    if (it == h.out.end()) return MMHRT_E_INVALID;
+    const uint64_t n = it->second;
+    h.out.erase(it);
+    h.out_bytes -= n;
+    bool keep = h.contexts > 0 && h.idle_bytes + n <= HostPool::KEEP;
+    if (keep) {
+        try {
+            h.idle.emplace(n, p);
+            h.idle_bytes += n;
+        } catch (const std::bad_alloc&) {
+            keep = false;
+        }
+    }
+    if (!keep) (void)hipHostFree(p);
+    return MMHRT_OK;
+}
 
 int32_t mmhrt_create(int32_t device, mmhrt_ctx* out) {
     g_create_error.clear();
@@ -143,6 +228,8 @@ int32_t mmhrt_create(int32_t device, mmhrt_ctx* out) {
     }
     hipDeviceGetAttribute(&c->cu_count, hipDeviceAttributeMultiprocessorCount, device);
     if (c->cu_count <= 0) c->cu_count = 1;
+    size_t mem_free = 0;
+    if (hipMemGetInfo(&mem_free, &c->mem_total) != hipSuccess) (void)hipGetLastError();
     for (int i = 0; i < 12; ++i) hipEventCreate(&c->tm.ev[i]);
     c->tm.init = true;
     // the device address of this device's scratch array for mmhrt_render_noalloc; on failure that
@@ -156,6 +243,7 @@ int32_t mmhrt_create(int32_t device, mmhrt_ctx* out) {
         (void)hipGetLastError();
         c->rounds_host = nullptr;
     }
+    host_pool_contexts(1);
     *out = c;
     return MMHRT_OK;
 }
@@ -175,11 +263,7 @@ int32_t mmhrt_destroy(mmhrt_ctx c) {
     release(c->ts_sph); release(c->ts_col); release(c->bt_col); release(c->bt_depth); release(c->bt_t);
     release(c->bt_id); release(c->bt_rgba8); release(c->batch_ctr); release(c->batch_prefix);
     release(c->batch_jobs);
-    for (auto& sl : c->ts_slots) {
-        release(sl.nodes); release(sl.leaf); release(sl.id); release(sl.info); release(sl.dim); release(sl.box);
-        release(sl.rmax);
-    }
-    c->ts_slots.clear();
+    release_series(c);
     if (c->rounds_host) (void)hipHostFree(c->rounds_host);
     c->rounds_host = nullptr;
     if (c->dn) {
@@ -191,6 +275,7 @@ int32_t mmhrt_destroy(mmhrt_ctx c) {
         for (int i = 0; i < 12; ++i) hipEventDestroy(c->tm.ev[i]);
     hipStreamDestroy(c->stream);
     delete c;
+    host_pool_contexts(-1);
     return MMHRT_OK;
 }
 

@@ -73,6 +73,7 @@ struct mmhrt_ctx_s {
     std::string err;
     std::string noalloc_err;  // why mmhrt_render_noalloc cannot run on this device ("" = it can)
     int cu_count = 0;
+    size_t mem_total = 0;  // bytes of device memory
 
     // scene (original particle order)
     uint64_t n = 0;
@@ -177,7 +178,8 @@ struct mmhrt_ctx_s {
     mmhrt::DevBuf<int32_t> bt_id;
     mmhrt::DevBuf<uint32_t> bt_rgba8, batch_ctr, batch_prefix;
     mmhrt::DevBuf<uint8_t> batch_jobs;
-    std::vector<mmhrt::SeriesSlot> ts_slots;  // per timestep but the last (one-launch series)
+    std::vector<mmhrt::SeriesSlot> ts_slots;  // per timestep but the last (one-launch series), kept between calls
+    bool ts_busy = false;                     // a series is being built and traced
 
     // learned denoiser (created on first use)
     mmhrt::dn::Denoiser* dn = nullptr;
@@ -196,6 +198,10 @@ namespace mmhrt {
 int fail(mmhrt_ctx_s* c, int code, const std::string& msg);
 int hip_fail(mmhrt_ctx_s* c, hipError_t e, const char* what);
 
+// batch.hip: the structures that a series keeps between calls are given back; false if there were none
+// to give (or they are in use)
+bool release_series(mmhrt_ctx_s* c);
+
 template <typename T>
 int ensure(mmhrt_ctx_s* c, DevBuf<T>& b, size_t n, const char* what) {
     if (b.cap >= n && b.p) return 0;
@@ -209,6 +215,10 @@ int ensure(mmhrt_ctx_s* c, DevBuf<T>& b, size_t n, const char* what) {
     }
     size_t bytes = (n ? n : 1) * sizeof(T);
     hipError_t e = hipMalloc((void**)&b.p, bytes);
+    if (e != hipSuccess && release_series(c)) {  // the kept structures make room for what is needed now
+        (void)hipGetLastError();
+        e = hipMalloc((void**)&b.p, bytes);
+    }
     if (e != hipSuccess) {
         (void)hipGetLastError();
         b.p = nullptr;
@@ -246,15 +256,16 @@ void launch_fill_u32(hipStream_t s, uint32_t* p, uint32_t v, uint64_t n);
 void launch_fill_f4(hipStream_t s, float4* p, float4 v, uint64_t n);
 
 // lbvh.hip
-int build_lbvh(mmhrt_ctx_s* c, int bits);
+// reserve_only: allocate every buffer of the build (and set what a series needs of it), launch nothing of it
+int build_lbvh(mmhrt_ctx_s* c, int bits, bool reserve_only = false);
 int refit_lbvh(mmhrt_ctx_s* c);
 int reduce_scene(mmhrt_ctx_s* c);
 int count_leaf_pairs(mmhrt_ctx_s* c, int64_t* out);
 
-int sort_spheres(mmhrt_ctx_s* c, int bits);
+int sort_spheres(mmhrt_ctx_s* c, int bits, bool reserve_only = false);
 
 // pkd.hip
-int build_pkd(mmhrt_ctx_s* c, int bits);
+int build_pkd(mmhrt_ctx_s* c, int bits, bool reserve_only = false);
 
 // trace.hip
 // Spilled traversal stack words per lane: with at least 4 entries in LDS, room for an LBVH's height

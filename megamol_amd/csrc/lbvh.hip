@@ -49,6 +49,7 @@ __device__ __forceinline__ void lds_barrier() {
 
 // ---------------------------------------------------------------- scene reduction
 constexpr int NRED = 13;
+constexpr int REDUCE_BLOCKS = 1024;
 
 __global__ __launch_bounds__(256) void k_reduce_partial(const float4* __restrict__ sph, uint64_t n,
                                                         float* __restrict__ partial) {
@@ -1609,7 +1610,8 @@ __global__ void k_build_init(uint32_t* cnt, uint32_t gen, uint32_t* pair_h, uint
 // pass writes them there). The Morton pass also produces the first digit's tile histograms, and
 // the first pass takes the particle indices as its values.
 template <typename K, int RI, int DB>
-int morton_sort_t(mmhrt_ctx_s* c, K* ka, K* kb, uint32_t* va, uint32_t* vb, uint32_t* vfinal, uint64_t n) {
+int morton_sort_t(mmhrt_ctx_s* c, K* ka, K* kb, uint32_t* va, uint32_t* vb, uint32_t* vfinal, uint64_t n,
+                  bool reserve_only) {
     constexpr int RT = RB * RI, ND = 1 << DB;
     const int passes = ((sizeof(K) == 8 ? 63 : 30) + DB - 1) / DB;
     uint32_t tiles = (uint32_t)((n + RT - 1) / RT);
@@ -1620,6 +1622,11 @@ int morton_sort_t(mmhrt_ctx_s* c, K* ka, K* kb, uint32_t* va, uint32_t* vb, uint
     if (int e = ensure(c, c->scan_tmp, std::max((size_t)(groups + 1) * ND, (size_t)passes * 512 + 16),
                        "radix column sums"))
         return e;
+    if (os && !c->sort_fault.p) {
+        if (int e = ensure(c, c->sort_fault, 1, "radix fault flag")) return e;
+        launch_fill_u32(c->stream, c->sort_fault.p, 0u, 1);
+    }
+    if (reserve_only) return 0;
     uint32_t* hist = c->hist.p;
     uint32_t* offs = c->hist.p + hlen;
     // an odd number of passes starts from kb, so that the sorted keys end in ka
@@ -1634,10 +1641,6 @@ int morton_sort_t(mmhrt_ctx_s* c, K* ka, K* kb, uint32_t* va, uint32_t* vb, uint
     if (os) {
         // single-pass passes: status words per pass and tile, digit counts of all passes,
         // tickets and the fault flag
-        if (!c->sort_fault.p) {
-            if (int e = ensure(c, c->sort_fault, 1, "radix fault flag")) return e;
-            launch_fill_u32(c->stream, c->sort_fault.p, 0u, 1);
-        }
         uint32_t* ghist = c->scan_tmp.p;
         uint32_t* dstart = ghist + passes * 256;
         uint32_t* tickets = dstart + passes * 256;
@@ -1689,17 +1692,19 @@ int morton_sort_t(mmhrt_ctx_s* c, K* ka, K* kb, uint32_t* va, uint32_t* vb, uint
 // passes took 1.20 ms against 0.97 ms for four 8-bit passes: a 10-bit scatter pass costs 265 us
 // against 183 us (four keys per digit run, against sixteen, write shorter runs).
 template <typename K, int RI>
-int morton_sort_d(mmhrt_ctx_s* c, K* ka, K* kb, uint32_t* va, uint32_t* vb, uint32_t* vfinal, uint64_t n) {
+int morton_sort_d(mmhrt_ctx_s* c, K* ka, K* kb, uint32_t* va, uint32_t* vb, uint32_t* vfinal, uint64_t n,
+                  bool reserve_only) {
     if (c->opt_sort_digit != 0 || c->opt_sort_onesweep != 0)
-        return morton_sort_t<K, RI, 8>(c, ka, kb, va, vb, vfinal, n);
-    return morton_sort_t<K, RI, sizeof(K) == 8 ? 11 : 10>(c, ka, kb, va, vb, vfinal, n);
+        return morton_sort_t<K, RI, 8>(c, ka, kb, va, vb, vfinal, n, reserve_only);
+    return morton_sort_t<K, RI, sizeof(K) == 8 ? 11 : 10>(c, ka, kb, va, vb, vfinal, n, reserve_only);
 }
 
 template <typename K>
-int morton_sort(mmhrt_ctx_s* c, K* ka, K* kb, uint32_t* va, uint32_t* vb, uint32_t* vfinal, uint64_t n) {
-    if (c->opt_sort_ri == 8) return morton_sort_d<K, 8>(c, ka, kb, va, vb, vfinal, n);
-    if (c->opt_sort_ri == 32 && sizeof(K) == 4) return morton_sort_d<K, 32>(c, ka, kb, va, vb, vfinal, n);
-    return morton_sort_d<K, 16>(c, ka, kb, va, vb, vfinal, n);
+int morton_sort(mmhrt_ctx_s* c, K* ka, K* kb, uint32_t* va, uint32_t* vb, uint32_t* vfinal, uint64_t n,
+                bool reserve_only) {
+    if (c->opt_sort_ri == 8) return morton_sort_d<K, 8>(c, ka, kb, va, vb, vfinal, n, reserve_only);
+    if (c->opt_sort_ri == 32 && sizeof(K) == 4) return morton_sort_d<K, 32>(c, ka, kb, va, vb, vfinal, n, reserve_only);
+    return morton_sort_d<K, 16>(c, ka, kb, va, vb, vfinal, n, reserve_only);
 }
 
 // Persistent grid of the chunk pass: as many workgroups as fit on the device at once.
@@ -1727,9 +1732,41 @@ void launch_chunk_ls(mmhrt_ctx_s* c, const K* keys, const uint32_t* ids, uint32_
 // the particle of leaf k (the sorted values after a build, leaf_id on a refit, which keeps the
 // tree of the same keys and takes the boxes of the current spheres).
 template <typename K>
-int hierarchy(mmhrt_ctx_s* c, const K* keys, const uint32_t* ids) {
+int hierarchy(mmhrt_ctx_s* c, const K* keys, const uint32_t* ids, bool reserve_only = false) {
     uint64_t n = c->n;
     hipStream_t s = c->stream;
+    const uint64_t m = n - 1;
+    // leaves per chunk workgroup: 1024 (two per CU), 512 or 256; level-synchronous rounds unless
+    // the option build_ls is 0
+    const int bc = c->opt_build_chunk == 256 ? 256 : (c->opt_build_chunk == 512 ? 512 : 1024);
+    const int64_t nchunks = ((int64_t)n + bc - 1) / bc;
+    const bool bounds_stored = c->opt_build_ls != 0 && c->opt_build_span > 0;
+    // spans of build_span chunks, one workgroup each, then the tail over their exports (at
+    // most three per span: its right boundary from the chunk pass, its two boundary splits).
+    // Without flags2 at most 256 spans: every span's workgroup then scans the chunk pass's
+    // whole list, so larger scenes take longer spans rather than more of them
+    const int64_t span_chunks =
+        bounds_stored ? c->opt_build_span : std::max<int64_t>(c->opt_build_span, (nchunks + 255) / 256);
+    const int64_t span = span_chunks * (int64_t)bc;
+    const uint64_t spans = c->opt_build_span > 0 ? (n + span - 1) / span : 0;
+    const size_t xcap = 4 * spans + 64;
+    if (n > 1) {
+        if (int e = ensure(c, c->box_cnt, BOX_SLOTS, "box round counters")) return e;
+        if (int e = ensure(c, c->meet, m, "meeting records")) return e;
+        if (int e = ensure(c, c->meet_far, m, "meeting ranges")) return e;
+        const bool fresh = !c->flags.p || c->flags.cap < m;
+        if (int e = ensure(c, c->flags, m, "meeting counters")) return e;
+        if (fresh) launch_fill_u32(s, c->flags.p, 0xffffffffu, c->flags.cap);  // no generation yet
+        if (bounds_stored) {
+            const uint64_t m2 = 2 * (uint64_t)(nchunks + 1);
+            const bool fresh2 = !c->flags2.p || c->flags2.cap < m2;
+            if (int e = ensure(c, c->flags2, m2, "chunk boundary arrivals")) return e;
+            if (fresh2) launch_fill_u32(s, c->flags2.p, 0xffffffffu, c->flags2.cap);
+        }
+        if (c->opt_build_span > 0)
+            if (int e = ensure(c, c->xlist, 2 * xcap, "span export lists")) return e;
+    }
+    if (reserve_only) return 0;
     if (n == 1 || c->opt_build_ls == 0)
         hipLaunchKernelGGL(k_regather, dim3(blocks_for(n, 256)), dim3(256), 0, s, cur_spheres(c), ids, c->leaf_sph.p,
                            n);
@@ -1739,13 +1776,6 @@ int hierarchy(mmhrt_ctx_s* c, const K* keys, const uint32_t* ids) {
         rec(c, 9);
         return 0;
     }
-    uint64_t m = n - 1;
-    if (int e = ensure(c, c->box_cnt, BOX_SLOTS, "box round counters")) return e;
-    if (int e = ensure(c, c->meet, m, "meeting records")) return e;
-    if (int e = ensure(c, c->meet_far, m, "meeting ranges")) return e;
-    const bool fresh = !c->flags.p || c->flags.cap < m;
-    if (int e = ensure(c, c->flags, m, "meeting counters")) return e;
-    if (fresh) launch_fill_u32(s, c->flags.p, 0xffffffffu, c->flags.cap);  // no generation yet
     // each pass takes a new generation; builds captured into a graph keep theirs, so such a
     // graph is launched once (the batched time series), never replayed
     if (++c->build_gen == 0xffffffffu) c->build_gen = 1;
@@ -1756,20 +1786,9 @@ int hierarchy(mmhrt_ctx_s* c, const K* keys, const uint32_t* ids) {
     // the spare value buffer
     uint32_t* l0 = sizeof(K) == 8 ? reinterpret_cast<uint32_t*>(c->klb.p) : reinterpret_cast<uint32_t*>(c->kb.p);
     uint32_t* l1 = c->vb.p;
-    // leaves per chunk workgroup: 1024 (two per CU), 512 or 256; level-synchronous rounds unless
-    // the option build_ls is 0
-    const int bc = c->opt_build_chunk == 256 ? 256 : (c->opt_build_chunk == 512 ? 512 : 1024);
-    const int64_t nchunks = ((int64_t)n + bc - 1) / bc;
     // per-side arrival records at the chunk boundaries: the level-synchronous chunk pass followed
     // by span passes stores its boundary arrivals there instead of exchanging them
-    uint32_t* flags2 = nullptr;
-    if (c->opt_build_ls != 0 && c->opt_build_span > 0) {
-        const uint64_t m2 = 2 * (uint64_t)(nchunks + 1);
-        const bool fresh2 = !c->flags2.p || c->flags2.cap < m2;
-        if (int e = ensure(c, c->flags2, m2, "chunk boundary arrivals")) return e;
-        if (fresh2) launch_fill_u32(s, c->flags2.p, 0xffffffffu, c->flags2.cap);
-        flags2 = c->flags2.p;
-    }
+    uint32_t* flags2 = bounds_stored ? c->flags2.p : nullptr;
     rec(c, 8);
     if (c->opt_build_ls != 0) {
         if (bc == 256)
@@ -1792,16 +1811,6 @@ int hierarchy(mmhrt_ctx_s* c, const K* keys, const uint32_t* ids) {
     // that round had (the counts come back through pinned host memory one build late; they are
     // hints only: the rounds loop over any list size and the tail finishes whatever is left)
     if (c->opt_build_span > 0) {
-        // spans of build_span chunks, one workgroup each, then the tail over their exports (at
-        // most three per span: its right boundary from the chunk pass, its two boundary splits).
-        // Without flags2 at most 256 spans: every span's workgroup then scans the chunk pass's
-        // whole list, so larger scenes take longer spans rather than more of them
-        const int64_t span_chunks =
-            flags2 ? c->opt_build_span : std::max<int64_t>(c->opt_build_span, (nchunks + 255) / 256);
-        const int64_t span = span_chunks * (int64_t)bc;
-        const uint64_t spans = (n + span - 1) / span;
-        const size_t xcap = 4 * spans + 64;
-        if (int e = ensure(c, c->xlist, 2 * xcap, "span export lists")) return e;
         hipLaunchKernelGGL(k_bu_span<K>, dim3((unsigned)spans), dim3(1024), 0, s, keys, (int64_t)n, c->nodes.p,
                            c->meet.p, c->meet_far.p, c->flags.p, flags2, (int64_t)bc, l0, c->va.p, c->vb.p,
                            c->xlist.p, c->box_cnt.p, span, c->info.p);
@@ -1834,10 +1843,11 @@ int hierarchy(mmhrt_ctx_s* c, const K* keys, const uint32_t* ids) {
 }
 
 template <typename K>
-int build_typed(mmhrt_ctx_s* c, K* ka, K* kb) {
+int build_typed(mmhrt_ctx_s* c, K* ka, K* kb, bool reserve_only) {
     uint64_t n = c->n;
     hipStream_t s = c->stream;
-    if (int e = morton_sort<K>(c, ka, kb, c->va.p, c->vb.p, c->leaf_id.p, n)) return e;
+    if (int e = morton_sort<K>(c, ka, kb, c->va.p, c->vb.p, c->leaf_id.p, n, reserve_only)) return e;
+    if (reserve_only) return hierarchy<K>(c, ka, c->leaf_id.p, true);
     rec(c, 3);
     rec(c, 4);  // the leaf gather runs inside the hierarchy pass
     // the sort's last pass wrote its values (the leaf -> particle map) straight into leaf_id
@@ -1872,10 +1882,13 @@ void launch_fill_u32(hipStream_t s, uint32_t* p, uint32_t v, uint64_t n) {
     hipLaunchKernelGGL(k_fill, dim3(g), dim3(256), 0, s, p, v, n);
 }
 
+static int reserve_reduction(mmhrt_ctx_s* c) {
+    if (int e = ensure(c, c->partial, (size_t)REDUCE_BLOCKS * NRED, "reduction partials")) return e;
+    return ensure(c, c->info, 1, "scene info");
+}
 int reduce_scene(mmhrt_ctx_s* c) {
-    const int nb = 1024;
-    if (int e = ensure(c, c->partial, (size_t)nb * NRED, "reduction partials")) return e;
-    if (int e = ensure(c, c->info, 1, "scene info")) return e;
+    const int nb = REDUCE_BLOCKS;
+    if (int e = reserve_reduction(c)) return e;
     hipLaunchKernelGGL(k_reduce_partial, dim3(nb), dim3(256), 0, c->stream, cur_spheres(c), c->n, c->partial.p);
     hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(256), 0, c->stream, c->partial.p, nb, c->info.p, c->bits);
     return 0;
@@ -1883,7 +1896,7 @@ int reduce_scene(mmhrt_ctx_s* c) {
 
 // The first half of a build, shared by the treelet P-k-d build: scene bounds, Morton codes and
 // the stable radix sort; leaf_id receives the particle of each sorted position, ka / kla the keys.
-int sort_spheres(mmhrt_ctx_s* c, int bits) {
+int sort_spheres(mmhrt_ctx_s* c, int bits, bool reserve_only) {
     uint64_t n = c->n;
     if (n == 0) return fail(c, MMHRT_E_STATE, "build: no spheres set");
     if (n > 0x7fffffffull) return fail(c, MMHRT_E_UNSUPPORTED, "build: more than 2^31-1 spheres");
@@ -1899,13 +1912,13 @@ int sort_spheres(mmhrt_ctx_s* c, int bits) {
         if ((e = ensure(c, c->ka, n, "keys"))) return e;
         if ((e = ensure(c, c->kb, n, "keys"))) return e;
     }
-    rec(c, 0);
-    if ((e = reduce_scene(c))) return e;
-    if (bits == 63) return morton_sort<uint64_t>(c, c->kla.p, c->klb.p, c->va.p, c->vb.p, c->leaf_id.p, n);
-    return morton_sort<uint32_t>(c, c->ka.p, c->kb.p, c->va.p, c->vb.p, c->leaf_id.p, n);
+    if (!reserve_only) rec(c, 0);
+    if ((e = reserve_only ? reserve_reduction(c) : reduce_scene(c))) return e;
+    if (bits == 63) return morton_sort<uint64_t>(c, c->kla.p, c->klb.p, c->va.p, c->vb.p, c->leaf_id.p, n, reserve_only);
+    return morton_sort<uint32_t>(c, c->ka.p, c->kb.p, c->va.p, c->vb.p, c->leaf_id.p, n, reserve_only);
 }
 
-int build_lbvh(mmhrt_ctx_s* c, int bits) {
+int build_lbvh(mmhrt_ctx_s* c, int bits, bool reserve_only) {
     uint64_t n = c->n;
     if (n == 0) return fail(c, MMHRT_E_STATE, "build: no spheres set");
     if (n > 0x7fffffffull) return fail(c, MMHRT_E_UNSUPPORTED, "build: more than 2^31-1 spheres");
@@ -1924,13 +1937,17 @@ int build_lbvh(mmhrt_ctx_s* c, int bits) {
         if ((e = ensure(c, c->ka, n, "keys"))) return e;
         if ((e = ensure(c, c->kb, n, "keys"))) return e;
     }
-    rec(c, 0);
-    if ((e = reduce_scene(c))) return e;
+    if (!reserve_only) rec(c, 0);
+    if ((e = reserve_only ? reserve_reduction(c) : reduce_scene(c))) return e;
     if (bits == 63)
-        e = build_typed<uint64_t>(c, c->kla.p, c->klb.p);
+        e = build_typed<uint64_t>(c, c->kla.p, c->klb.p, reserve_only);
     else
-        e = build_typed<uint32_t>(c, c->ka.p, c->kb.p);
+        e = build_typed<uint32_t>(c, c->ka.p, c->kb.p, reserve_only);
     if (e) return e;
+    if (reserve_only) {
+        c->accel = 0;
+        return 0;
+    }
     rec(c, 5);
     hipError_t he = hipGetLastError();
     if (he != hipSuccess) return hip_fail(c, he, "LBVH build launch");

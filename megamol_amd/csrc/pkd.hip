@@ -278,11 +278,11 @@ __global__ __launch_bounds__(256) void k_pkd_top_level(Node* __restrict__ nodes,
 
 }  // namespace
 
-int build_pkd(mmhrt_ctx_s* c, int bits) {
+int build_pkd(mmhrt_ctx_s* c, int bits, bool reserve_only) {
     const int64_t M = c->opt_treelet;
     if (M != 256 && M != 512 && M != 1024)
         return fail(c, MMHRT_E_INVALID, "build: option treelet must be 256, 512 or 1024");
-    if (int e = sort_spheres(c, bits)) return e;
+    if (int e = sort_spheres(c, bits, reserve_only)) return e;
     const uint64_t n = c->n;
     const uint32_t T = (uint32_t)((n + M - 1) / M);
     uint32_t L = 2;
@@ -293,6 +293,13 @@ int build_pkd(mmhrt_ctx_s* c, int bits) {
     if ((e = ensure(c, c->tl_box, (size_t)T * 6, "treelet boxes"))) return e;
     if ((e = ensure(c, c->tl_rmax, T, "treelet radii"))) return e;
     if ((e = ensure(c, c->nodes, L - 1, "top nodes"))) return e;
+    if (reserve_only) {
+        c->pkd_M = (uint32_t)M;
+        c->pkd_T = T;
+        c->pkd_L = L;
+        c->accel = 1;
+        return 0;
+    }
     rec(c, 3);
     rec(c, 4);
     const float4* sph = cur_spheres(c);

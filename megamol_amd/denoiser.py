@@ -145,7 +145,7 @@ class Denoiser:
         if feats.ndim == 3:
             feats = feats[None]
         b, h, w, _ = feats.shape
-        out = np.empty((b, h, w, 3), np.float32)
+        out = L.host_empty((b, h, w, 3), np.float32)
         bgv = (C.c_float * 4)(*bg)
         self._ck(self.lib.mmhrt_denoise_features(self.r.ctx, feats.ctypes.data, b, h, w, depth_scale, bgv,
                                                  out.ctypes.data))
@@ -157,7 +157,7 @@ class Denoiser:
         target = np.ascontiguousarray(target, np.float32)
         b, h, w, _ = feats.shape
         loss = C.c_float()
-        g = np.empty(self.n, np.float32) if want_grads else None
+        g = L.host_empty((self.n,), np.float32) if want_grads else None
         bgv = (C.c_float * 4)(*bg)
         self._ck(self.lib.mmhrt_denoiser_train_step(self.r.ctx, feats.ctypes.data, target.ctypes.data, b, h, w,
                                                     depth_scale, bgv, lr, 1 if apply else 0, C.byref(loss),

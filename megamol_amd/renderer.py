@@ -198,11 +198,11 @@ class SphereRenderer:
                 "t": (np.float32, (H, W)), "hit_id": (np.int32, (H, W))}
         for name in outputs:
             dt, shp = spec[name]
-            a = np.empty(shp, dt)
+            a = L.host_empty(shp, dt)
             setattr(fr, name, a)
             setattr(fb, name, a.ctypes.data)
         if aux:
-            fr.aux = np.empty((H, W, 8), np.float16)
+            fr.aux = L.host_empty((H, W, 8), np.float16)
             fb.aux = fr.aux.ctypes.data
 
     def sync(self) -> None:
@@ -234,8 +234,8 @@ class SphereRenderer:
             w, h = (p.window[2], p.window[3]) if p.window[2] > 0 else (p.width, p.height)
             sizes.append((w, h, off))
             off += w * h
-        rgba = np.empty(off, np.uint32)
-        depth = np.empty(off, np.float32)
+        rgba = L.host_empty((off,), np.uint32)
+        depth = L.host_empty((off,), np.float32)
         ms = C.c_float()
         self._ck(self.lib.mmhrt_render_batch(self.ctx, arr, len(jobs), refit_period, bits, 1 if use_graph else 0,
                                              rgba.ctypes.data, depth.ctypes.data, C.byref(ms)))
