@@ -7,6 +7,7 @@
 //   2. Morton codes, 30-bit (10 per axis) or 63-bit (21 per axis), over one uniform scale
 //   3. LSD radix sort of (key, particle index), 8-bit digits, stable: a tile's keys are ranked
 //      with wavefront ballots (8 ballots give each lane the mask of same-digit lanes)
+//      (up to 16384 spheres steps 1 to 3 are one workgroup's)
 //   4. hierarchy and boxes together, bottom-up, with the gather of the spheres into Morton order
 //      (leaf k) on the way: the second arrival at a parent merges and writes the whole node
 //      (Karras 2012 numbering and index tie-break for equal keys, Apetrei 2014 parent rule; LDS
@@ -102,8 +103,38 @@ __global__ __launch_bounds__(256) void k_reduce_partial(const float4* __restrict
     if (threadIdx.x < NRED) partial[(size_t)blockIdx.x * NRED + threadIdx.x] = red[threadIdx.x][0];
 }
 
+// What a hierarchy pass starts from: list counters cleared, the pass's generation number, the leaf-pair
+// height. Written by the kernel that finishes the scene reduction (cnt null: a reduction without a
+// build).
+struct PassInit {
+    uint32_t* cnt;
+    uint32_t gen, pair_h;
+    __device__ __forceinline__ void write(SceneInfo* info) const {
+        if (!cnt) return;
+        for (uint32_t i = threadIdx.x; i < (uint32_t)(BOX_ROUNDS + 3); i += blockDim.x) cnt[i] = 0u;
+        if (threadIdx.x == 0) {
+            cnt[BOX_ROUNDS + 3] = gen;  // GEN_SLOT
+            info->pair_h = pair_h;
+        }
+    }
+};
+
+__device__ __forceinline__ void write_info(SceneInfo* info, const float v[NRED], int bits) {
+    for (int a = 0; a < 3; ++a) {
+        info->clo[a] = v[a];
+        info->chi[a] = v[3 + a];
+        info->blo[a] = v[6 + a];
+        info->bhi[a] = v[9 + a];
+    }
+    info->absmax = v[12];
+    float ext = fmaxf(fmaxf(v[3] - v[0], v[4] - v[1]), v[5] - v[2]);
+    float cells = bits == 63 ? 2097152.0f : 1024.0f;
+    info->scale = ext > 0.0f ? cells / ext : 0.0f;
+}
+
 __global__ __launch_bounds__(256) void k_reduce_final(const float* __restrict__ partial, int nblocks,
-                                                      SceneInfo* info, int bits) {
+                                                      SceneInfo* info, int bits, PassInit init) {
+    init.write(info);
     __shared__ float red[NRED][256];
     float v[NRED];
     for (int k = 0; k < NRED; ++k) {
@@ -129,16 +160,7 @@ __global__ __launch_bounds__(256) void k_reduce_final(const float* __restrict__ 
     }
     if (threadIdx.x != 0) return;
     for (int k = 0; k < NRED; ++k) v[k] = red[k][0];
-    for (int a = 0; a < 3; ++a) {
-        info->clo[a] = v[a];
-        info->chi[a] = v[3 + a];
-        info->blo[a] = v[6 + a];
-        info->bhi[a] = v[9 + a];
-    }
-    info->absmax = v[12];
-    float ext = fmaxf(fmaxf(v[3] - v[0], v[4] - v[1]), v[5] - v[2]);
-    float cells = bits == 63 ? 2097152.0f : 1024.0f;
-    info->scale = ext > 0.0f ? cells / ext : 0.0f;
+    write_info(info, v, bits);
 }
 
 // ---------------------------------------------------------------- Morton codes
@@ -178,8 +200,8 @@ __device__ __forceinline__ void hist_add(uint32_t* h, uint32_t d) {
     if (!eq) atomicAdd(&h[d], 1u);
 }
 
-__device__ __forceinline__ uint32_t morton30(const float4 s, const SceneInfo* info, float sc) {
-    const float f[3] = {(s.x - info->clo[0]) * sc, (s.y - info->clo[1]) * sc, (s.z - info->clo[2]) * sc};
+__device__ __forceinline__ uint32_t morton30(const float4 s, const float* clo, float sc) {
+    const float f[3] = {(s.x - clo[0]) * sc, (s.y - clo[1]) * sc, (s.z - clo[2]) * sc};
     uint32_t q[3];
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
@@ -188,8 +210,8 @@ __device__ __forceinline__ uint32_t morton30(const float4 s, const SceneInfo* in
     }
     return (spread10(q[0]) << 2) | (spread10(q[1]) << 1) | spread10(q[2]);
 }
-__device__ __forceinline__ uint64_t morton63(const float4 s, const SceneInfo* info, float sc) {
-    const float f[3] = {(s.x - info->clo[0]) * sc, (s.y - info->clo[1]) * sc, (s.z - info->clo[2]) * sc};
+__device__ __forceinline__ uint64_t morton63(const float4 s, const float* clo, float sc) {
+    const float f[3] = {(s.x - clo[0]) * sc, (s.y - clo[1]) * sc, (s.z - clo[2]) * sc};
     uint32_t q[3];
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
@@ -231,9 +253,9 @@ __global__ __launch_bounds__(RB) void k_morton_tile(const float4* __restrict__ s
             const uint64_t i = base + (uint64_t)(r0 + j) * 64;
             K key;
             if constexpr (sizeof(K) == 8)
-                key = morton63(sb[j], info, sc);
+                key = morton63(sb[j], info->clo, sc);
             else
-                key = morton30(sb[j], info, sc);
+                key = morton30(sb[j], info->clo, sc);
             if (whole || i < n) {
                 keys[i] = key;
                 hist_add(h, (uint32_t)(key & (K)(ND - 1)));
@@ -566,6 +588,203 @@ __global__ __launch_bounds__(256) void k_col_offsets(const uint32_t* __restrict_
     for (int k = 0; k < CG; ++k) {
         if (t0 + k < tiles) offs[(size_t)(t0 + k) * nd + d] = run;
         run += v[k];
+    }
+}
+
+// The three column kernels in one launch, for 8-bit digits and at most COL_FEW tiles: every block reads
+// all tiles' counts itself (1 KB rows, four threads per digit), for the sums before its group and over
+// all, and then writes its group's offsets. Each of the three is a few microseconds of latency and a
+// launch; 62 tiles: 11.5 -> 4.6 us a pass and two launches less, 245 tiles: 12 -> 8.3 us. The rows read
+// grow with the square of the tiles, hence the limit.
+constexpr uint32_t COL_FEW = 512;
+__global__ __launch_bounds__(1024) void k_col_fused(const uint32_t* __restrict__ hist, uint32_t tiles,
+                                                    uint32_t* __restrict__ offs) {
+    __shared__ uint32_t p_before[4][256], p_all[4][256], p_own[4][256], wsum[4];
+    const uint32_t d = threadIdx.x & 255u, q = threadIdx.x >> 8;
+    const uint32_t t0 = blockIdx.x * CG;  // the group's first tile
+    constexpr uint32_t OWN = CG / 4;      // tiles whose offsets a thread writes: t0 + q OWN on
+    uint32_t own[OWN];
+#pragma unroll
+    for (uint32_t k = 0; k < OWN; ++k) {
+        const uint32_t t = t0 + q * OWN + k;
+        own[k] = hist[(size_t)(t < tiles ? t : tiles - 1) * 256 + d];
+    }
+    uint32_t before = 0, all = 0;
+    for (uint32_t t = q; t < tiles; t += 64) {  // 16 loads in flight, at clamped rows, masked where summed
+        uint32_t v[16];
+#pragma unroll
+        for (uint32_t k = 0; k < 16; ++k) v[k] = hist[(size_t)(t + 4 * k < tiles ? t + 4 * k : tiles - 1) * 256 + d];
+#pragma unroll
+        for (uint32_t k = 0; k < 16; ++k) {
+            const uint32_t w = t + 4 * k < tiles ? v[k] : 0u;
+            all += w;
+            before += t + 4 * k < t0 ? w : 0u;
+        }
+    }
+    uint32_t sum = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < OWN; ++k) sum += t0 + q * OWN + k < tiles ? own[k] : 0u;
+    p_before[q][d] = before;
+    p_all[q][d] = all;
+    p_own[q][d] = sum;
+    __syncthreads();
+    // keys with a smaller digit: exclusive scan of the totals (each wavefront holds 64 digits)
+    const uint32_t lane = __lane_id();
+    const uint32_t tot = p_all[0][d] + p_all[1][d] + p_all[2][d] + p_all[3][d];
+    uint32_t inc = tot;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t y = __shfl_up(inc, o, 64);
+        if (lane >= (uint32_t)o) inc += y;
+    }
+    if (lane == 63 && q == 0) wsum[d >> 6] = inc;
+    __syncthreads();
+    uint32_t run = inc - tot + p_before[0][d] + p_before[1][d] + p_before[2][d] + p_before[3][d];
+    for (uint32_t w = 0; w < (d >> 6); ++w) run += wsum[w];
+    for (uint32_t k = 0; k < q; ++k) run += p_own[k][d];
+#pragma unroll
+    for (uint32_t k = 0; k < OWN; ++k) {
+        const uint32_t t = t0 + q * OWN + k;
+        if (t < tiles) offs[(size_t)t * 256 + d] = run;
+        run += own[k];
+    }
+}
+
+// ---------------------------------------------------------------- small scenes in one workgroup
+// Scene bounds, Morton codes and the stable sort of up to 1024 R spheres in one 1024-thread workgroup:
+// the keys stay in registers and LDS through all passes, ranked as in k_radix_scatter. The same
+// values, keys and order as the kernels above, which take some 20 launches of 2 to 9 us each for it,
+// whatever the size: 10k spheres 0.11 ms -> 0.05 ms (a preview frame of them 353 -> 288 us).
+template <typename K, int R>
+__global__ __launch_bounds__(1024) void k_small_sort(const float4* __restrict__ sph, uint32_t n, SceneInfo* info,
+                                                     int bits, PassInit init, K* __restrict__ keys,
+                                                     uint32_t* __restrict__ ids) {
+    constexpr int W = 16;
+    __shared__ K s_key[1024 * R];
+    __shared__ uint16_t s_val[1024 * R];
+    __shared__ uint16_t wc[W][256];
+    __shared__ uint32_t wsum[4];
+    __shared__ float s_red[W][NRED];
+    const uint32_t lane = __lane_id(), wave = threadIdx.x >> 6;
+    const uint32_t base = wave * 64u * R + lane;  // the thread's keys: base + 64 r
+    init.write(info);
+    float4 sb[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const uint32_t i = base + 64u * r;
+        sb[r] = sph[i < n ? i : n - 1];
+    }
+    float v[NRED];
+    for (int i = 0; i < 3; ++i) {
+        v[i] = INFINITY;
+        v[3 + i] = -INFINITY;
+        v[6 + i] = INFINITY;
+        v[9 + i] = -INFINITY;
+    }
+    v[12] = 0.0f;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const float c[3] = {sb[r].x, sb[r].y, sb[r].z}, w = sb[r].w;
+        for (int a = 0; a < 3; ++a) {
+            v[a] = fminf(v[a], c[a]);
+            v[3 + a] = fmaxf(v[3 + a], c[a]);
+            v[6 + a] = fminf(v[6 + a], c[a] - w);
+            v[9 + a] = fmaxf(v[9 + a], c[a] + w);
+            v[12] = fmaxf(v[12], fabsf(c[a]) + fabsf(w));
+        }
+    }
+    for (int k = 0; k < NRED; ++k) {
+        const bool is_min = (k < 3) || (k >= 6 && k < 9);
+        for (int o = 32; o > 0; o >>= 1) {
+            const float x = __shfl_xor(v[k], o, 64);
+            v[k] = is_min ? fminf(v[k], x) : fmaxf(v[k], x);
+        }
+        if (lane == 0) s_red[wave][k] = v[k];
+    }
+    __syncthreads();
+    if (threadIdx.x < NRED) {
+        const int k = threadIdx.x;
+        const bool is_min = (k < 3) || (k >= 6 && k < 9);
+        float x = s_red[0][k];
+        for (int w = 1; w < W; ++w) x = is_min ? fminf(x, s_red[w][k]) : fmaxf(x, s_red[w][k]);
+        s_red[0][k] = x;  // (read by this thread alone until the barrier)
+    }
+    __syncthreads();
+    for (int k = 0; k < NRED; ++k) v[k] = s_red[0][k];
+    if (threadIdx.x == 0) write_info(info, v, bits);
+    const float ext = fmaxf(fmaxf(v[3] - v[0], v[4] - v[1]), v[5] - v[2]);
+    const float sc = ext > 0.0f ? (sizeof(K) == 8 ? 2097152.0f : 1024.0f) / ext : 0.0f;
+    K key[R];
+    uint32_t val[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        if constexpr (sizeof(K) == 8)
+            key[r] = morton63(sb[r], v, sc);
+        else
+            key[r] = morton30(sb[r], v, sc);
+        val[r] = base + 64u * r;
+    }
+    constexpr int passes = sizeof(K) == 8 ? 8 : 4;
+    for (int p = 0; p < passes; ++p) {
+        const int shift = 8 * p;
+        for (uint32_t d = lane; d < 256; d += 64) wc[wave][d] = 0;
+        uint32_t rank[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const bool valid = base + 64u * r < n;
+            const uint32_t d = (uint32_t)((key[r] >> shift) & (K)255);
+            const uint64_t peers = match_digit<8>(d, valid);
+            const uint32_t before = valid ? wc[wave][d] : 0u;
+            rank[r] = before + (uint32_t)__popcll(peers & lanemask_lt());
+            if (valid && (__ffsll((unsigned long long)peers) - 1) == (int)lane)
+                wc[wave][d] = (uint16_t)(before + (uint32_t)__popcll(peers));
+        }
+        __syncthreads();
+        uint32_t cnt = 0, inc = 0;
+        if (threadIdx.x < 256) {  // thread = digit: exclusive scan over digits, then down the wavefronts
+            for (int w = 0; w < W; ++w) cnt += wc[w][threadIdx.x];
+            inc = cnt;
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const uint32_t y = __shfl_up(inc, o, 64);
+                if (lane >= (uint32_t)o) inc += y;
+            }
+            if (lane == 63) wsum[wave] = inc;
+        }
+        __syncthreads();
+        if (threadIdx.x < 256) {
+            uint32_t run = inc - cnt;
+            for (uint32_t w = 0; w < wave; ++w) run += wsum[w];
+            for (int w = 0; w < W; ++w) {
+                const uint32_t k = wc[w][threadIdx.x];
+                wc[w][threadIdx.x] = (uint16_t)run;
+                run += k;
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            if (base + 64u * r < n) {
+                const uint32_t pos = wc[wave][(uint32_t)((key[r] >> shift) & (K)255)] + rank[r];
+                s_key[pos] = key[r];
+                s_val[pos] = (uint16_t)val[r];
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const uint32_t i = base + 64u * r;
+            key[r] = s_key[i];  // (past n: whatever lies there, not used)
+            val[r] = s_val[i];
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const uint32_t i = base + 64u * r;
+        if (i < n) {
+            keys[i] = key[r];
+            ids[i] = val[r];
+        }
     }
 }
 
@@ -1594,17 +1813,6 @@ __global__ void k_fill(uint32_t* p, uint32_t v, uint64_t n) {
 
 inline unsigned blocks_for(uint64_t n, unsigned b) { return (unsigned)((n + b - 1) / b); }
 
-// Per hierarchy pass: list counters cleared, the pass's generation number, the leaf-pair height
-// (one launch instead of three fills).
-__global__ void k_build_init(uint32_t* cnt, uint32_t gen, uint32_t* pair_h, uint32_t pv) {
-    const uint32_t i = threadIdx.x;
-    if (i < (uint32_t)(BOX_ROUNDS + 3)) cnt[i] = 0u;
-    if (i == 0) {
-        cnt[GEN_SLOT] = gen;
-        *pair_h = pv;
-    }
-}
-
 // Morton codes of the current spheres into ka, then the LSD radix sort of (key, particle index)
 // over `passes` 8-bit digits; the sorted keys end in ka, the sorted values in vfinal (the last
 // pass writes them there). The Morton pass also produces the first digit's tile histograms, and
@@ -1664,9 +1872,14 @@ int morton_sort_t(mmhrt_ctx_s* c, K* ka, K* kb, uint32_t* va, uint32_t* vb, uint
         int shift = DB * p;
         if (p > 0)
             hipLaunchKernelGGL((k_radix_hist<K, RI, DB>), dim3(tiles), dim3(RB), 0, c->stream, src, n, shift, hist);
-        hipLaunchKernelGGL(k_col_sums, dim3(groups, ND / 256), dim3(256), 0, c->stream, hist, tiles, c->scan_tmp.p,
-                           (uint32_t)ND);
-        if (ND == 256) {
+        if (ND == 256 && tiles <= COL_FEW) {
+            hipLaunchKernelGGL(k_col_fused, dim3(groups), dim3(1024), 0, c->stream, hist, tiles, offs);
+        } else {
+            hipLaunchKernelGGL(k_col_sums, dim3(groups, ND / 256), dim3(256), 0, c->stream, hist, tiles,
+                               c->scan_tmp.p, (uint32_t)ND);
+        }
+        if (ND == 256 && tiles <= COL_FEW) {
+        } else if (ND == 256) {
             hipLaunchKernelGGL(k_col_scan, dim3(4), dim3(1024), 0, c->stream, c->scan_tmp.p, groups);
             hipLaunchKernelGGL(k_col_offsets<true>, dim3(groups), dim3(256), 0, c->stream, hist, tiles, groups,
                                c->scan_tmp.p, offs, (uint32_t)ND);
@@ -1702,7 +1915,9 @@ int morton_sort_d(mmhrt_ctx_s* c, K* ka, K* kb, uint32_t* va, uint32_t* vb, uint
 template <typename K>
 int morton_sort(mmhrt_ctx_s* c, K* ka, K* kb, uint32_t* va, uint32_t* vb, uint32_t* vfinal, uint64_t n,
                 bool reserve_only) {
-    if (c->opt_sort_ri == 8) return morton_sort_d<K, 8>(c, ka, kb, va, vb, vfinal, n, reserve_only);
+    // tiles of 16 keys per thread (the default) halve where they would leave CUs idle: 250k spheres (62
+    // tiles of 16) build in 170 us with them, in 157 us with tiles of 8; 1M in 255 and 258 us
+    if (c->opt_sort_ri == 8 || (c->opt_sort_ri == 16 && n <= (1u << 19))) return morton_sort_d<K, 8>(c, ka, kb, va, vb, vfinal, n, reserve_only);
     if (c->opt_sort_ri == 32 && sizeof(K) == 4) return morton_sort_d<K, 32>(c, ka, kb, va, vb, vfinal, n, reserve_only);
     return morton_sort_d<K, 16>(c, ka, kb, va, vb, vfinal, n, reserve_only);
 }
@@ -1745,13 +1960,17 @@ int hierarchy(mmhrt_ctx_s* c, const K* keys, const uint32_t* ids, bool reserve_o
     // most three per span: its right boundary from the chunk pass, its two boundary splits).
     // Without flags2 at most 256 spans: every span's workgroup then scans the chunk pass's
     // whole list, so larger scenes take longer spans rather than more of them
-    const int64_t span_chunks =
-        bounds_stored ? c->opt_build_span : std::max<int64_t>(c->opt_build_span, (nchunks + 255) / 256);
+    // Where those make few spans they take 64 chunks at most, which trades levels of a span's workgroup
+    // for levels of the top's and runs more spans side by side: 1M spheres (977 chunks) build in 254 us
+    // with spans of 256, 242, 235, 234, 233, 243 us with 128, 64, 32, 16, 8; 4M refit in 310 us, then 300,
+    // 295, 299, 322, 387; 50M (48.8k chunks) in 1.60 ms of boxes with 128 against 1.53 with 256
+    const int64_t span_chunks = !bounds_stored ? std::max<int64_t>(c->opt_build_span, (nchunks + 255) / 256)
+                                : nchunks <= 8192 ? std::min<int64_t>(c->opt_build_span, 64)
+                                                  : c->opt_build_span;
     const int64_t span = span_chunks * (int64_t)bc;
     const uint64_t spans = c->opt_build_span > 0 ? (n + span - 1) / span : 0;
     const size_t xcap = 4 * spans + 64;
     if (n > 1) {
-        if (int e = ensure(c, c->box_cnt, BOX_SLOTS, "box round counters")) return e;
         if (int e = ensure(c, c->meet, m, "meeting records")) return e;
         if (int e = ensure(c, c->meet_far, m, "meeting ranges")) return e;
         const bool fresh = !c->flags.p || c->flags.cap < m;
@@ -1776,11 +1995,6 @@ int hierarchy(mmhrt_ctx_s* c, const K* keys, const uint32_t* ids, bool reserve_o
         rec(c, 9);
         return 0;
     }
-    // each pass takes a new generation; builds captured into a graph keep theirs, so such a
-    // graph is launched once (the batched time series), never replayed
-    if (++c->build_gen == 0xffffffffu) c->build_gen = 1;
-    hipLaunchKernelGGL(k_build_init, dim3(1), dim3(64), 0, s, c->box_cnt.p, c->build_gen, &c->info.p->pair_h,
-                       c->opt_leaf_pairs ? 1u : 0u);
     c->bvh_pairs = c->opt_leaf_pairs != 0;
     // worklists of the straddler rounds: the spare key buffer (free once the sort is done) and
     // the spare value buffer
@@ -1842,18 +2056,6 @@ int hierarchy(mmhrt_ctx_s* c, const K* keys, const uint32_t* ids, bool reserve_o
     return 0;
 }
 
-template <typename K>
-int build_typed(mmhrt_ctx_s* c, K* ka, K* kb, bool reserve_only) {
-    uint64_t n = c->n;
-    hipStream_t s = c->stream;
-    if (int e = morton_sort<K>(c, ka, kb, c->va.p, c->vb.p, c->leaf_id.p, n, reserve_only)) return e;
-    if (reserve_only) return hierarchy<K>(c, ka, c->leaf_id.p, true);
-    rec(c, 3);
-    rec(c, 4);  // the leaf gather runs inside the hierarchy pass
-    // the sort's last pass wrote its values (the leaf -> particle map) straight into leaf_id
-    return hierarchy<K>(c, ka, c->leaf_id.p);
-}
-
 }  // namespace
 
 int count_leaf_pairs(mmhrt_ctx_s* c, int64_t* out) {
@@ -1884,14 +2086,62 @@ void launch_fill_u32(hipStream_t s, uint32_t* p, uint32_t v, uint64_t n) {
 
 static int reserve_reduction(mmhrt_ctx_s* c) {
     if (int e = ensure(c, c->partial, (size_t)REDUCE_BLOCKS * NRED, "reduction partials")) return e;
+    if (int e = ensure(c, c->box_cnt, BOX_SLOTS, "box round counters")) return e;
     return ensure(c, c->info, 1, "scene info");
 }
-int reduce_scene(mmhrt_ctx_s* c) {
-    const int nb = REDUCE_BLOCKS;
+// What the next hierarchy pass starts from. Each pass takes a new generation; builds captured into a
+// graph keep theirs, so such a graph is launched once (the batched time series), never replayed.
+static PassInit pass_init(mmhrt_ctx_s* c) {
+    if (++c->build_gen == 0xffffffffu) c->build_gen = 1;
+    return PassInit{c->box_cnt.p, c->build_gen, c->opt_leaf_pairs ? 1u : 0u};
+}
+static int reduce_scene(mmhrt_ctx_s* c, const PassInit& init) {
     if (int e = reserve_reduction(c)) return e;
+    // 8 spheres per thread, at most REDUCE_BLOCKS blocks (fewer leave the final block less to read)
+    const int nb = (int)std::min<uint64_t>(REDUCE_BLOCKS, (c->n + 2047) / 2048);
     hipLaunchKernelGGL(k_reduce_partial, dim3(nb), dim3(256), 0, c->stream, cur_spheres(c), c->n, c->partial.p);
-    hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(256), 0, c->stream, c->partial.p, nb, c->info.p, c->bits);
+    hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(256), 0, c->stream, c->partial.p, nb, c->info.p, c->bits, init);
     return 0;
+}
+int reduce_scene(mmhrt_ctx_s* c) { return reduce_scene(c, PassInit{nullptr, 0u, 0u}); }
+
+// Spheres that one workgroup sorts by itself: as many keys and 16-bit values as LDS holds.
+template <typename K>
+constexpr uint64_t small_sort_max() { return sizeof(K) == 8 ? 8192 : 16384; }
+
+// Scene bounds, Morton codes and sort: the sorted keys in ka, the particle of each place in ids.
+template <typename K>
+static int bounds_and_sort(mmhrt_ctx_s* c, K* ka, K* kb, uint32_t* ids, bool reserve_only) {
+    const uint64_t n = c->n;
+    if (int e = reserve_reduction(c)) return e;
+    const bool plain = c->opt_sort_digit != 0 && c->opt_sort_onesweep == 0 && c->opt_sort_ri == 16;
+    if (plain && n <= small_sort_max<K>()) {
+        if (reserve_only) return 0;
+        rec(c, 1);
+        rec(c, 2);
+        const PassInit init = pass_init(c);
+        auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(1), dim3(1024), 0, c->stream, cur_spheres(c), (uint32_t)n, c->info.p, c->bits,
+                               init, ka, ids);
+        };
+        // (every key a thread may hold costs its share of each pass, whether it is there or not)
+        if (n <= 2048)
+            go(k_small_sort<K, 2>);
+        else if (n <= 5120)
+            go(k_small_sort<K, 5>);
+        else if (n <= 8192)
+            go(k_small_sort<K, 8>);
+        else if constexpr (sizeof(K) == 4) {
+            if (n <= 12288)
+                go(k_small_sort<K, 12>);
+            else
+                go(k_small_sort<K, 16>);
+        }
+        return 0;
+    }
+    if (!reserve_only)
+        if (int e = reduce_scene(c, pass_init(c))) return e;
+    return morton_sort<K>(c, ka, kb, c->va.p, c->vb.p, ids, n, reserve_only);
 }
 
 // The first half of a build, shared by the treelet P-k-d build: scene bounds, Morton codes and
@@ -1913,9 +2163,18 @@ int sort_spheres(mmhrt_ctx_s* c, int bits, bool reserve_only) {
         if ((e = ensure(c, c->kb, n, "keys"))) return e;
     }
     if (!reserve_only) rec(c, 0);
-    if ((e = reserve_only ? reserve_reduction(c) : reduce_scene(c))) return e;
-    if (bits == 63) return morton_sort<uint64_t>(c, c->kla.p, c->klb.p, c->va.p, c->vb.p, c->leaf_id.p, n, reserve_only);
-    return morton_sort<uint32_t>(c, c->ka.p, c->kb.p, c->va.p, c->vb.p, c->leaf_id.p, n, reserve_only);
+    if (bits == 63) return bounds_and_sort<uint64_t>(c, c->kla.p, c->klb.p, c->leaf_id.p, reserve_only);
+    return bounds_and_sort<uint32_t>(c, c->ka.p, c->kb.p, c->leaf_id.p, reserve_only);
+}
+
+template <typename K>
+static int build_typed(mmhrt_ctx_s* c, K* ka, K* kb, bool reserve_only) {
+    if (int e = bounds_and_sort<K>(c, ka, kb, c->leaf_id.p, reserve_only)) return e;
+    if (reserve_only) return hierarchy<K>(c, ka, c->leaf_id.p, true);
+    rec(c, 3);
+    rec(c, 4);  // the leaf gather runs inside the hierarchy pass
+    // the sort's last pass wrote its values (the leaf -> particle map) straight into leaf_id
+    return hierarchy<K>(c, ka, c->leaf_id.p);
 }
 
 int build_lbvh(mmhrt_ctx_s* c, int bits, bool reserve_only) {
@@ -1938,7 +2197,6 @@ int build_lbvh(mmhrt_ctx_s* c, int bits, bool reserve_only) {
         if ((e = ensure(c, c->kb, n, "keys"))) return e;
     }
     if (!reserve_only) rec(c, 0);
-    if ((e = reserve_only ? reserve_reduction(c) : reduce_scene(c))) return e;
     if (bits == 63)
         e = build_typed<uint64_t>(c, c->kla.p, c->klb.p, reserve_only);
     else
@@ -1962,7 +2220,8 @@ int refit_lbvh(mmhrt_ctx_s* c) {
     if (!c->built || c->built_n != c->n || c->accel != 0)
         return fail(c, MMHRT_E_STATE, "refit: no matching LBVH to refit");
     rec(c, 0);
-    if (int e = reduce_scene(c)) return e;
+    if (int e = reserve_reduction(c)) return e;
+    if (int e = reduce_scene(c, pass_init(c))) return e;
     rec(c, 1);
     rec(c, 2);
     rec(c, 3);
