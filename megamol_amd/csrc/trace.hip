@@ -475,8 +475,15 @@ __device__ __forceinline__ float slab_io(const RayPre& r, float lx, float ly, fl
 // [t0, min(slab exit, t1, best)], the far child [max(t0, slab entry), min(t1, best)]. Closed
 // intervals, so that equal-t hits still reach the lowest particle id. Before its exact test a
 // sphere must also meet the ray in its own box. A pushed P-k-d entry keeps
-// its entry distance (two stack words: t0 below the reference) and resumes with t1 = the best
-// hit at the time it is popped. A treelet is entered at its root over its box's [entry, exit].
+// its entry distance and resumes with t1 = the best hit at the time it is popped. A treelet is
+// entered at its root over its box's [entry, exit].
+// The lowest three levels of a treelet are not walked: at a node whose great-grandchildren are past the
+// treelet's end the up to 7 spheres of its subtree are fetched together and tested against their own
+// boxes. Most of the visits were there, each a sphere and a split axis behind the one before. As in the
+// LBVH's two phases, a wavefront's lanes visit top nodes until at most 3/8 of them still do, then P-k-d
+// nodes. 8M clustered spheres at 1280x720, 1-spp AO: 8.1 ms walked to the leaves, 7.3 with the lowest two
+// levels together, 6.6 with three (bound by the latency of dependent fetches: vector ALU 40 % and address
+// unit 50 % busy); at 4, 5, 6 and 7 wavefronts per SIMD 7.0, 6.6, 7.4 and 8.1 (from 6 on it spills).
 // Closest hit (ANY false): returns the position of the hit (or -1) and its t in t_best. ANY:
 // returns 1 at the first hit of a sphere other than position `skip`, else 0.
 template <int S, bool COUNT, bool ANY>
@@ -491,9 +498,39 @@ __device__ int trace_tl(const TraceArgs& A, const RayPre& r, float tmin, float t
     float rmax = 0.0f;
     const uint32_t lg = A.tl_log2;
     const uint32_t msk = (1u << lg) - 1u;
-    for (;;) {
-        bool pop = false;
-        if (node >= 0) {
+    auto pop = [&]() {
+        node = REF_NONE;
+        while (st.sp > 0) {
+            const int2 e = st.take();
+            if (__int_as_float(e.y) > t_best) continue;
+            node = e.x;
+            t0 = __int_as_float(e.y);
+            t1 = t_best;
+            break;
+        }
+    };
+    // a sphere against its own box (centre -+ radius: the leaf box an LBVH traversal tests before
+    // its sphere; a filter that changes no result, most spheres near the ray lie off it), then exactly
+    auto test = [&](uint32_t p, const float4& sp) -> bool {
+        if ((ANY && (int)p == skip) || slab(r, sp.x - sp.w, sp.y - sp.w, sp.z - sp.w, sp.x + sp.w, sp.y + sp.w,
+                                            sp.z + sp.w, tmin, t_best) == INFINITY)
+            return false;
+        if (COUNT) cnt.tests++;
+        const float t = sphere_t(r.o, r.d, sp, tmin, tmax);
+        if (t >= 0.0f) {
+            if (ANY) return true;
+            if (t < t_best) {
+                t_best = t;
+                best = (int)p;
+            } else if (t == t_best && best >= 0 && A.leaf_id[p] < A.leaf_id[best]) {
+                best = (int)p;
+            }
+        }
+        return false;
+    };
+    while (node != REF_NONE) {
+        const int few_top = (int)__popcll(__ballot(node >= 0)) * 3 / 8;
+        while (node >= 0) {
             const float4* q = reinterpret_cast<const float4*>(A.nodes + node);
             const float4 a = q[0], b = q[1], c = q[2];
             const int4 d = reinterpret_cast<const int4*>(q)[3];
@@ -505,26 +542,19 @@ __device__ int trace_tl(const TraceArgs& A, const RayPre& r, float tmin, float t
             // a treelet child ~t becomes the P-k-d root at position t << lg
             const int32_t r0 = d.x >= 0 ? d.x : (int32_t)~((uint32_t)(~d.x) << lg);
             const int32_t r1 = d.y >= 0 ? d.y : (int32_t)~((uint32_t)(~d.y) << lg);
-            if (h0 && h1) {
-                const bool first0 = tn0 <= tn1;
-                const int32_t rn = first0 ? r0 : r1, rf = first0 ? r1 : r0;
-                const float tnf = first0 ? tn1 : tn0;
-                st.push(rf, tnf);
-                node = rn;
+            if (h0 || h1) {
+                const bool first0 = h0 && (!h1 || tn0 <= tn1);
+                if (h0 && h1) st.push(first0 ? r1 : r0, first0 ? tn1 : tn0);
+                node = first0 ? r0 : r1;
                 t0 = first0 ? tn0 : tn1;
                 t1 = first0 ? tf0 : tf1;
-            } else if (h0) {
-                node = r0;
-                t0 = tn0;
-                t1 = tf0;
-            } else if (h1) {
-                node = r1;
-                t0 = tn1;
-                t1 = tf1;
             } else {
-                pop = true;
+                pop();
             }
-        } else {
+            if ((int)__popcll(__ballot(node >= 0)) <= few_top) break;
+        }
+        const int few_tl = (int)__popcll(__ballot(node < 0 && node != REF_NONE)) * 3 / 8;
+        while (node < 0 && node != REF_NONE) {
             const uint32_t p = ~(uint32_t)node;
             const uint32_t tl = p >> lg;
             if (tl != cur_tl) {
@@ -535,68 +565,53 @@ __device__ int trace_tl(const TraceArgs& A, const RayPre& r, float tmin, float t
             }
             const uint32_t i = p & msk, bs = p - i;
             const float4 sp = A.leaf_sph[p];
-            const int dd = A.pkd_dim[p];
-            if (COUNT) cnt.visits++;
-            const float sc = dd == 0 ? sp.x : (dd == 1 ? sp.y : sp.z);
-            const float inv = dd == 0 ? r.inv.x : (dd == 1 ? r.inv.y : r.inv.z);
-            const float oil = dd == 0 ? r.oil.x : (dd == 1 ? r.oil.y : r.oil.z);
-            const float oih = dd == 0 ? r.oih.x : (dd == 1 ? r.oih.y : r.oih.z);
-            const float tlo = __builtin_fmaf(sc - rmax, inv, -oil), thi = __builtin_fmaf(sc + rmax, inv, -oih);
-            const float tnr = fminf(tlo, thi), tfr = fmaxf(tlo, thi);
-            float lim = fminf(t1, t_best);
-            // a sphere in the node's interval is tested against its own box first (centre -+
-            // radius: the leaf box an LBVH traversal tests before its sphere), a filter that
-            // changes no result: most spheres in a slab lie off the ray in the other two axes
-            if (fmaxf(t0, tnr) <= fminf(tfr, lim) && (!ANY || (int)p != skip) &&
-                slab(r, sp.x - sp.w, sp.y - sp.w, sp.z - sp.w, sp.x + sp.w, sp.y + sp.w, sp.z + sp.w, tmin,
-                     t_best) != INFINITY) {
-                if (COUNT) cnt.tests++;
-                const float t = sphere_t(r.o, r.d, sp, tmin, tmax);
-                if (t >= 0.0f) {
-                    if (ANY) return 1;
-                    if (t < t_best) {
-                        t_best = t;
-                        best = (int)p;
-                    } else if (t == t_best && best >= 0 && A.leaf_id[p] < A.leaf_id[best]) {
-                        best = (int)p;
-                    }
-                    lim = fminf(t1, t_best);
+            if (8 * i + 7 >= m) {
+                // (a place past the end repeats the node)
+                float4 g[6];
+                uint32_t pg[6];
+#pragma unroll
+                for (uint32_t k = 0; k < 6; ++k) {
+                    const uint32_t c = k < 2 ? 2 * i + 1 + k : 4 * i + 1 + k;
+                    pg[k] = c < m ? bs + c : p;
+                    g[k] = A.leaf_sph[pg[k]];
                 }
-            }
-            const float n_t1 = fminf(tfr, lim), f_t0 = fmaxf(t0, tnr);
-            const uint32_t sg = inv < 0.0f ? 1u : 0u;
-            const uint32_t nc = 2 * i + 1 + sg, fc = 2 * i + 2 - sg;
-            const bool need_n = nc < m && t0 <= n_t1;
-            const bool need_f = fc < m && f_t0 <= lim;
-            if (need_n && need_f) {
-                st.push(~(int32_t)(bs + fc), f_t0);
-                node = ~(int32_t)(bs + nc);
-                t1 = n_t1;
-            } else if (need_n) {
-                node = ~(int32_t)(bs + nc);
-                t1 = n_t1;
-            } else if (need_f) {
-                node = ~(int32_t)(bs + fc);
-                t0 = f_t0;
-                t1 = lim;
+                if (COUNT) cnt.visits += 7;
+                bool hit = test(p, sp);
+#pragma unroll
+                for (uint32_t k = 0; k < 6; ++k) hit = hit || test(pg[k], g[k]);
+                if (ANY && hit) return 1;
+                pop();
             } else {
-                pop = true;
-            }
-        }
-        if (pop) {
-            for (;;) {
-                if (st.sp == 0) return ANY ? 0 : best;
-                const int2 e = st.take();
-                const float a0 = __int_as_float(e.y);
-                if (a0 <= t_best) {
-                    node = e.x;
-                    t0 = a0;
-                    t1 = t_best;
-                    break;
+                const int dd = A.pkd_dim[p];
+                if (COUNT) cnt.visits++;
+                const float sc = dd == 0 ? sp.x : (dd == 1 ? sp.y : sp.z);
+                const float inv = dd == 0 ? r.inv.x : (dd == 1 ? r.inv.y : r.inv.z);
+                const float oil = dd == 0 ? r.oil.x : (dd == 1 ? r.oil.y : r.oil.z);
+                const float oih = dd == 0 ? r.oih.x : (dd == 1 ? r.oih.y : r.oih.z);
+                const float tlo = __builtin_fmaf(sc - rmax, inv, -oil), thi = __builtin_fmaf(sc + rmax, inv, -oih);
+                const float tnr = fminf(tlo, thi), tfr = fmaxf(tlo, thi);
+                if (fmaxf(t0, tnr) <= fminf(tfr, fminf(t1, t_best)) && test(p, sp)) return 1;  // (true only for ANY)
+                const float lim = fminf(t1, t_best);
+                const float n_t1 = fminf(tfr, lim), f_t0 = fmaxf(t0, tnr);
+                const uint32_t sg = inv < 0.0f ? 1u : 0u;
+                const uint32_t nc = 2 * i + 1 + sg, fc = 2 * i + 2 - sg;  // both lie inside the treelet here
+                const bool need_n = t0 <= n_t1, need_f = f_t0 <= lim;
+                if (need_n) {
+                    if (need_f) st.push(~(int32_t)(bs + fc), f_t0);
+                    node = ~(int32_t)(bs + nc);
+                    t1 = n_t1;
+                } else if (need_f) {
+                    node = ~(int32_t)(bs + fc);
+                    t0 = f_t0;
+                    t1 = lim;
+                } else {
+                    pop();
                 }
             }
+            if ((int)__popcll(__ballot(node < 0 && node != REF_NONE)) <= few_tl) break;
         }
     }
+    return ANY ? 0 : best;
 }
 
 // The structure a kernel traverses: TL = treelet P-k-d trees, else the LBVH.
@@ -799,7 +814,7 @@ __device__ void shade_pixel(const TraceArgs& A, uint32_t px, uint32_t py, float 
 // ms; 60M clustered at 4K: 6.7 against 5.7; 10k spheres at 320x240: 92 against 80 us): bound by the
 // vector memory unit's address rate (busy 60-90 %), then by VALU issue (50-70 %).
 template <int S, int MODE, bool COUNT, bool STEAL, bool TL = false>
-__global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(7, 8))) void k_trace(TraceArgs A) {
+__global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(TL ? 5 : 7, 8))) void k_trace(TraceArgs A) {
     __shared__ int2 lds_stack[LaneStack<S>::N * TB];
     const uint32_t gtid = blockIdx.x * TB + threadIdx.x;
     LaneStack<S> st{lds_stack + threadIdx.x, A.spill + gtid, A.spill_stride, 0, A.ctr + 1};
@@ -892,7 +907,7 @@ __device__ __forceinline__ void shade_sample(const TraceArgs& A, uint32_t px, ui
 // vector ALU issue before; 16 spp of 3M spheres at 1000x621: 3.66 -> 1.97 ms). Held to 72 VGPRs (7
 // wavefronts per SIMD, a few registers spilled) like the other lane kernels.
 template <int S, int MODE, bool COUNT, bool TL = false>
-__global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(7, 8))) void k_trace_sl(TraceArgs A) {
+__global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(TL ? 5 : 7, 8))) void k_trace_sl(TraceArgs A) {
     __shared__ int2 lds_stack[LaneStack<S>::N * TB];
     const uint32_t gtid = blockIdx.x * TB + threadIdx.x;
     LaneStack<S> st{lds_stack + threadIdx.x, A.spill + gtid, A.spill_stride, 0, A.ctr + 1};
@@ -1299,7 +1314,7 @@ void launch_refill(const TraceArgs& A, const Grid& g, uint32_t refill, bool coun
 // with its job's constants and output buffers.
 // Held to 72 VGPRs (7 wavefronts per SIMD) like the single-frame kernels.
 template <int S, int MODE, bool TL = false>
-__global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(7, 8))) void k_trace_batch(const TraceArgs* __restrict__ jobs,
+__global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(TL ? 5 : 7, 8))) void k_trace_batch(const TraceArgs* __restrict__ jobs,
                                                     const uint32_t* __restrict__ prefix, uint32_t n_jobs,
                                                     uint32_t* ctr) {
     __shared__ int2 lds_stack[LaneStack<S>::N * TB];
