@@ -17,12 +17,12 @@
 // Memory beyond the spheres in treelet order: one byte per sphere (the split axis), 28 bytes per
 // treelet and 64 bytes per top node, against 64 bytes per stored LBVH node.
 //
-// One 256-thread workgroup builds one treelet in LDS, level by level: the spheres never move;
-// 64-bit keys (segment start, coordinate on the segment's axis, local index) are bitonic-sorted
-// once per level, which orders every segment on its own axis in place, and the element of rank
-// |left subtree| in each segment is fixed at its in-order position. A key whose segment start is
-// its own position marks an element already fixed: the keys stay ordered by position, so it never
-// moves.
+// One 256-thread workgroup builds one treelet in LDS. The spheres never move: three lists hold their
+// local indices in the order of each coordinate (sorted once, stably, so that equal coordinates keep
+// the Morton order). Level by level every segment's node takes the element of rank |left subtree| from
+// the list of its axis, and the three lists are partitioned stably about it, so that each segment stays
+// sorted on every axis. (Sorting the segments anew at every level, bitonically, 55 exchange steps for
+// 1024 spheres, took 3.3 ms for 8M spheres; this takes 1.0 ms.)
 #include <float.h>
 
 #include <algorithm>
@@ -65,39 +65,73 @@ __device__ __forceinline__ int widest_axis(const float* b) {
     return d;
 }
 
+// Mask of the lanes whose (valid) 8-bit digit equals ours.
+__device__ __forceinline__ uint64_t same_digit(uint32_t d, bool valid) {
+    uint64_t m = __ballot(valid);
+#pragma unroll
+    for (int b = 0; b < 8; ++b) {
+        const uint64_t bm = __ballot((d >> b) & 1u);
+        m &= ((d >> b) & 1u) ? bm : ~bm;
+    }
+    return m;
+}
+
 template <int M>
 __global__ __launch_bounds__(256) void k_pkd_treelet(const float4* __restrict__ sph, uint32_t* __restrict__ ids,
                                                      float4* __restrict__ out_sph, uint8_t* __restrict__ out_dim,
                                                      float* __restrict__ tl_box, float* __restrict__ tl_rmax,
                                                      uint64_t n) {
-    constexpr int NT = M / 256;
+    constexpr int NT = M / 256;        // elements or positions per thread
+    constexpr int HALF = M / 2 + 1;    // nodes that can have children
+    struct Sort {                      // the initial sorts
+        uint32_t key[M];
+        uint16_t val[M];
+        uint16_t wc[4][256];
+        uint32_t wsum[4];
+    };
+    struct Level {                     // the levels
+        float box[HALF * 6];           // cell of heap node i
+        uint16_t pre[3][M];            // lefts before a position of a list, counted from its wavefront's first
+        uint16_t mpos[3][HALF];        // where a list holds the median of a level's k-th node
+        uint16_t wtot[3][4];           // lefts of each wavefront's positions
+    };
+    union Scratch {
+        Sort s;
+        Level l;
+    };
     __shared__ float4 s_sph[M];
-    __shared__ uint32_t s_id[M];
-    __shared__ uint64_t s_key[M];
-    __shared__ float s_box[M * 6];   // cell of heap node i
+    __shared__ uint16_t s_list[3][M];
+    __shared__ Scratch u;
     __shared__ uint16_t s_start[M];  // in-order start of node i's segment
     __shared__ uint16_t s_pos[M];    // segment (heap node) holding position p; bit 15: p is fixed
     __shared__ uint16_t s_elem[M];   // node i's sphere (local index)
     __shared__ uint8_t s_dim[M];
+    __shared__ uint8_t s_side[M];    // an element's place about its segment's median: 0 left, 1 median, 2 right
     __shared__ float s_red[4][7];
-    const uint32_t tid = threadIdx.x;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wv = tid >> 6;
+    const uint64_t lt = (1ull << lane) - 1ull;
     const uint64_t base = (uint64_t)blockIdx.x * M;
     const uint32_t m = (uint32_t)std::min<uint64_t>(M, n - base);
+    // positions of a thread: wavefront w holds M / 4 consecutive ones and walks them 64 at a time
+    const uint32_t pb = wv * (M / 4) + lane;
     float lo[3] = {FLT_MAX, FLT_MAX, FLT_MAX}, hi[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
     float rmax = 0.0f;
     uint32_t idv[NT];
 #pragma unroll
     for (int k = 0; k < NT; ++k) {
-        const uint32_t j = tid + 256u * k;
+        const uint32_t j = pb + 64u * k;
         idv[k] = j < m ? ids[base + j] : 0u;
     }
+    float4 own[NT];
 #pragma unroll
     for (int k = 0; k < NT; ++k) {
-        const uint32_t j = tid + 256u * k;
+        const uint32_t j = pb + 64u * k;
+        own[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+        s_pos[j] = j < m ? 0 : 0x8000u;
         if (j < m) {
             const float4 q = sph[idv[k]];
+            own[k] = q;
             s_sph[j] = q;
-            s_id[j] = idv[k];
             lo[0] = fminf(lo[0], q.x - q.w);
             lo[1] = fminf(lo[1], q.y - q.w);
             lo[2] = fminf(lo[2], q.z - q.w);
@@ -105,10 +139,6 @@ __global__ __launch_bounds__(256) void k_pkd_treelet(const float4* __restrict__ 
             hi[1] = fmaxf(hi[1], q.y + q.w);
             hi[2] = fmaxf(hi[2], q.z + q.w);
             rmax = fmaxf(rmax, q.w);
-        }
-        if (j < M) {
-            s_key[j] = j;
-            s_pos[j] = 0;
         }
     }
     // treelet bounds: min / max are exact in any order
@@ -119,15 +149,78 @@ __global__ __launch_bounds__(256) void k_pkd_treelet(const float4* __restrict__ 
         }
         rmax = fmaxf(rmax, __shfl_xor(rmax, o, 64));
     }
-    const uint32_t wv = tid >> 6;
-    if ((tid & 63) == 0) {
+    if (lane == 0) {
         for (int a = 0; a < 3; ++a) {
             s_red[wv][a] = lo[a];
             s_red[wv][3 + a] = hi[a];
         }
         s_red[wv][6] = rmax;
     }
-    __syncthreads();
+    // the three sorts: least significant digit first, ranked with ballots (wavefront, round and lane
+    // order together are the input order, so each pass is stable)
+    for (int ax = 0; ax < 3; ++ax) {
+        uint32_t key[NT], val[NT], rank[NT];
+#pragma unroll
+        for (int k = 0; k < NT; ++k) {
+            key[k] = ford(coord(own[k], ax));
+            val[k] = pb + 64u * k;
+        }
+        for (int shift = 0; shift < 32; shift += 8) {
+            for (uint32_t d = lane; d < 256; d += 64) u.s.wc[wv][d] = 0;
+#pragma unroll
+            for (int k = 0; k < NT; ++k) {
+                const bool valid = pb + 64u * k < m;
+                const uint32_t d = (key[k] >> shift) & 255u;
+                const uint64_t peers = same_digit(d, valid);
+                const uint32_t before = valid ? u.s.wc[wv][d] : 0u;
+                rank[k] = before + (uint32_t)__popcll(peers & lt);
+                if (valid && (peers & lt) == 0) u.s.wc[wv][d] = (uint16_t)(before + (uint32_t)__popcll(peers));
+            }
+            __syncthreads();
+            uint32_t c[4], cnt = 0;  // thread = digit
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                c[w] = u.s.wc[w][tid];
+                cnt += c[w];
+            }
+            uint32_t inc = cnt;
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const uint32_t y = __shfl_up(inc, o, 64);
+                if (lane >= (uint32_t)o) inc += y;
+            }
+            if (lane == 63) u.s.wsum[wv] = inc;
+            __syncthreads();
+            uint32_t run = inc - cnt;
+            for (uint32_t w = 0; w < wv; ++w) run += u.s.wsum[w];
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                u.s.wc[w][tid] = (uint16_t)run;
+                run += c[w];
+            }
+            __syncthreads();
+            const bool last = shift == 24;
+#pragma unroll
+            for (int k = 0; k < NT; ++k)
+                if (pb + 64u * k < m) {
+                    const uint32_t pos = u.s.wc[wv][(key[k] >> shift) & 255u] + rank[k];
+                    if (last) {
+                        s_list[ax][pos] = (uint16_t)val[k];
+                    } else {
+                        u.s.key[pos] = key[k];
+                        u.s.val[pos] = (uint16_t)val[k];
+                    }
+                }
+            __syncthreads();
+            if (!last) {
+#pragma unroll
+                for (int k = 0; k < NT; ++k) {
+                    key[k] = u.s.key[pb + 64u * k];  // (past m: not used)
+                    val[k] = u.s.val[pb + 64u * k];
+                }
+            }
+        }
+    }
     if (tid == 0) {
         float b[6];
         for (int a = 0; a < 3; ++a) {
@@ -136,96 +229,117 @@ __global__ __launch_bounds__(256) void k_pkd_treelet(const float4* __restrict__ 
         }
         const float r = fmaxf(fmaxf(s_red[0][6], s_red[1][6]), fmaxf(s_red[2][6], s_red[3][6]));
         for (int a = 0; a < 6; ++a) {
-            s_box[a] = b[a];
+            u.l.box[a] = b[a];
             tl_box[(size_t)blockIdx.x * 6 + a] = b[a];
         }
         tl_rmax[blockIdx.x] = r;
         s_dim[0] = (uint8_t)widest_axis(b);
         s_start[0] = 0;
     }
-    uint32_t mp = 1;
-    while (mp < m) mp <<= 1;
     __syncthreads();
     for (uint32_t first = 0; first < m; first = 2 * first + 1) {
         const uint32_t last = std::min(2 * first, m - 1);  // the nodes of this level
-        if (2 * first + 1 < m) {
-            // keys: (segment start, coordinate on the segment's axis, local index); a fixed
-            // element's segment is its own position
-            for (uint32_t p = tid; p < mp; p += 256) {
-                uint64_t key = ~0ull;
-                if (p < m) {
-                    const uint32_t j = (uint32_t)(s_key[p] & 0x3ffu);
-                    const uint32_t code = s_pos[p];
-                    if (code & 0x8000u) {
-                        key = ((uint64_t)p << 42) | j;
-                    } else {
-                        const float cv = coord(s_sph[j], s_dim[code]);
-                        key = ((uint64_t)s_start[code] << 42) | ((uint64_t)ford(cv) << 10) | j;
-                    }
-                }
-                s_key[p] = key;
-            }
-            __syncthreads();
-            for (uint32_t k = 2; k <= mp; k <<= 1)
-                for (uint32_t jj = k >> 1; jj > 0; jj >>= 1) {
-                    for (uint32_t q = tid; q < mp / 2; q += 256) {
-                        const uint32_t a = ((q & ~(jj - 1)) << 1) | (q & (jj - 1));
-                        const uint32_t b = a | jj;
-                        const uint64_t x = s_key[a], y = s_key[b];
-                        if ((x > y) == ((a & k) == 0)) {
-                            s_key[a] = y;
-                            s_key[b] = x;
-                        }
-                    }
-                    __syncthreads();
-                }
-        }
-        // fix each segment's element of rank |left subtree|; the rest go to the children
-        for (uint32_t p = tid; p < m; p += 256) {
-            const uint32_t code = s_pos[p];
-            if (code & 0x8000u) continue;
-            const uint32_t i = code;
-            const uint32_t L = 2 * i + 1 < m ? subtree_size(2 * i + 1, m) : 0u;
-            const uint32_t med = s_start[i] + L;
-            if (p == med) {
-                s_pos[p] = (uint16_t)(i | 0x8000u);
-                s_elem[i] = (uint16_t)(s_key[p] & 0x3ffu);
-            } else {
-                s_pos[p] = (uint16_t)(p < med ? 2 * i + 1 : 2 * i + 2);
+        const bool inner = 2 * first + 1 < m;              // some of them have children
+        // each segment's median is where the list of its axis has it; the elements of that list know
+        // their sides by their positions
+        uint32_t code[NT], med[NT];
+#pragma unroll
+        for (int k = 0; k < NT; ++k) {
+            const uint32_t p = pb + 64u * k;
+            code[k] = s_pos[p];
+            med[k] = 0;
+            if (!(code[k] & 0x8000u)) {
+                const uint32_t i = code[k];
+                const uint32_t L = 2 * i + 1 < m ? subtree_size(2 * i + 1, m) : 0u;
+                med[k] = s_start[i] + L;
+                const uint32_t j = s_list[s_dim[i]][p];
+                s_side[j] = p < med[k] ? 0 : (p == med[k] ? 1 : 2);
+                if (p == med[k]) s_elem[i] = (uint16_t)j;
             }
         }
         __syncthreads();
+        if (inner) {
+            // stable partition of the three lists: lefts before each position, by ballots
+            uint32_t el[3][NT];
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+                uint32_t run = 0;
+#pragma unroll
+                for (int k = 0; k < NT; ++k) {
+                    const uint32_t p = pb + 64u * k;
+                    const bool live = !(code[k] & 0x8000u);
+                    el[a][k] = live ? s_list[a][p] : 0u;
+                    const uint32_t sd = live ? s_side[el[a][k]] : 2u;
+                    const uint64_t lefts = __ballot(sd == 0u);
+                    u.l.pre[a][p] = (uint16_t)(run + (uint32_t)__popcll(lefts & lt));
+                    run += (uint32_t)__popcll(lefts);
+                    if (sd == 1u) u.l.mpos[a][code[k] - first] = (uint16_t)p;
+                    el[a][k] |= sd << 16;
+                }
+                if (lane == 0) u.l.wtot[a][wv] = (uint16_t)run;
+            }
+            __syncthreads();
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+#pragma unroll
+                for (int k = 0; k < NT; ++k) {
+                    if (code[k] & 0x8000u) continue;
+                    const uint32_t p = pb + 64u * k, i = code[k];
+                    const uint32_t st = s_start[i], sw = st / (M / 4);  // the segment's start and its wavefront
+                    uint32_t lefts = (uint32_t)u.l.pre[a][p] - (uint32_t)u.l.pre[a][st];
+                    for (uint32_t w = sw; w < wv; ++w) lefts += u.l.wtot[a][w];
+                    const uint32_t sd = el[a][k] >> 16;
+                    const uint32_t np = sd == 0u ? st + lefts
+                                       : sd == 1u ? med[k]
+                                                  : med[k] + 1 + (p - st) - lefts - (u.l.mpos[a][i - first] < p ? 1u : 0u);
+                    s_list[a][np] = (uint16_t)el[a][k];
+                }
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < NT; ++k) {
+            if (code[k] & 0x8000u) continue;
+            const uint32_t p = pb + 64u * k, i = code[k];
+            s_pos[p] = (uint16_t)(p == med[k] ? (i | 0x8000u) : (p < med[k] ? 2 * i + 1 : 2 * i + 2));
+        }
+        __syncthreads();
         // the children's cells, axes and segment starts
-        for (uint32_t i = first + tid; i <= last; i += 256) {
+        for (uint32_t i = first + tid; inner && i <= last; i += 256) {
+            if (2 * i + 1 >= m) continue;
             const int d = s_dim[i];
             const float cv = coord(s_sph[s_elem[i]], d);
-            const uint32_t L = 2 * i + 1 < m ? subtree_size(2 * i + 1, m) : 0u;
+            const uint32_t L = subtree_size(2 * i + 1, m);
             float b[6];
-            for (int a = 0; a < 6; ++a) b[a] = s_box[6 * i + a];
-            if (2 * i + 1 < m) {
+            for (int a = 0; a < 6; ++a) b[a] = u.l.box[6 * i + a];
+            for (uint32_t sd = 0; sd < 2; ++sd) {
+                const uint32_t ch = 2 * i + 1 + sd;
+                if (ch >= m) break;
                 float c[6];
                 for (int a = 0; a < 6; ++a) c[a] = b[a];
-                c[3 + d] = cv;
-                for (int a = 0; a < 6; ++a) s_box[6 * (2 * i + 1) + a] = c[a];
-                s_dim[2 * i + 1] = (uint8_t)widest_axis(c);
-                s_start[2 * i + 1] = s_start[i];
-            }
-            if (2 * i + 2 < m) {
-                float c[6];
-                for (int a = 0; a < 6; ++a) c[a] = b[a];
-                c[d] = cv;
-                for (int a = 0; a < 6; ++a) s_box[6 * (2 * i + 2) + a] = c[a];
-                s_dim[2 * i + 2] = (uint8_t)widest_axis(c);
-                s_start[2 * i + 2] = (uint16_t)(s_start[i] + L + 1);
+                c[sd ? d : 3 + d] = cv;
+                if (2 * ch + 1 < m)  // (a leaf's cell is not read again)
+                    for (int a = 0; a < 6; ++a) u.l.box[6 * ch + a] = c[a];
+                s_dim[ch] = (uint8_t)widest_axis(c);
+                s_start[ch] = (uint16_t)(sd ? s_start[i] + L + 1 : s_start[i]);
             }
         }
         __syncthreads();
     }
-    for (uint32_t i = tid; i < m; i += 256) {
-        const uint32_t j = s_elem[i];
-        out_sph[base + i] = s_sph[j];
-        ids[base + i] = s_id[j];
-        out_dim[base + i] = s_dim[i];
+    // the ids are permuted in place: all are read before any is written
+#pragma unroll
+    for (int k = 0; k < NT; ++k) {
+        const uint32_t i = tid + 256u * k;
+        idv[k] = i < m ? ids[base + s_elem[i]] : 0u;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < NT; ++k) {
+        const uint32_t i = tid + 256u * k;
+        if (i < m) {
+            out_sph[base + i] = s_sph[s_elem[i]];
+            ids[base + i] = idv[k];
+            out_dim[base + i] = s_dim[i];
+        }
     }
 }
 
