@@ -325,8 +325,8 @@ MMHRT_API int32_t mmhrt_denoiser_train_step(mmhrt_ctx ctx, const uint16_t* feats
                                             uint32_t h, uint32_t w, float depth_scale, const float bg[4], float lr,
                                             int32_t apply, float* loss_out, float* grads_out);
 
-/* Tuning knobs (autotuner output): "stack_lds" (LDS words of the traversal stack per lane: 8, 16, 24
- * or 32, default 16; an entry, a reference and its entry distance, takes two),
+/* Tuning knobs (autotuner output): "stack_lds" (part of the traversal stack in LDS: 8, 16, 24 or
+ * 32, default 16; 6, 10, 14 or 18 entries per lane of two words, a reference and its entry distance),
  * "tile_w", "tile_h", "persistent" (0/1), "refill" (ballot refill threshold in lanes; below 1,
  * the default: off), "blocks_per_cu" (persistent
  * workgroups per CU, at most as many as fit), "refit_period" (MMHRT_BUILD_AUTO: refits between rebuilds), "build_chunk"

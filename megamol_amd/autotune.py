@@ -2,7 +2,8 @@
 
 Knobs (library options, see include/mmhrt.h):
   tile_w         pixel tile width; a tile is one wavefront of 64 pixels (tile_w x 64/tile_w)
-  stack_lds      LDS words of the traversal stack per lane, two per entry (deeper entries spill to HBM)
+  stack_lds      part of the traversal stack in LDS: 8, 16, 24, 32 hold 6, 10, 14, 18 entries per lane
+                 (deeper entries spill to HBM)
   blocks_per_cu  persistent workgroups per compute unit
   refill         ballot-refill threshold in active lanes (0 = plain persistent kernel)
   refit_period   batched series: rebuild every k-th timestep, refit in between

@@ -136,7 +136,7 @@ struct mmhrt_ctx_s {
     mmhrt::DevBuf<uint32_t> counters;  // TRACE_CTR_WORDS: overflow flag, visit counters (u64 pairs), work queues
 
     // options
-    int64_t opt_stack_lds = 16;  // LDS words per lane (8 entries): leaves the LDS for 7 wavefronts per SIMD
+    int64_t opt_stack_lds = 16;  // LDS part of the stack, 10 entries: leaves the LDS for 8 workgroups per CU
     int64_t opt_persistent = 1;
     int64_t opt_refill = -1;  // ballot-refill threshold; below 1: off (the lane-per-pixel kernels)
     int64_t opt_count = 0;

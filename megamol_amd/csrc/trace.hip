@@ -113,49 +113,79 @@ constexpr int32_t REF_NONE = INT32_MIN;
 // Traversal stack of one lane: (reference, entry distance of its box), the lowest N entries in
 // LDS, lane-interleaved. Deeper entries spill their reference alone to the lane's global words
 // and come back with an entry distance below every ray's (they are visited without the test).
-// With SPILL_DIST in S they spill both words: for the treelets' shallow trees (at most 22 top levels
-// and 10 inside a treelet) the lane's words hold them, and an LDS stack of 8 entries instead of 16
-// keeps two more wavefronts per SIMD.
+// With SPILL_DIST in S they spill both words: the treelets' shallow trees (at most 22 top levels
+// and 10 inside a treelet) fit the lane's words that way.
+// Entry 0 is a sentinel (REF_NONE, nearer than everything), so a pop needs no test for an empty stack,
+// and the LDS accesses are 8 bytes through the LDS address space: with a pointer that could be to either
+// memory the compiler merged the LDS read with that of a spilled entry into a flat load after an address
+// select, on each pop's chain. The wavefront pops at one place per visit (a leaf put aside and a visit
+// without a hit are the same loop). Trace kernel: 60M clustered spheres at 4K 5.75 ms, then 5.49; 50M
+// FCC spheres at 1080p with AO, 1 sample 0.72, then 0.66, 64 samples 13.7, then 13.5; 8M treelets 6.9,
+// then 6.1. N = 10 is the most that leaves room for eight workgroups per CU (20 KB each); with 9, 8
+// (and the sentinel) the clusters take 5.58 and 5.51, the FCC spheres 13.8 and 13.9.
 constexpr int SPILL_DIST = 256;
+typedef int i32x2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) i32x2* lds_i32x2;
 template <int S>
 struct LaneStack {
     static constexpr int N = S & (SPILL_DIST - 1);
-    static constexpr int W = S & SPILL_DIST ? 2 : 1;                // words per spilled entry
+    static constexpr int W = S & SPILL_DIST ? 2 : 1;  // words per spilled entry
     static constexpr int CAP = N + TRACE_SPILL_PER_LANE / W;
-    int2* lds;  // element k at lds[k * TB]
+    lds_i32x2 lds;  // element k at lds[k * TB]
     int32_t* spill;
     uint32_t stride;
     int sp;
     uint32_t* overflow;
-    __device__ __forceinline__ void push(int32_t ref, float tn) {
-        if (__builtin_expect(sp < N, 1)) {
-            lds[sp * TB] = make_int2(ref, __float_as_int(tn));
-        } else if (sp < CAP) {
-            spill[(size_t)(W * (sp - N)) * stride] = ref;
-            if (W == 2) spill[(size_t)(W * (sp - N) + 1) * stride] = __float_as_int(tn);
-        } else {
-            *overflow = 1u;  // cannot happen for a valid tree; recorded, entry dropped
-            return;
-        }
-        ++sp;
+    __device__ __forceinline__ LaneStack(int2* shared, int32_t* sl, uint32_t st, uint32_t* ov)
+        : lds((lds_i32x2)shared), spill(sl), stride(st), sp(1), overflow(ov) {}
+    __device__ __forceinline__ void reset() {
+        lds[0] = (i32x2){REF_NONE, (int)0xff800000u};
+        sp = 1;
     }
-    // the top entry (the stack is not empty)
-    __device__ __forceinline__ int2 take() {
+    // on: this lane pushes
+    __device__ __forceinline__ void push(bool on, int32_t ref, float tn) {
+        if (__builtin_expect(on && sp >= N, 0)) {
+            if (sp < CAP) {
+                spill[(size_t)(W * (sp - N)) * stride] = ref;
+                if (W == 2) spill[(size_t)(W * (sp - N) + 1) * stride] = __float_as_int(tn);
+                ++sp;
+            } else {
+                *overflow = 1u;  // cannot happen for a valid tree; recorded, entry dropped
+            }
+            on = false;
+        }
+        if (on) {
+            lds[sp * TB] = (i32x2){ref, __float_as_int(tn)};
+            ++sp;
+        }
+    }
+    // the top entry (the stack holds at least the sentinel)
+    __device__ __forceinline__ i32x2 take() {
         --sp;
-        int2 e = lds[(sp < N ? sp : N - 1) * TB];
+        i32x2 e = lds[(sp < N ? sp : N - 1) * TB];
         if (__builtin_expect(sp >= N, 0)) {
             e.x = spill[(size_t)(W * (sp - N)) * stride];
             e.y = W == 2 ? spill[(size_t)(W * (sp - N) + 1) * stride] : (int)0xff800000u;
         }
         return e;
     }
-    // the topmost reference whose box starts no farther than t_best; REF_NONE when there is none
-    __device__ __forceinline__ int32_t pop(float t_best) {
-        while (sp > 0) {
-            const int2 e = take();
-            if (__int_as_float(e.y) <= t_best) return e.x;
+    // for the lanes with `on`: the topmost reference whose box starts no farther than t_best becomes the
+    // node (REF_NONE when there is none), or, if it is a leaf and none is aside, the one aside, and the
+    // next one the node
+    __device__ __forceinline__ void pop(bool on, float t_best, int32_t& node, int32_t& leaf) {
+        if (on) {
+            for (;;) {
+                i32x2 e;
+                do {
+                    e = take();
+                } while (__int_as_float(e.y) > t_best);
+                if (e.x >= 0 || e.x == REF_NONE || leaf != REF_NONE) {
+                    node = e.x;
+                    break;
+                }
+                leaf = e.x;
+            }
         }
-        return REF_NONE;
     }
 };
 
@@ -205,11 +235,12 @@ struct Count {
 // A stack entry keeps its box's entry distance, and one that lies beyond the best hit when its
 // turn comes is dropped without a fetch.
 
-// One visit: both child boxes against the ray; the near child becomes the node, a far one that is
-// hit too goes to the stack; with neither, the next from the stack.
+// One visit: both child boxes against the ray. The near child becomes the node, a far one that is hit
+// too goes to the stack. A leaf reference is put aside if the lane has none aside yet; then, and with
+// no child hit, the node is the next one from the stack.
 template <int S, bool COUNT>
 __device__ __forceinline__ void visit(const TraceArgs& A, const RayPre& r, float tmin, float t_best, int32_t& node,
-                                      LaneStack<S>& st, Count& cnt) {
+                                      int32_t& leaf, LaneStack<S>& st, Count& cnt) {
     const float4* q = reinterpret_cast<const float4*>(A.nodes + node);
     const float4 a = q[0], b = q[1], c = q[2];
     const int2 d = *reinterpret_cast<const int2*>(q + 3);
@@ -219,10 +250,11 @@ __device__ __forceinline__ void visit(const TraceArgs& A, const RayPre& r, float
     const bool first0 = tn0 <= tn1;
     const float tnear = first0 ? tn0 : tn1, tfar = first0 ? tn1 : tn0;
     node = first0 ? d.x : d.y;
-    if (tfar != INFINITY)
-        st.push(first0 ? d.y : d.x, tfar);
-    else if (tnear == INFINITY)
-        node = st.pop(t_best);
+    st.push(tfar != INFINITY, first0 ? d.y : d.x, tfar);
+    const bool none = tnear == INFINITY;
+    const bool put = !none && node < 0 && leaf == REF_NONE;
+    if (put) leaf = node;
+    st.pop(none || put, t_best, node, leaf);
 }
 
 // The part of sphere_t before its square root: false when that sphere reports no hit. (With b < 0
@@ -296,11 +328,7 @@ __device__ __forceinline__ void inner_phase(const TraceArgs& A, const RayPre& r,
                                             int32_t& node, int32_t& leaf, LaneStack<S>& st, Count& cnt) {
     const int few = (int)__popcll(__ballot(node >= 0)) * 3 / 8;
     while (node >= 0) {
-        visit<S, COUNT>(A, r, tmin, t_best, node, st, cnt);
-        if (node < 0 && leaf == REF_NONE && node != REF_NONE) {
-            leaf = node;
-            node = st.pop(t_best);
-        }
+        visit<S, COUNT>(A, r, tmin, t_best, node, leaf, st, cnt);
         if ((int)__popcll(__ballot(leaf == REF_NONE)) <= few) break;
     }
 }
@@ -312,16 +340,14 @@ __device__ int trace_closest(const TraceArgs& A, const RayPre& r, float tmin, fl
     int best = -1;
     t_best = tmax;
     int32_t node = 0, leaf = REF_NONE;
-    st.sp = 0;
+    st.reset();
     while (node != REF_NONE) {
         inner_phase<S, COUNT>(A, r, tmin, t_best, node, leaf, st, cnt);
         while (leaf != REF_NONE) {
             test_leaf<COUNT>(A, r, tmin, tmax, leaf, -1, false, t_best, best, cnt);
-            leaf = REF_NONE;
-            if (node < 0 && node != REF_NONE) {
-                leaf = node;
-                node = st.pop(t_best);
-            }
+            const bool more = node < 0;  // (REF_NONE, too: nothing aside then)
+            leaf = more ? node : REF_NONE;
+            st.pop(more && node != REF_NONE, t_best, node, leaf);
         }
     }
     return best;
@@ -332,18 +358,16 @@ template <int S, bool COUNT>
 __device__ bool trace_any(const TraceArgs& A, const RayPre& r, float tmin, float tmax, int skip, LaneStack<S>& st,
                           Count& cnt) {
     int32_t node = 0, leaf = REF_NONE;
-    st.sp = 0;
+    st.reset();
     float tb = tmax;
     int best = -1;
     while (node != REF_NONE) {
         inner_phase<S, COUNT>(A, r, tmin, tmax, node, leaf, st, cnt);
         while (leaf != REF_NONE) {
             if (test_leaf<COUNT>(A, r, tmin, tmax, leaf, skip, true, tb, best, cnt)) return true;
-            leaf = REF_NONE;
-            if (node < 0 && node != REF_NONE) {
-                leaf = node;
-                node = st.pop(tmax);
-            }
+            const bool more = node < 0;
+            leaf = more ? node : REF_NONE;
+            st.pop(more && node != REF_NONE, tmax, node, leaf);
         }
     }
     return false;
@@ -373,7 +397,8 @@ __device__ __forceinline__ int trace_closest_packet(const TraceArgs& A, const Ra
     int best = -1;
     t_best = tmax;
     int32_t node = 0;
-    int sp = 0;
+    st.reset();
+    int sp = 1;
     auto slab_oct = [&](float lx, float ly, float lz, float hx, float hy, float hz) -> float {
         const float xn = __builtin_fmaf(sx ? hx : lx, r.inv.x, -on.x), xf = __builtin_fmaf(sx ? lx : hx, r.inv.x, -of.x);
         const float yn = __builtin_fmaf(sy ? hy : ly, r.inv.y, -on.y), yf = __builtin_fmaf(sy ? ly : hy, r.inv.y, -of.y);
@@ -396,8 +421,8 @@ __device__ __forceinline__ int trace_closest_packet(const TraceArgs& A, const Ra
                 // the child that is nearer for more of the lanes first
                 const bool first0 = 2 * __popcll(__ballot(tn0 <= tn1 && tn0 != INFINITY)) >= __popcll(m0 | m1);
                 st.sp = sp;
-                st.push(first0 ? d.y : d.x, first0 ? tn1 : tn0);
-                sp = st.sp;
+                st.push(true, first0 ? d.y : d.x, first0 ? tn1 : tn0);
+                sp = __builtin_amdgcn_readfirstlane(st.sp);
                 node = first0 ? d.x : d.y;
                 pop = false;
             } else if (m0 | m1) {
@@ -432,9 +457,9 @@ __device__ __forceinline__ int trace_closest_packet(const TraceArgs& A, const Ra
             }
         }
         while (pop) {
-            if (sp == 0) return best;
+            if (sp == 1) return best;
             st.sp = sp;
-            const int2 e = st.take();
+            const i32x2 e = st.take();
             --sp;
             if (!__ballot(__int_as_float(e.y) <= t_best)) continue;
             node = __builtin_amdgcn_readfirstlane(e.x);
@@ -491,23 +516,21 @@ __device__ int trace_tl(const TraceArgs& A, const RayPre& r, float tmin, float t
                         LaneStack<S>& st, Count& cnt) {
     int best = -1;
     t_best = tmax;
-    st.sp = 0;
+    st.reset();
     int32_t node = 0;
     float t0 = 0.0f, t1 = 0.0f;
     uint32_t cur_tl = 0xffffffffu, m = 0;
     float rmax = 0.0f;
     const uint32_t lg = A.tl_log2;
     const uint32_t msk = (1u << lg) - 1u;
-    auto pop = [&]() {
-        node = REF_NONE;
-        while (st.sp > 0) {
-            const int2 e = st.take();
-            if (__int_as_float(e.y) > t_best) continue;
-            node = e.x;
-            t0 = __int_as_float(e.y);
-            t1 = t_best;
-            break;
-        }
+    auto pop = [&]() {  // (the sentinel ends it)
+        i32x2 e;
+        do {
+            e = st.take();
+        } while (__int_as_float(e.y) > t_best);
+        node = e.x;
+        t0 = __int_as_float(e.y);
+        t1 = t_best;
     };
     // a sphere against its own box (centre -+ radius: the leaf box an LBVH traversal tests before
     // its sphere; a filter that changes no result, most spheres near the ray lie off it), then exactly
@@ -544,7 +567,7 @@ __device__ int trace_tl(const TraceArgs& A, const RayPre& r, float tmin, float t
             const int32_t r1 = d.y >= 0 ? d.y : (int32_t)~((uint32_t)(~d.y) << lg);
             if (h0 || h1) {
                 const bool first0 = h0 && (!h1 || tn0 <= tn1);
-                if (h0 && h1) st.push(first0 ? r1 : r0, first0 ? tn1 : tn0);
+                st.push(h0 && h1, first0 ? r1 : r0, first0 ? tn1 : tn0);
                 node = first0 ? r0 : r1;
                 t0 = first0 ? tn0 : tn1;
                 t1 = first0 ? tf0 : tf1;
@@ -597,7 +620,7 @@ __device__ int trace_tl(const TraceArgs& A, const RayPre& r, float tmin, float t
                 const uint32_t nc = 2 * i + 1 + sg, fc = 2 * i + 2 - sg;  // both lie inside the treelet here
                 const bool need_n = t0 <= n_t1, need_f = f_t0 <= lim;
                 if (need_n) {
-                    if (need_f) st.push(~(int32_t)(bs + fc), f_t0);
+                    st.push(need_f, ~(int32_t)(bs + fc), f_t0);
                     node = ~(int32_t)(bs + nc);
                     t1 = n_t1;
                 } else if (need_f) {
@@ -817,7 +840,7 @@ template <int S, int MODE, bool COUNT, bool STEAL, bool TL = false>
 __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(TL ? 5 : 7, 8))) void k_trace(TraceArgs A) {
     __shared__ int2 lds_stack[LaneStack<S>::N * TB];
     const uint32_t gtid = blockIdx.x * TB + threadIdx.x;
-    LaneStack<S> st{lds_stack + threadIdx.x, A.spill + gtid, A.spill_stride, 0, A.ctr + 1};
+    LaneStack<S> st(lds_stack + threadIdx.x, A.spill + gtid, A.spill_stride, A.ctr + 1);
     Count cnt;
     // slab padding: a bound on the rounding of the FP32 sphere and slab tests, which scale with
     // the magnitude of ray origins and sphere centres (fc.pad carries max |camera coordinate|)
@@ -910,7 +933,7 @@ template <int S, int MODE, bool COUNT, bool TL = false>
 __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(TL ? 5 : 7, 8))) void k_trace_sl(TraceArgs A) {
     __shared__ int2 lds_stack[LaneStack<S>::N * TB];
     const uint32_t gtid = blockIdx.x * TB + threadIdx.x;
-    LaneStack<S> st{lds_stack + threadIdx.x, A.spill + gtid, A.spill_stride, 0, A.ctr + 1};
+    LaneStack<S> st(lds_stack + threadIdx.x, A.spill + gtid, A.spill_stride, A.ctr + 1);
     Count cnt;
     const FrameConsts& f = A.fc;
     const float amax = A.info->absmax;
@@ -1041,7 +1064,7 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(5, 8))) void
                                                                                                 uint32_t refill) {
     __shared__ int2 lds_stack[LaneStack<S>::N * TB];
     const uint32_t gtid = blockIdx.x * TB + threadIdx.x;
-    LaneStack<S> st{lds_stack + threadIdx.x, A.spill + gtid, A.spill_stride, 0, A.ctr + 1};
+    LaneStack<S> st(lds_stack + threadIdx.x, A.spill + gtid, A.spill_stride, A.ctr + 1);
     Count cnt;
     const FrameConsts& f = A.fc;
     const float amax = A.info->absmax;
@@ -1114,7 +1137,7 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(5, 8))) void
             t_best = tmax;
             best = -1;
             node = 0;
-            st.sp = 0;
+            st.reset();
             if (COUNT) cnt.rays++;
             state = L_PRIM;
         }
@@ -1129,14 +1152,13 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(5, 8))) void
                 inner_phase<S, COUNT>(A, r, tmin, t_best, node, leaf, st, cnt);
                 while (leaf != REF_NONE) {
                     const bool occ = test_leaf<COUNT>(A, r, tmin, tmax, leaf, ao ? skip : -1, ao, t_best, best, cnt);
-                    leaf = REF_NONE;
                     if (occ) {
                         best = 2;
                         node = REF_NONE;
-                    } else if (node < 0 && node != REF_NONE) {
-                        leaf = node;
-                        node = st.pop(t_best);
                     }
+                    const bool more = node < 0;
+                    leaf = more ? node : REF_NONE;
+                    st.pop(more && node != REF_NONE, t_best, node, leaf);
                 }
                 if (node == REF_NONE) state = ao ? L_AO_DONE : L_PRIM_DONE;
             }
@@ -1179,7 +1201,7 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(5, 8))) void
                     skip = best;
                     best = -1;
                     node = 0;
-                    st.sp = 0;
+                    st.reset();
                     if (COUNT) cnt.rays++;
                     state = L_AO;
                 } else {
@@ -1275,7 +1297,7 @@ void launch_sl(const TraceArgs& A, const Grid& g, bool count, int mode) {
 }
 
 // Kernels over the treelet P-k-d trees.
-constexpr int TL_STACK = 8 + SPILL_DIST;
+constexpr int TL_STACK = 10 + SPILL_DIST;
 template <int MODE, bool COUNT>
 void launch_tl_m(const TraceArgs& A, const Grid& g, bool sl) {
     if (sl && MODE != 2)
@@ -1319,7 +1341,7 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(TL ? 5 : 7, 
                                                     uint32_t* ctr) {
     __shared__ int2 lds_stack[LaneStack<S>::N * TB];
     const uint32_t gtid = blockIdx.x * TB + threadIdx.x;
-    LaneStack<S> st{lds_stack + threadIdx.x, jobs[0].spill + gtid, jobs[0].spill_stride, 0, ctr + 1};
+    LaneStack<S> st(lds_stack + threadIdx.x, jobs[0].spill + gtid, jobs[0].spill_stride, ctr + 1);
     Count cnt;
     const uint32_t lane = __lane_id();
     WorkQueue wq(ctr, prefix[n_jobs]);
@@ -1370,10 +1392,10 @@ void launch_trace_batch(mmhrt_ctx_s* c, const void* jobs, const uint32_t* prefix
     else                                                                    \
         launch_resident<k_trace_batch<SV, 0>>(g, J, prefix, n_jobs, ctr);
     switch (S) {
-    case 8: MMHRT_BATCH(4) break;
-    case 24: MMHRT_BATCH(12) break;
-    case 32: MMHRT_BATCH(16) break;
-    default: MMHRT_BATCH(8) break;
+    case 8: MMHRT_BATCH(6) break;
+    case 24: MMHRT_BATCH(14) break;
+    case 32: MMHRT_BATCH(18) break;
+    default: MMHRT_BATCH(10) break;
     }
 #undef MMHRT_BATCH
 }
@@ -1456,24 +1478,24 @@ void dispatch_trace(mmhrt_ctx_s* c, TraceArgs& A, unsigned grid, bool count) {
     }
     if (sl) {
         switch (S) {
-        case 8: launch_sl<4>(A, g, count, fc.mode); break;
-        case 24: launch_sl<12>(A, g, count, fc.mode); break;
-        case 32: launch_sl<16>(A, g, count, fc.mode); break;
-        default: launch_sl<8>(A, g, count, fc.mode); break;
+        case 8: launch_sl<6>(A, g, count, fc.mode); break;
+        case 24: launch_sl<14>(A, g, count, fc.mode); break;
+        case 32: launch_sl<18>(A, g, count, fc.mode); break;
+        default: launch_sl<10>(A, g, count, fc.mode); break;
         }
     } else if (refill > 0 && fc.mode != 2) {
         switch (S) {
-        case 8: launch_refill<4>(A, g, refill, count, fc.mode); break;
-        case 24: launch_refill<12>(A, g, refill, count, fc.mode); break;
-        case 32: launch_refill<16>(A, g, refill, count, fc.mode); break;
-        default: launch_refill<8>(A, g, refill, count, fc.mode); break;
+        case 8: launch_refill<6>(A, g, refill, count, fc.mode); break;
+        case 24: launch_refill<14>(A, g, refill, count, fc.mode); break;
+        case 32: launch_refill<18>(A, g, refill, count, fc.mode); break;
+        default: launch_refill<10>(A, g, refill, count, fc.mode); break;
         }
     } else {
         switch (S) {
-        case 8: launch1<4>(A, g, steal, count, fc.mode); break;
-        case 24: launch1<12>(A, g, steal, count, fc.mode); break;
-        case 32: launch1<16>(A, g, steal, count, fc.mode); break;
-        default: launch1<8>(A, g, steal, count, fc.mode); break;
+        case 8: launch1<6>(A, g, steal, count, fc.mode); break;
+        case 24: launch1<14>(A, g, steal, count, fc.mode); break;
+        case 32: launch1<18>(A, g, steal, count, fc.mode); break;
+        default: launch1<10>(A, g, steal, count, fc.mode); break;
         }
     }
 }
