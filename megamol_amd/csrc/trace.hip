@@ -695,7 +695,10 @@ __device__ __forceinline__ void write_pixel_main(const TraceArgs& A, uint32_t op
     A.out_rgba8[opix] = pack_rgba8(col);
 }
 
+// The values are rounded to 32 bits first: without the (empty) statement the compiler may take the
+// product or sum that makes one with the conversion as a single operation (v_fma_mixlo_f16), rounded once.
 __device__ __forceinline__ uint32_t half2_bits(float lo, float hi) {
+    asm("" : "+v"(lo), "+v"(hi));
     return (uint32_t)__half_as_ushort(__float2half(lo)) | ((uint32_t)__half_as_ushort(__float2half(hi)) << 16);
 }
 
@@ -923,11 +926,14 @@ __device__ __forceinline__ void shade_sample(const TraceArgs& A, uint32_t px, ui
 // pass, the lanes hold L = min(spp, 64) consecutive samples of each of 64/L pixels, so the
 // primary rays of a lane group start in one pixel and a background pixel costs one quick pass.
 // Sample s of a pixel draws its jitter from the pixel's stream advanced by 2s steps
-// (lcg_skip), and the group folds its samples into the pixel in sample order (colour sums,
+// (lcg_map), and the group folds its samples into the pixel in sample order (colour sums,
 // first strictly nearer hit, visibility, sample-0 features), so every output is bit-identical
 // to the lane-per-pixel kernels. The primary rays of a pass take one packet walk, the AO rays the
 // two-phase traversal lane by lane; 50M FCC spheres at 1080p, 64-spp AO: 31.5 -> 18.4 ms (bound by
-// vector ALU issue before; 16 spp of 3M spheres at 1000x621: 3.66 -> 1.97 ms). Held to 72 VGPRs (7
+// vector ALU issue before and after; 16 spp of 3M spheres at 1000x621: 3.66 -> 1.97 ms). What a pass
+// costs beside its rays was a quarter of the issue: the streams of a unit's pixels are set up together,
+// one per lane, four lanes sum a colour component each, the features are written by the lane that has
+// them, and a pass without a hit ends there (13.5 -> 12.7 ms, and 1.40 -> 1.34 ms). Held to 72 VGPRs (7
 // wavefronts per SIMD, a few registers spilled) like the other lane kernels.
 template <int S, int MODE, bool COUNT, bool TL = false>
 __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(TL ? 5 : 7, 8))) void k_trace_sl(TraceArgs A) {
@@ -946,95 +952,96 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(TL ? 5 : 7, 
     const uint32_t base = g * L;  // first lane of this lane's pixel group
     const uint32_t tw = 1u << A.tw_log2, th = 64u >> A.tw_log2;
     const uint32_t passes = L >> A.sub_log2;  // of a unit (a tile has 64 / G = L)
+    uint32_t ja, jc, ra, rc;  // the random stream's maps over 2 * sl draws and over a round's 2 * L
+    lcg_map(2u * sl, ja, jc);
+    lcg_map(2u * L, ra, rc);
     WorkQueue wq(A.ctr, A.n_tiles << A.sub_log2);
     for (;;) {
         const uint32_t unit = wq.grab();
         if (unit == 0xffffffffu) break;
         const uint32_t tile = unit >> A.sub_log2, q0 = (unit - (tile << A.sub_log2)) * passes;
         const uint32_t tx = tile % A.tiles_x, ty = tile / A.tiles_x;
+        // the stream of the tile's pixel `lane`
+        const uint32_t tseed = tea16((f.win_y0 + ty * th + (lane >> A.tw_log2)) * f.width + f.win_x0 + tx * tw +
+                                         (lane & (tw - 1)), f.frame_idx);
         for (uint32_t q = q0; q < q0 + passes; ++q) {
             const uint32_t tp = q * G + g;  // pixel of this group inside the tile
             const uint32_t px = f.win_x0 + tx * tw + (tp & (tw - 1)), py = f.win_y0 + ty * th + (tp >> A.tw_log2);
             const bool valid = px < f.win_x0 + f.win_w && py < f.win_y0 + f.win_h;
             const uint32_t pix = py * f.width + px;
-            const uint32_t seed0 = tea16(pix, f.frame_idx);
-            float4 col = make_float4(0.f, 0.f, 0.f, 0.f);
+            uint32_t seed0 = __shfl(tseed, (int)tp, 64);
+            float acc = 0.0f;  // colour sum of component sl
+            float4 sc;
             // best_t is the least hit distance over the samples, the pixel's depth (FLT_MAX without a hit)
             float best_t = INFINITY, vis_sum = 0.0f;
             int best_leaf = -1;
-            float aux[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+            float t0 = 0.0f;  // t of sample 0
             for (uint32_t rd = 0; rd < rounds; ++rd) {
                 const uint32_t s = rd * L + sl;
-                float4 sc = make_float4(0.f, 0.f, 0.f, 0.f);
+                sc = make_float4(0.f, 0.f, 0.f, 0.f);
                 float ray_depth = FLT_MAX, t = INFINITY, V = 0.0f;
                 int leaf = -1;
                 float4 alb = make_float4(0.f, 0.f, 0.f, 0.f);
                 V3 N = V3{0.f, 0.f, 0.f};
                 if (valid) {
-                    uint32_t seed = lcg_skip(seed0, 2u * s);
+                    uint32_t seed = ja * seed0 + jc;
                     float jx = rnd(seed);
                     float jy = rnd(seed);
                     shade_sample<S, MODE, COUNT, TL>(A, px, py, pix, s, jx, jy, pad, st, cnt, sc, ray_depth,
                                                             t, leaf, V, alb, N);
                 }
+                seed0 = ra * seed0 + rc;
+                const uint32_t opix = (py - f.win_y0) * f.win_w + (px - f.win_x0);
+                if (rd == 0 && valid && sl == 0) {  // features of sample 0
+                    write_aux_head(A, opix, alb.x, alb.y, alb.z, N.x, N.y, N.z);
+                    if (leaf >= 0) t0 = t;
+                }
+                // a pixel without a hit takes the background whatever its samples' colours sum to
+                if (rounds == 1 && __ballot(leaf >= 0) == 0) break;
                 // visibility is 0 or 1 per sample, so its sum is exact in any order: the count of
                 // the group's unoccluded hits
                 const uint64_t gmask = L == 64u ? ~0ull : ((1ull << L) - 1ull) << base;
                 vis_sum += (float)__popcll(__ballot(leaf >= 0 && V > 0.0f) & gmask);
                 // the group's closest hit, the first sample of least t (an exchange over lane ^ m
                 // stays inside the aligned group of L lanes); an earlier round wins ties
-                float rt = leaf >= 0 ? t : INFINITY;
-                int rl = leaf;
-                uint32_t rs = s;
-                for (uint32_t m = L >> 1; m > 0; m >>= 1) {
-                    const float ot = __shfl_xor(rt, (int)m, 64);
-                    const int ol = __shfl_xor(rl, (int)m, 64);
-                    const uint32_t os = __shfl_xor(rs, (int)m, 64);
-                    if (ot < rt || (ot == rt && os < rs)) {
-                        rt = ot;
-                        rl = ol;
-                        rs = os;
-                    }
-                }
-                if (rl >= 0 && rt < best_t) {
+                const float ht = leaf >= 0 ? t : INFINITY;
+                float rt = ht;
+                for (uint32_t m = L >> 1; m > 0; m >>= 1) rt = fminf(rt, __shfl_xor(rt, (int)m, 64));
+                if (rt < best_t) {
                     best_t = rt;
-                    best_leaf = rl;
+                    best_leaf = __shfl(leaf, __ffsll((unsigned long long)(__ballot(ht == rt) & gmask)) - 1, 64);
                 }
-                // colours are summed in sample order by the group's first lane (the one that
-                // writes the pixel), through the first two stack rows of the wavefront's lanes (no
-                // ray is under way here)
-                int2* wcol = lds_stack + (threadIdx.x - lane);
-                wcol[lane] = make_int2(__float_as_int(sc.x), __float_as_int(sc.y));
-                wcol[TB + lane] = make_int2(__float_as_int(sc.z), __float_as_int(sc.w));
+                // colours are summed in sample order, a component per lane, through the first two
+                // stack rows of the wavefront's lanes (no ray is under way here)
+                float* wxy = reinterpret_cast<float*>(lds_stack + (threadIdx.x - lane));
+                float* wzw = reinterpret_cast<float*>(lds_stack + TB + (threadIdx.x - lane));
+                wxy[lane] = sc.x;
+                wxy[64 + lane] = sc.y;
+                wzw[lane] = sc.z;
+                wzw[64 + lane] = sc.w;
                 __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
                 __builtin_amdgcn_wave_barrier();
-                if (sl == 0) {
-                    for (uint32_t i = 0; i < L; ++i) {
-                        const int2 c = wcol[base + i], d = wcol[TB + base + i];
-                        col.x += __int_as_float(c.x);
-                        col.y += __int_as_float(c.y);
-                        col.z += __int_as_float(d.x);
-                        col.w += __int_as_float(d.y);
+                if (sl < 4u && L > 2u) {
+                    const float4* w = reinterpret_cast<const float4*>((sl < 2u ? wxy : wzw) + 64 * (sl & 1u) + base);
+                    for (uint32_t i = 0; i < L / 4; ++i) {
+                        const float4 v = w[i];
+                        acc = acc + v.x + v.y + v.z + v.w;
                     }
                 }
                 __builtin_amdgcn_wave_barrier();
                 __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-                if (rd == 0) {  // features of sample 0
-                    const int src = (int)base;
-                    const int l0 = __shfl(leaf, src, 64);
-                    const float a0 = __shfl(alb.x, src, 64), a1 = __shfl(alb.y, src, 64), a2 = __shfl(alb.z, src, 64);
-                    const float n0 = __shfl(N.x, src, 64), n1 = __shfl(N.y, src, 64), n2 = __shfl(N.z, src, 64);
-                    const float t0s = __shfl(t, src, 64);
-                    if (l0 >= 0) {
-                        aux[0] = a0; aux[1] = a1; aux[2] = a2;
-                        aux[3] = n0; aux[4] = n1; aux[5] = n2;
-                        aux[6] = t0s;
-                    }
-                }
             }
+            const uint32_t opix = (py - f.win_y0) * f.win_w + (px - f.win_x0);
+            float4 col;
+            if (L == 2u)  // (0 + sample 0 + sample 1, without the rows)
+                col = make_float4(0.0f + sc.x + __shfl(sc.x, (int)base + 1, 64), 0.0f + sc.y + __shfl(sc.y, (int)base + 1, 64),
+                                  0.0f + sc.z + __shfl(sc.z, (int)base + 1, 64), 0.0f + sc.w + __shfl(sc.w, (int)base + 1, 64));
+            else
+                col = make_float4(acc, __shfl(acc, (int)base + 1, 64), __shfl(acc, (int)base + 2, 64),
+                                  __shfl(acc, (int)base + 3, 64));
             if (valid && sl == 0) {
-                const uint32_t opix = (py - f.win_y0) * f.win_w + (px - f.win_x0);
-                write_pixel(A, opix, col, best_t < INFINITY ? best_t : FLT_MAX, best_t, best_leaf, aux, vis_sum);
+                write_pixel_main(A, opix, col, best_t < INFINITY ? best_t : FLT_MAX, best_t, best_leaf);
+                write_aux_tail(A, opix, t0, vis_sum);
             }
         }
     }
@@ -1446,9 +1453,11 @@ uint32_t tile_log2(int64_t tw) {
 
 namespace {
 // Units of work the sample-lanes kernel wants per wavefront. 64-spp AO of 50M spheres at 1080p: 18.4 ms
-// in whole tiles, 15.4, 14.4, 13.8 and 13.8 ms at 4, 8, 16 and 32 (16 spp of 3M spheres at 1000x621:
-// 1.97 ms, then 1.38, 1.35, 1.42, 1.43): the last tiles of 64 passes each ran on an idle device.
-constexpr uint64_t SUB_UNITS = 16;
+// in whole tiles, 15.4, 14.4, 13.8 and 13.8 ms at 4, 8, 16 and 32: the last tiles of 64 passes each ran
+// on an idle device. Units of fewer than four passes only up to FEW_UNITS: a unit's random streams are
+// set up together (16 spp of 3M spheres at 1000x621: 1.42 ms at one pass per unit, 1.34 at four; 800x600
+// at 8 spp, 1M spheres: 0.72 ms so, 0.78 and 0.90 with FEW_UNITS 2 and 1).
+constexpr uint64_t SUB_UNITS = 16, FEW_UNITS = 4;
 
 // Kernel choice for one frame (the same for both entry points): sample-parallel lanes for Lambert
 // and AO with spp a power of two up to 64 or a multiple of 64, the ballot-refill kernel when a
@@ -1463,10 +1472,10 @@ void dispatch_trace(mmhrt_ctx_s* c, TraceArgs& A, unsigned grid, bool count) {
     const bool sl_shape = fc.spp > 1 && ((fc.spp >= 64 && fc.spp % 64 == 0) || (fc.spp < 64 && 64 % fc.spp == 0));
     const bool sl = c->opt_sample_lanes != 0 && fc.mode != 2 && sl_shape && (c->accel == 1 || refill == 0);
     // the sample-lanes kernel divides its tiles (min(spp, 64) passes each) until every wavefront
-    // of the full grid has SUB_UNITS units, and no launch has more wavefronts than units
+    // of the full grid has its units, and no launch has more wavefronts than units
     if (sl)
-        while ((1u << A.sub_log2) < std::min(fc.spp, 64u) &&
-               ((uint64_t)A.n_tiles << A.sub_log2) < SUB_UNITS * grid * (TB / 64))
+        for (uint32_t p = std::min(fc.spp, 64u);
+             p > 1 && ((uint64_t)A.n_tiles << A.sub_log2) < (p > 4 ? SUB_UNITS : FEW_UNITS) * grid * (TB / 64); p >>= 1)
             ++A.sub_log2;
     const uint64_t need = (((uint64_t)A.n_tiles << A.sub_log2) + TB / 64 - 1) / (TB / 64);
     const Grid g{(unsigned)std::min<uint64_t>(grid, need), (unsigned)c->cu_count, c->stream};

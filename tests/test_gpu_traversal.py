@@ -96,3 +96,36 @@ def test_work_queues(gpu_renderer, w, h, blocks):
                       refill=refill)
     finally:
         gpu_renderer.set_option("blocks_per_cu", 8)
+
+
+@pytest.mark.parametrize("spp", [2, 4, 16, 64, 192])
+@pytest.mark.parametrize("window", [None, (3, 5, 13, 11)])
+def test_passes_without_a_hit(gpu_renderer, spp, window):
+    """A few spheres on a wide background: whole passes that miss (they end early where a pass is the
+    pixel) next to pixels hit by some of their samples, over two accumulated frames and with the window
+    at an odd offset, against the lane-per-pixel kernels bit for bit."""
+    r = gpu_renderer
+    xyzr, rgba = scenes.random_spheres(40, seed=41, rmin=0.01, rmax=0.06)
+    w, h = 29, 23
+    cam = look_at((0.5, 0.5, 2.5), (0.5, 0.5, 0.5), (0, 1, 0), 50.0, w / h, 0.1, 10.0)
+    frames = {}
+    try:
+        r.set_spheres(xyzr, rgba)
+        r.build(L.BUILD_REBUILD, 30)
+        for lanes in (1, 0):
+            r.set_option("sample_lanes", lanes)
+            for k in range(2):
+                case(f"missed passes spp {spp} window {window} lanes {lanes} frame {k}")
+                p = params(w, h, spp=spp, mode=L.MODE_AO, ao_distance=0.3, frame_idx=k, accumulate=1,
+                           background=(0.2, 0.3, 0.4, 0.5), flags=L.FLAG_AUX)
+                if window:
+                    p.window[:] = window
+                frames[lanes, k] = r.render(cam, p)
+    finally:
+        r.set_option("sample_lanes", 1)
+    for k in range(2):
+        a, b = frames[1, k], frames[0, k]
+        hit = b.hit_id >= 0
+        assert 0 < hit.sum() < 0.5 * hit.size
+        assert_frames_equal(a, {n: getattr(b, n) for n in ("hit_id", "t", "depth", "color", "rgba8", "aux")}, aux=True,
+                            what=f"missed passes spp {spp} window {window} frame {k}")
