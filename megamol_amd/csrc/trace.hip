@@ -333,15 +333,67 @@ __device__ __forceinline__ void inner_phase(const TraceArgs& A, const RayPre& r,
     }
 }
 
-// Closest hit: returns the leaf index of the nearest reported intersection (or -1) and its t.
+// Node and sphere words read at a wavefront-uniform address: through the constant address space, so
+// that they arrive in scalar registers (the structure is written by earlier kernels only).
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+typedef const __attribute__((address_space(4))) f32x4* const_f32x4;
+typedef const __attribute__((address_space(4))) i32x4* const_i32x4;
+
+// The start of a walk whose rays begin alike, as the primary rays of a tile and the AO rays of a pixel
+// do: the wavefront goes down from the root together, by scalar loads, while at least 3/4 of its lanes
+// meet the child that most of them meet first, and pushes the other child with each lane's own entry
+// distance (infinite where the lane misses it). From the first node that is left with fewer lanes, that
+// is over a leaf, or where the LDS part of the stack is nearly full, each lane goes on by itself. At 1
+// sample 60M clustered spheres at 4K take 5.45 -> 5.25 ms, at 64 samples with AO 50M FCC spheres 12.8 ->
+// 12.2 ms (all lanes, half or 3/4 of them: the same within 0.5 %). Not for a path's bounces, which
+// part at once: 16 passes over 1M spheres took 10 % longer with it.
 template <int S, bool COUNT>
+__device__ __forceinline__ void descend_together(const TraceArgs& A, const RayPre& r, float tmin, float t_best,
+                                                 int32_t& node, int32_t& leaf, LaneStack<S>& st, Count& cnt) {
+    int32_t u = 0;
+    const int keep = max(1, (int)__popcll(__ballot(true)) * 3 / 4);
+    int sp = 1;
+    for (;;) {
+        const_f32x4 q = (const_f32x4)(uintptr_t)(A.nodes + u);
+        const f32x4 a = q[0], b = q[1], c = q[2];
+        const i32x4 d = *(const_i32x4)(q + 3);
+        if (COUNT) cnt.visits++;
+        const float tn0 = slab(r, a.x, a.y, a.z, a.w, b.x, b.y, tmin, t_best);
+        const float tn1 = slab(r, b.z, b.w, c.x, c.y, c.z, c.w, tmin, t_best);
+        const bool first0 = tn0 <= tn1;
+        const uint64_t m0 = __ballot(tn0 != INFINITY), m1 = __ballot(tn1 != INFINITY);
+        const bool pick0 = 2 * __popcll(__ballot(first0) & (m0 | m1)) >= __popcll(m0 | m1);
+        const int32_t ch = pick0 ? d.x : d.y;
+        if (ch < 0 || sp >= LaneStack<S>::N - 2 || (int)__popcll(pick0 ? m0 : m1) < keep) {
+            const float tnear = first0 ? tn0 : tn1, tfar = first0 ? tn1 : tn0;
+            node = first0 ? d.x : d.y;
+            st.sp = sp;
+            st.push(tfar != INFINITY, first0 ? d.y : d.x, tfar);
+            const bool none = tnear == INFINITY;
+            const bool put = !none && node < 0;
+            if (put) leaf = node;
+            st.pop(none || put, t_best, node, leaf);
+            return;
+        }
+        if (pick0 ? m1 : m0) {
+            st.lds[sp * TB] = (i32x2){pick0 ? d.y : d.x, __float_as_int(pick0 ? tn1 : tn0)};
+            ++sp;
+        }
+        u = ch;
+    }
+}
+
+// Closest hit: returns the leaf index of the nearest reported intersection (or -1) and its t.
+template <int S, bool COUNT, bool TOG>
 __device__ int trace_closest(const TraceArgs& A, const RayPre& r, float tmin, float tmax, float& t_best,
                              LaneStack<S>& st, Count& cnt) {
     int best = -1;
     t_best = tmax;
     int32_t node = 0, leaf = REF_NONE;
     st.reset();
-    while (node != REF_NONE) {
+    if (TOG) descend_together<S, COUNT>(A, r, tmin, t_best, node, leaf, st, cnt);
+    while (node != REF_NONE || leaf != REF_NONE) {
         inner_phase<S, COUNT>(A, r, tmin, t_best, node, leaf, st, cnt);
         while (leaf != REF_NONE) {
             test_leaf<COUNT>(A, r, tmin, tmax, leaf, -1, false, t_best, best, cnt);
@@ -361,7 +413,8 @@ __device__ bool trace_any(const TraceArgs& A, const RayPre& r, float tmin, float
     st.reset();
     float tb = tmax;
     int best = -1;
-    while (node != REF_NONE) {
+    descend_together<S, COUNT>(A, r, tmin, tmax, node, leaf, st, cnt);
+    while (node != REF_NONE || leaf != REF_NONE) {
         inner_phase<S, COUNT>(A, r, tmin, tmax, node, leaf, st, cnt);
         while (leaf != REF_NONE) {
             if (test_leaf<COUNT>(A, r, tmin, tmax, leaf, skip, true, tb, best, cnt)) return true;
@@ -372,13 +425,6 @@ __device__ bool trace_any(const TraceArgs& A, const RayPre& r, float tmin, float
     }
     return false;
 }
-
-// Node and sphere words read at a wavefront-uniform address: through the constant address space, so
-// that they arrive in scalar registers (the structure is written by earlier kernels only).
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef int i32x4 __attribute__((ext_vector_type(4)));
-typedef const __attribute__((address_space(4))) f32x4* const_f32x4;
-typedef const __attribute__((address_space(4))) i32x4* const_i32x4;
 
 // Closest hit of a whole wavefront whose rays lie in one octant of directions, as the samples of a
 // pixel do: all lanes walk the same nodes together (a node is visited while any lane's ray meets
@@ -477,7 +523,7 @@ __device__ __forceinline__ int trace_closest_group(const TraceArgs& A, const Ray
     const uint64_t bx = __ballot(r.inv.x < 0.0f), by = __ballot(r.inv.y < 0.0f), bz = __ballot(r.inv.z < 0.0f);
     if ((bx == 0 || bx == act) && (by == 0 || by == act) && (bz == 0 || bz == act))
         return trace_closest_packet<S, COUNT>(A, r, tmin, tmax, bx != 0, by != 0, bz != 0, t_best, st, cnt);
-    return trace_closest<S, COUNT>(A, r, tmin, tmax, t_best, st, cnt);
+    return trace_closest<S, COUNT, true>(A, r, tmin, tmax, t_best, st, cnt);
 }
 
 // Slab test of one child box returning the entry distance (+inf when missed) and the exit.
@@ -638,11 +684,12 @@ __device__ int trace_tl(const TraceArgs& A, const RayPre& r, float tmin, float t
 }
 
 // The structure a kernel traverses: TL = treelet P-k-d trees, else the LBVH.
-template <int S, bool COUNT, bool TL>
+// TOG: the active lanes' rays are coherent (primary rays).
+template <int S, bool COUNT, bool TL, bool TOG>
 __device__ __forceinline__ int trace_closest_x(const TraceArgs& A, const RayPre& r, float tmin, float tmax,
                                                float& t_best, LaneStack<S>& st, Count& cnt) {
     if (TL) return trace_tl<S, COUNT, false>(A, r, tmin, tmax, -1, t_best, st, cnt);
-    return trace_closest<S, COUNT>(A, r, tmin, tmax, t_best, st, cnt);
+    return trace_closest<S, COUNT, TOG>(A, r, tmin, tmax, t_best, st, cnt);
 }
 template <int S, bool COUNT, bool TL>
 __device__ __forceinline__ bool trace_any_x(const TraceArgs& A, const RayPre& r, float tmin, float tmax, int skip,
@@ -749,7 +796,7 @@ __device__ void shade_pixel(const TraceArgs& A, uint32_t px, uint32_t py, float 
         RayPre r = prep(o, d, pad);
         float t;
         if (COUNT) cnt.rays++;
-        int leaf = trace_closest_x<S, COUNT, TL>(A, r, 1e-6f, 1e20f, t, st, cnt);
+        int leaf = trace_closest_x<S, COUNT, TL, true>(A, r, 1e-6f, 1e20f, t, st, cnt);
         float4 sc;
         float ray_depth = FLT_MAX;
         if (leaf < 0) {
@@ -793,7 +840,7 @@ __device__ void shade_pixel(const TraceArgs& A, uint32_t px, uint32_t py, float 
                     RayPre rb = prep(so, sd, pad);
                     float tb;
                     if (COUNT) cnt.rays++;
-                    int lb = trace_closest_x<S, COUNT, TL>(A, rb, 1e-3f, 1e8f, tb, st, cnt);
+                    int lb = trace_closest_x<S, COUNT, TL, false>(A, rb, 1e-3f, 1e8f, tb, st, cnt);
                     if (lb < 0) {
                         res = make_float4(cc.x * 0.8f, cc.y * 0.8f, cc.z * 0.8f, 1.0f);
                         break;
@@ -885,7 +932,7 @@ __device__ __forceinline__ void shade_sample(const TraceArgs& A, uint32_t px, ui
     RayPre r = prep(o, d, pad);
     if (COUNT) cnt.rays++;
     if (TL)
-        leaf = trace_closest_x<S, COUNT, TL>(A, r, 1e-6f, 1e20f, t, st, cnt);
+        leaf = trace_closest_x<S, COUNT, TL, true>(A, r, 1e-6f, 1e20f, t, st, cnt);
     else
         leaf = trace_closest_group<S, COUNT>(A, r, 1e-6f, 1e20f, t, st, cnt);
     ray_depth = FLT_MAX;
