@@ -549,12 +549,15 @@ __device__ __forceinline__ float slab_io(const RayPre& r, float lx, float ly, fl
 // its entry distance and resumes with t1 = the best hit at the time it is popped. A treelet is
 // entered at its root over its box's [entry, exit].
 // The lowest three levels of a treelet are not walked: at a node whose great-grandchildren are past the
-// treelet's end the up to 7 spheres of its subtree are fetched together and tested against their own
-// boxes. Most of the visits were there, each a sphere and a split axis behind the one before. As in the
-// LBVH's two phases, a wavefront's lanes visit top nodes until at most 3/8 of them still do, then P-k-d
-// nodes. 8M clustered spheres at 1280x720, 1-spp AO: 8.1 ms walked to the leaves, 7.3 with the lowest two
-// levels together, 6.6 with three (bound by the latency of dependent fetches: vector ALU 40 % and address
-// unit 50 % busy); at 4, 5, 6 and 7 wavefronts per SIMD 7.0, 6.6, 7.4 and 8.1 (from 6 on it spills).
+// treelet's end the up to 7 spheres of its subtree are fetched together and pass the first part of the
+// sphere test (up to its square root) together; the rest runs for the few that pass. Most of the visits
+// were there, each a sphere and a split axis behind the one before. As in the LBVH's two phases, a
+// wavefront's lanes visit top nodes, then P-k-d nodes, then subtrees, each until at most 3/8 of the lanes
+// that began still do: with the two kinds of P-k-d visit in one loop nearly each iteration ran both for
+// part of the lanes. 8M clustered spheres at 1280x720, 1-spp AO: 8.1 ms walked to the leaves, 7.3 with
+// the lowest two levels together, 6.3 with three, 5.2 with the visits in phases (5.6, 5.2 and 5.3 at 1/8,
+// 3/8 and 5/8). At 4, 5, 6 and 7 wavefronts per SIMD 5.5, 5.2, 5.4 and 6.7 (from 6 on it spills). Bound by
+// the latency of dependent fetches: the tiles along a line of clusters take nearly the kernel's time.
 // Closest hit (ANY false): returns the position of the hit (or -1) and its t in t_best. ANY:
 // returns 1 at the first hit of a sphere other than position `skip`, else 0.
 template <int S, bool COUNT, bool ANY>
@@ -565,7 +568,7 @@ __device__ int trace_tl(const TraceArgs& A, const RayPre& r, float tmin, float t
     st.reset();
     int32_t node = 0;
     float t0 = 0.0f, t1 = 0.0f;
-    uint32_t cur_tl = 0xffffffffu, m = 0;
+    uint32_t cur_tl = 0xffffffffu;
     float rmax = 0.0f;
     const uint32_t lg = A.tl_log2;
     const uint32_t msk = (1u << lg) - 1u;
@@ -577,6 +580,11 @@ __device__ int trace_tl(const TraceArgs& A, const RayPre& r, float tmin, float t
         node = e.x;
         t0 = __int_as_float(e.y);
         t1 = t_best;
+    };
+    // whether ref is a P-k-d node above the lowest three levels of its treelet
+    auto inner = [&](int32_t ref) -> bool {
+        const uint32_t i = ~(uint32_t)ref & msk, bs = ~(uint32_t)ref - i;
+        return ref < 0 && ref != REF_NONE && 8 * i + 7 < min(A.n_sph - bs, msk + 1u);
     };
     // a sphere against its own box (centre -+ radius: the leaf box an LBVH traversal tests before
     // its sphere; a filter that changes no result, most spheres near the ray lie off it), then exactly
@@ -622,62 +630,78 @@ __device__ int trace_tl(const TraceArgs& A, const RayPre& r, float tmin, float t
             }
             if ((int)__popcll(__ballot(node >= 0)) <= few_top) break;
         }
-        const int few_tl = (int)__popcll(__ballot(node < 0 && node != REF_NONE)) * 3 / 8;
-        while (node < 0 && node != REF_NONE) {
+        // P-k-d nodes down to the lowest three levels
+        const int few_in = (int)__popcll(__ballot(inner(node))) * 3 / 8;
+        while (inner(node)) {
             const uint32_t p = ~(uint32_t)node;
             const uint32_t tl = p >> lg;
             if (tl != cur_tl) {
                 cur_tl = tl;
                 rmax = A.tl_rmax[tl];
-                const uint32_t tb = tl << lg;
-                m = A.n_sph - tb < msk + 1u ? A.n_sph - tb : msk + 1u;
             }
             const uint32_t i = p & msk, bs = p - i;
             const float4 sp = A.leaf_sph[p];
-            if (8 * i + 7 >= m) {
-                // (a place past the end repeats the node)
-                float4 g[6];
-                uint32_t pg[6];
-#pragma unroll
-                for (uint32_t k = 0; k < 6; ++k) {
-                    const uint32_t c = k < 2 ? 2 * i + 1 + k : 4 * i + 1 + k;
-                    pg[k] = c < m ? bs + c : p;
-                    g[k] = A.leaf_sph[pg[k]];
-                }
-                if (COUNT) cnt.visits += 7;
-                bool hit = test(p, sp);
-#pragma unroll
-                for (uint32_t k = 0; k < 6; ++k) hit = hit || test(pg[k], g[k]);
-                if (ANY && hit) return 1;
-                pop();
+            const int dd = A.pkd_dim[p];
+            if (COUNT) cnt.visits++;
+            const float sc = dd == 0 ? sp.x : (dd == 1 ? sp.y : sp.z);
+            const float inv = dd == 0 ? r.inv.x : (dd == 1 ? r.inv.y : r.inv.z);
+            const float oil = dd == 0 ? r.oil.x : (dd == 1 ? r.oil.y : r.oil.z);
+            const float oih = dd == 0 ? r.oih.x : (dd == 1 ? r.oih.y : r.oih.z);
+            const float tlo = __builtin_fmaf(sc - rmax, inv, -oil), thi = __builtin_fmaf(sc + rmax, inv, -oih);
+            const float tnr = fminf(tlo, thi), tfr = fmaxf(tlo, thi);
+            if (fmaxf(t0, tnr) <= fminf(tfr, fminf(t1, t_best)) && test(p, sp)) return 1;  // (true only for ANY)
+            const float lim = fminf(t1, t_best);
+            const float n_t1 = fminf(tfr, lim), f_t0 = fmaxf(t0, tnr);
+            const uint32_t sg = inv < 0.0f ? 1u : 0u;
+            const uint32_t nc = 2 * i + 1 + sg, fc = 2 * i + 2 - sg;  // both lie inside the treelet here
+            const bool need_n = t0 <= n_t1, need_f = f_t0 <= lim;
+            if (need_n) {
+                st.push(need_f, ~(int32_t)(bs + fc), f_t0);
+                node = ~(int32_t)(bs + nc);
+                t1 = n_t1;
+            } else if (need_f) {
+                node = ~(int32_t)(bs + fc);
+                t0 = f_t0;
+                t1 = lim;
             } else {
-                const int dd = A.pkd_dim[p];
-                if (COUNT) cnt.visits++;
-                const float sc = dd == 0 ? sp.x : (dd == 1 ? sp.y : sp.z);
-                const float inv = dd == 0 ? r.inv.x : (dd == 1 ? r.inv.y : r.inv.z);
-                const float oil = dd == 0 ? r.oil.x : (dd == 1 ? r.oil.y : r.oil.z);
-                const float oih = dd == 0 ? r.oih.x : (dd == 1 ? r.oih.y : r.oih.z);
-                const float tlo = __builtin_fmaf(sc - rmax, inv, -oil), thi = __builtin_fmaf(sc + rmax, inv, -oih);
-                const float tnr = fminf(tlo, thi), tfr = fmaxf(tlo, thi);
-                if (fmaxf(t0, tnr) <= fminf(tfr, fminf(t1, t_best)) && test(p, sp)) return 1;  // (true only for ANY)
-                const float lim = fminf(t1, t_best);
-                const float n_t1 = fminf(tfr, lim), f_t0 = fmaxf(t0, tnr);
-                const uint32_t sg = inv < 0.0f ? 1u : 0u;
-                const uint32_t nc = 2 * i + 1 + sg, fc = 2 * i + 2 - sg;  // both lie inside the treelet here
-                const bool need_n = t0 <= n_t1, need_f = f_t0 <= lim;
-                if (need_n) {
-                    st.push(need_f, ~(int32_t)(bs + fc), f_t0);
-                    node = ~(int32_t)(bs + nc);
-                    t1 = n_t1;
-                } else if (need_f) {
-                    node = ~(int32_t)(bs + fc);
-                    t0 = f_t0;
-                    t1 = lim;
-                } else {
-                    pop();
-                }
+                pop();
             }
-            if ((int)__popcll(__ballot(node < 0 && node != REF_NONE)) <= few_tl) break;
+            if ((int)__popcll(__ballot(inner(node))) <= few_in) break;
+        }
+        // the subtrees of the lowest three levels
+        const int few_g = (int)__popcll(__ballot(node < 0 && node != REF_NONE && !inner(node))) * 3 / 8;
+        while (node < 0 && node != REF_NONE && !inner(node)) {
+            const uint32_t p = ~(uint32_t)node;
+            const uint32_t i = p & msk, bs = p - i, m = min(A.n_sph - bs, msk + 1u);
+            const float4 sp = A.leaf_sph[p];
+            // the part of the sphere test before the square root for all seven (a place past the end
+            // repeats the node), the rest for the few that pass
+            float4 g[6];
+#pragma unroll
+            for (uint32_t k = 0; k < 6; ++k) {
+                const uint32_t c = k < 2 ? 2 * i + 1 + k : 4 * i + 1 + k;
+                g[k] = A.leaf_sph[c < m ? bs + c : p];
+            }
+            if (COUNT) cnt.visits += 7;
+            uint32_t near = 0;
+#pragma unroll
+            for (uint32_t k = 0; k < 7; ++k) {
+                V3 oc;
+                float b_, e_;
+                near |= sphere_near(r, k < 6 ? g[k] : sp, oc, b_, e_) ? 1u << k : 0u;
+            }
+            bool hit = false;
+            while (near) {
+                const uint32_t k = __ffs(near) - 1;
+                near &= near - 1;
+                const uint32_t c = k < 2 ? 2 * i + 1 + k : (k < 6 ? 4 * i + 1 + k : i);
+                const uint32_t pc = c < m ? bs + c : p;
+                hit = test(pc, A.leaf_sph[pc]);
+                if (hit) break;
+            }
+            if (ANY && hit) return 1;
+            pop();
+            if ((int)__popcll(__ballot(node < 0 && node != REF_NONE && !inner(node))) <= few_g) break;
         }
     }
     return ANY ? 0 : best;
