@@ -259,7 +259,7 @@ int32_t mmhrt_destroy(mmhrt_ctx c) {
     release(c->leaf_sph); release(c->leaf_id); release(c->nodes); release(c->flags); release(c->flags2); release(c->box_cnt);
     release(c->partial); release(c->info); release(c->tf_buf);
     release(c->fb_col); release(c->fb_depth); release(c->fb_t); release(c->fb_id); release(c->fb_rgba8);
-    release(c->fb_aux); release(c->spill); release(c->counters);
+    release(c->fb_aux); release(c->spill); release(c->counters); release(c->tile_order);
     release(c->ts_sph); release(c->ts_col); release(c->bt_col); release(c->bt_depth); release(c->bt_t);
     release(c->bt_id); release(c->bt_rgba8); release(c->batch_ctr); release(c->batch_prefix);
     release(c->batch_jobs);

@@ -133,6 +133,7 @@ struct mmhrt_ctx_s {
     mmhrt::DevBuf<uint32_t> fb_rgba8;
     mmhrt::DevBuf<__half> fb_aux;
     mmhrt::DevBuf<int32_t> spill;
+    mmhrt::DevBuf<uint32_t> tile_order;  // treelet frames: cost and order of the tiles
     mmhrt::DevBuf<uint32_t> counters;  // TRACE_CTR_WORDS: overflow flag, visit counters (u64 pairs), work queues
 
     // options
@@ -284,7 +285,7 @@ struct FrameOutputs {
 };
 int render_frame(mmhrt_ctx_s* c, const FrameConsts& fc);
 int render_frame_into(mmhrt_ctx_s* c, const FrameConsts& fc, const FrameOutputs& out, uint32_t* ctr, int32_t* spill,
-                      uint32_t lanes, bool count);
+                      uint32_t lanes, bool count, uint32_t* order = nullptr);
 uint32_t tile_log2(int64_t tw);
 
 // noalloc.hip
