@@ -228,8 +228,7 @@ int32_t mmhrt_create(int32_t device, mmhrt_ctx* out) {
     }
     hipDeviceGetAttribute(&c->cu_count, hipDeviceAttributeMultiprocessorCount, device);
     if (c->cu_count <= 0) c->cu_count = 1;
-    size_t mem_free = 0;
-    if (hipMemGetInfo(&mem_free, &c->mem_total) != hipSuccess) (void)hipGetLastError();
+    if (hipDeviceTotalMem(&c->mem_total, device) != hipSuccess) (void)hipGetLastError();
     for (int i = 0; i < 12; ++i) hipEventCreate(&c->tm.ev[i]);
     c->tm.init = true;
     // the device address of this device's scratch array for mmhrt_render_noalloc; on failure that
