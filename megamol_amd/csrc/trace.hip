@@ -213,7 +213,10 @@ __device__ __forceinline__ RayPre prep(V3 o, V3 d, float pad) {
     return r;
 }
 
-// Slab test of one child box (lo, hi); returns the entry distance, or +inf when missed.
+// Slab test of one child box (lo, hi); returns the entry distance, or +inf when missed. Minima and maxima
+// issue at half the rate of multiply-adds (0.57e12 against 1.05e12 wavefront instructions/s over the device)
+// and take two thirds of it, but selects do too: the planes picked by the signs of the direction, lane by
+// lane, made 64 samples with AO over 50M spheres 2.5 % slower.
 __device__ __forceinline__ float slab(const RayPre& r, float lx, float ly, float lz, float hx, float hy, float hz,
                                       float tmin, float tmax) {
     float x0 = __builtin_fmaf(lx, r.inv.x, -r.oil.x), x1 = __builtin_fmaf(hx, r.inv.x, -r.oih.x);
@@ -1282,7 +1285,7 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(5, 8))) void
                     r = prep(Pp, ad, pad);
                     tmin = 0.0f;
                     tmax = f.ao_distance;
-                    t_best = tmax;  // an any-hit ray's bound in step_mixed
+                    t_best = tmax;  // an any-hit ray's bound
                     skip = best;
                     best = -1;
                     node = 0;
