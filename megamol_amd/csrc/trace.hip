@@ -919,8 +919,13 @@ __device__ void shade_pixel(const TraceArgs& A, uint32_t px, uint32_t py, float 
 // beats the refill kernel, which had been the default there (50M spheres, 1080p AO: 0.88 against 0.70
 // ms; 60M clustered at 4K: 6.7 against 5.7; 10k spheres at 320x240: 92 against 80 us): bound by the
 // vector memory unit's address rate (busy 60-90 %), then by VALU issue (50-70 %).
-template <int S, int MODE, bool COUNT, bool STEAL, bool TL = false>
-__global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(TL ? 5 : 7, 8))) void k_trace(TraceArgs A) {
+// Small frames (W = 5) are held to 102 VGPRs, without spills: their wavefronts have one or two tiles
+// each and the longest rays are the kernel's time. One sample, 1.5 tiles per wavefront (816x600), scenes
+// of 100k, 1M, 4M spheres: AO 238, 282, 310 -> 210, 255, 295 us, Lambert 189, 229, 266 -> 173, 198, 230 and
+// 4 bounces 0.51, 0.52, 0.56 -> 0.45, 0.48, 0.54 ms (640x480 0 to 12 % off, 320x240 the same); at 2.1 tiles
+// (960x720) 4 and 8 bounces take 5 to 22 % longer, at 1280x720 a Lambert frame 4 %.
+template <int S, int MODE, bool COUNT, bool STEAL, bool TL = false, int W = TL ? 5 : 7>
+__global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(W, 8))) void k_trace(TraceArgs A) {
     __shared__ int2 lds_stack[LaneStack<S>::N * TB];
     const uint32_t gtid = blockIdx.x * TB + threadIdx.x;
     LaneStack<S> st(lds_stack + threadIdx.x, A.spill + gtid, A.spill_stride, A.ctr + 1);
@@ -1356,6 +1361,8 @@ template <int S, int MODE>
 void launch2(const TraceArgs& A, const Grid& g, bool steal, bool count) {
     if (count)
         launch3<S, MODE, true>(A, g, steal);
+    else if (steal && A.fc.spp == 1 && A.n_tiles <= 30 * g.cus)  // 1.5 for each of 20 wavefronts per CU
+        launch_resident<k_trace<S, MODE, false, true, false, 5>>(g, A);
     else
         launch3<S, MODE, false>(A, g, steal);
 }

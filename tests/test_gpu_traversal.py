@@ -129,3 +129,22 @@ def test_passes_without_a_hit(gpu_renderer, spp, window):
         assert 0 < hit.sum() < 0.5 * hit.size
         assert_frames_equal(a, {n: getattr(b, n) for n in ("hit_id", "t", "depth", "color", "rgba8", "aux")}, aux=True,
                             what=f"missed passes spp {spp} window {window} frame {k}")
+
+
+@pytest.mark.parametrize("mode,bounces", [(L.MODE_LAMBERT, 0), (L.MODE_AO, 0), (L.MODE_BOUNCE, 1), (L.MODE_BOUNCE, 4)])
+def test_frames_about_the_small_size(gpu_renderer, mode, bounces):
+    """One sample: a small frame against the oracle, and a frame one tile row above 7680 tiles of 8x8
+    against a window of exactly that many."""
+    r = gpu_renderer
+    xyzr, rgba = scenes.random_spheres(3000, seed=51, rmin=0.01, rmax=0.05)
+    cam = lambda w, h: look_at((0.5, 0.5, 2.2), (0.5, 0.5, 0.5), (0, 1, 0), 40.0, w / h, 0.1, 10.0)
+    p = params(61, 47, mode=mode, max_bounces=bounces, ao_distance=0.3)
+    check(r, xyzr, rgba, cam(61, 47), p, f"mode {mode} bounces {bounces} small frame")
+    w, h = 1024, 488
+    case(f"mode {mode} bounces {bounces} {w}x{h} and window")
+    p = params(w, h, mode=mode, max_bounces=bounces, ao_distance=0.3, flags=L.FLAG_AUX)
+    a = r.render(cam(w, h), p)
+    p.window[:] = (0, 0, w, 480)
+    b = r.render(cam(w, h), p)
+    assert_frames_equal(b, {k: getattr(a, k)[:480] for k in ("hit_id", "t", "depth", "color", "rgba8", "aux")}, aux=True,
+                        what=f"mode {mode} bounces {bounces} window")
