@@ -919,7 +919,7 @@ __device__ void shade_pixel(const TraceArgs& A, uint32_t px, uint32_t py, float 
 // beats the refill kernel, which had been the default there (50M spheres, 1080p AO: 0.88 against 0.70
 // ms; 60M clustered at 4K: 6.7 against 5.7; 10k spheres at 320x240: 92 against 80 us): bound by the
 // vector memory unit's address rate (busy 60-90 %), then by VALU issue (50-70 %).
-// Small frames (W = 5) are held to 102 VGPRs, without spills: their wavefronts have one or two tiles
+// Small frames (W = 5) are held to 102 VGPRs, with hardly a spill: their wavefronts have one or two tiles
 // each and the longest rays are the kernel's time. One sample, 1.5 tiles per wavefront (816x600), scenes
 // of 100k, 1M, 4M spheres: AO 238, 282, 310 -> 210, 255, 295 us, Lambert 189, 229, 266 -> 173, 198, 230 and
 // 4 bounces 0.51, 0.52, 0.56 -> 0.45, 0.48, 0.54 ms (640x480 0 to 12 % off, 320x240 the same); at 2.1 tiles
