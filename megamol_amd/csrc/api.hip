@@ -103,6 +103,10 @@ int check_render_args(mmhrt_ctx_s* c, const mmhrt_camera* cam, const mmhrt_rende
     return MMHRT_OK;
 }
 
+int settle(mmhrt_ctx_s* c, int code) {
+    (void)hipStreamSynchronize(c->stream);
+    return code;
+}
 int check_ctx(mmhrt_ctx c) {
     if (!c) return MMHRT_E_INVALID;
     hipError_t e = hipSetDevice(c->device);
@@ -364,7 +368,7 @@ int32_t mmhrt_set_spheres(mmhrt_ctx c, const mmhrt_sphere_list* lists, uint32_t 
         if (L.count == 0 || L.vert_type == MMHRT_VERTDATA_NONE) continue;
         uint8_t* dv = c->staging.p + sp;
         hipError_t he = hipMemcpyAsync(dv, s.hv, s.vbytes, hipMemcpyHostToDevice, c->stream);
-        if (he != hipSuccess) return hip_fail(c, he, "particle upload");
+        if (he != hipSuccess) return settle(c, hip_fail(c, he, "particle upload"));
         sp += (s.vbytes + 255) & ~255ull;
         uint8_t* dc = dv;
         if (L.col_type != MMHRT_COLDATA_NONE) {
@@ -373,7 +377,7 @@ int32_t mmhrt_set_spheres(mmhrt_ctx c, const mmhrt_sphere_list* lists, uint32_t 
             } else {
                 dc = c->staging.p + sp;
                 he = hipMemcpyAsync(dc, s.hc, s.cbytes, hipMemcpyHostToDevice, c->stream);
-                if (he != hipSuccess) return hip_fail(c, he, "colour upload");
+                if (he != hipSuccess) return settle(c, hip_fail(c, he, "colour upload"));
                 sp += (s.cbytes + 255) & ~255ull;
             }
         }
@@ -389,7 +393,7 @@ int32_t mmhrt_set_spheres(mmhrt_ctx c, const mmhrt_sphere_list* lists, uint32_t 
         d.gradius = L.global_radius;
         for (int q = 0; q < 4; ++q) d.gcol[q] = (float)L.global_rgba[q] / 255.0f;  // SphereGeometry.cpp:179-181
         d.use_tf = tf_n > 0 && (L.col_type == MMHRT_COLDATA_FLOAT_I || L.col_type == MMHRT_COLDATA_DOUBLE_I);
-        if ((e = launch_convert_list(c, d, tf_dev, tf_n, tf_vmin, tf_fac))) return e;
+        if ((e = launch_convert_list(c, d, tf_dev, tf_n, tf_vmin, tf_fac))) return settle(c, e);
         off += L.count;
     }
     hipError_t he = hipStreamSynchronize(c->stream);
@@ -491,18 +495,17 @@ int32_t mmhrt_download(mmhrt_ctx c, mmhrt_framebuffer* out) {
     if (!out) return fail(c, MMHRT_E_INVALID, "download: out is NULL");
     if (c->fb_w == 0) return fail(c, MMHRT_E_STATE, "download: nothing rendered yet");
     size_t P = (size_t)c->fb_w * c->fb_h;
+    if (out->aux && (!c->fb_aux.p || c->fb_aux.cap < P * 8))  // before anything is queued
+        return fail(c, MMHRT_E_STATE, "download: no aux buffer rendered");
     hipError_t e = hipSuccess;
     if (out->rgba8 && e == hipSuccess) e = hipMemcpyAsync(out->rgba8, c->fb_rgba8.p, P * 4, hipMemcpyDeviceToHost, c->stream);
     if (out->depth && e == hipSuccess) e = hipMemcpyAsync(out->depth, c->fb_depth.p, P * 4, hipMemcpyDeviceToHost, c->stream);
     if (out->color && e == hipSuccess) e = hipMemcpyAsync(out->color, c->fb_col.p, P * 16, hipMemcpyDeviceToHost, c->stream);
     if (out->t && e == hipSuccess) e = hipMemcpyAsync(out->t, c->fb_t.p, P * 4, hipMemcpyDeviceToHost, c->stream);
     if (out->hit_id && e == hipSuccess) e = hipMemcpyAsync(out->hit_id, c->fb_id.p, P * 4, hipMemcpyDeviceToHost, c->stream);
-    if (out->aux && e == hipSuccess) {
-        if (!c->fb_aux.p || c->fb_aux.cap < P * 8) return fail(c, MMHRT_E_STATE, "download: no aux buffer rendered");
-        e = hipMemcpyAsync(out->aux, c->fb_aux.p, P * 16, hipMemcpyDeviceToHost, c->stream);
-    }
-    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    if (e != hipSuccess) return hip_fail(c, e, "download");
+    if (out->aux && e == hipSuccess) e = hipMemcpyAsync(out->aux, c->fb_aux.p, P * 16, hipMemcpyDeviceToHost, c->stream);
+    if (e != hipSuccess) return settle(c, hip_fail(c, e, "download"));
+    if ((e = hipStreamSynchronize(c->stream)) != hipSuccess) return hip_fail(c, e, "download");
     return MMHRT_OK;
 }
 

@@ -104,7 +104,7 @@ int32_t mmhrt_set_timesteps(mmhrt_ctx c, const float* xyzr, uint32_t timesteps, 
         g = make_float4(global_rgba[0] / 255.0f, global_rgba[1] / 255.0f, global_rgba[2] / 255.0f, global_rgba[3] / 255.0f);
     if (rgba) {
         he = hipMemcpyAsync(c->ts_col.p, rgba, count * 16, hipMemcpyHostToDevice, c->stream);
-        if (he != hipSuccess) return hip_fail(c, he, "set_timesteps colours");
+        if (he != hipSuccess) return settle(c, hip_fail(c, he, "set_timesteps colours"));
     } else {
         launch_fill_f4(c->stream, c->ts_col.p, g, count);
     }
@@ -279,8 +279,8 @@ int32_t mmhrt_render_batch(mmhrt_ctx c, const mmhrt_job* jobs, uint32_t n_jobs, 
     hipError_t he = hipMemcpyAsync(c->batch_jobs.p, hjobs.data(), hjobs.size(), hipMemcpyHostToDevice, c->stream);
     if (he == hipSuccess)
         he = hipMemcpyAsync(c->batch_prefix.p, hprefix.data(), hprefix.size() * 4, hipMemcpyHostToDevice, c->stream);
-    if (he == hipSuccess) he = hipStreamSynchronize(c->stream);
-    if (he != hipSuccess) return hip_fail(c, he, "render_batch upload");
+    if (he != hipSuccess) return settle(c, hip_fail(c, he, "render_batch upload"));
+    if ((he = hipStreamSynchronize(c->stream)) != hipSuccess) return hip_fail(c, he, "render_batch upload");
     auto launch = [&](size_t li) {
         const Launch& L = launches[li];
         launch_trace_batch(c, c->batch_jobs.p + js * L.first, c->batch_prefix.p + L.prefix, L.count,

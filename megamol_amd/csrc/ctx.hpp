@@ -198,6 +198,9 @@ namespace mmhrt {
 // error helper: records message, returns code
 int fail(mmhrt_ctx_s* c, int code, const std::string& msg);
 int hip_fail(mmhrt_ctx_s* c, hipError_t e, const char* what);
+// For an error return after copies from or to the caller's memory were queued: waits for them, since
+// the caller may free or reuse that memory once the call is over. Returns code.
+int settle(mmhrt_ctx_s* c, int code);
 
 // batch.hip: the structures that a series keeps between calls are given back; false if there were none
 // to give (or they are in use)

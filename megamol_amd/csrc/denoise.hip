@@ -1843,9 +1843,10 @@ int32_t mmhrt_denoise_features(mmhrt_ctx c, const uint16_t* feats, uint32_t b, u
     if (int e = mmhrt::ensure(c, d.raw, P * 12, "denoiser features")) return e;
     hipError_t he = hipMemcpyAsync(d.raw.p, feats, P * 24, hipMemcpyHostToDevice, c->stream);
     if (he != hipSuccess) return mmhrt::hip_fail(c, he, "denoise_features upload");
-    if (int e = dn_run(c, (int)b, (int)h, (int)w, depth_scale, bg, nullptr, nullptr, false)) return e;
+    if (int e = dn_run(c, (int)b, (int)h, (int)w, depth_scale, bg, nullptr, nullptr, false)) return mmhrt::settle(c, e);
     he = hipMemcpyAsync(out_color, d.color.p, P * 12, hipMemcpyDeviceToHost, c->stream);
-    if (he == hipSuccess) he = hipStreamSynchronize(c->stream);
+    if (he != hipSuccess) return mmhrt::settle(c, mmhrt::hip_fail(c, he, "denoise_features"));
+    he = hipStreamSynchronize(c->stream);
     return he == hipSuccess ? MMHRT_OK : mmhrt::hip_fail(c, he, "denoise_features");
 }
 
@@ -1862,15 +1863,15 @@ int32_t mmhrt_denoiser_train_step(mmhrt_ctx c, const uint16_t* feats, const floa
     hipStream_t s = c->stream;
     hipError_t he = hipMemcpyAsync(d.raw.p, feats, P * 24, hipMemcpyHostToDevice, s);
     if (he == hipSuccess) he = hipMemcpyAsync(d.target.p, target, P * 12, hipMemcpyHostToDevice, s);
-    if (he != hipSuccess) return mmhrt::hip_fail(c, he, "train_step upload");
+    if (he != hipSuccess) return mmhrt::settle(c, mmhrt::hip_fail(c, he, "train_step upload"));
     if (int e = dn_run(c, (int)b, (int)h, (int)w, depth_scale, bg, d.target.p, loss_out ? d.scalar.p : d.scalar.p, true))
-        return e;
+        return mmhrt::settle(c, e);
     size_t n = mmhrt::dn::param_count();
     mmhrt::dn::zero(s, d.grads.p, (long)n);
     d.backward(s, (int)b, ceil8((int)h), ceil8((int)w));
     if (grads_out) {
         he = hipMemcpyAsync(grads_out, d.grads.p, n * 4, hipMemcpyDeviceToHost, s);
-        if (he != hipSuccess) return mmhrt::hip_fail(c, he, "train_step grads");
+        if (he != hipSuccess) return mmhrt::settle(c, mmhrt::hip_fail(c, he, "train_step grads"));
     }
     if (apply) {
         d.step++;
@@ -1881,7 +1882,7 @@ int32_t mmhrt_denoiser_train_step(mmhrt_ctx c, const uint16_t* feats, const floa
     }
     if (loss_out) {
         he = hipMemcpyAsync(loss_out, d.scalar.p, 4, hipMemcpyDeviceToHost, s);
-        if (he != hipSuccess) return mmhrt::hip_fail(c, he, "train_step loss");
+        if (he != hipSuccess) return mmhrt::settle(c, mmhrt::hip_fail(c, he, "train_step loss"));
     }
     he = hipStreamSynchronize(s);
     return he == hipSuccess ? MMHRT_OK : mmhrt::hip_fail(c, he, "train_step");
