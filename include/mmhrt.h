@@ -228,7 +228,8 @@ MMHRT_API int32_t mmhrt_render_noalloc(mmhrt_ctx ctx, const mmhrt_camera* cam, c
 /* Page-locked host memory for the calls' host outputs, from a pool of the process (freed blocks are
  * kept, up to 256 MB, until the last context is destroyed). A copy into it runs at the link's rate
  * and needs no staging and no page faults. At most 1 GB is handed out at a time (then MMHRT_E_OOM: use
- * ordinary memory). Thread-safe; a block may outlive every context. */
+ * ordinary memory). Thread-safe; a block may outlive every context, and a child of fork() finds the blocks'
+ * contents at their addresses, in memory of its own. */
 MMHRT_API int32_t mmhrt_host_alloc(uint64_t bytes, void** out);
 MMHRT_API int32_t mmhrt_host_free(void* p);
 

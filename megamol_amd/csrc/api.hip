@@ -1,6 +1,8 @@
 // api.hip — the extern "C" boundary declared in include/mmhrt.h.
 #include <math.h>
+#include <pthread.h>
 #include <string.h>
+#include <sys/mman.h>
 
 #include <algorithm>
 #include <map>
@@ -118,16 +120,57 @@ namespace {
 // Page-locked host blocks (mmhrt_host_alloc), in sizes of 4 steps per power of two so that frames of
 // about the same size share them. The pool is never torn down with the process: the runtime may be
 // gone by then.
+// A block is a mapping of the device's file, which a child of fork() does not inherit (a worker that
+// read a frame of its parent's died of it). So a fork copies the blocks in use into ordinary memory, which
+// the child finds at the blocks' own addresses; to the parent they are what they were.
 struct HostPool {
     static constexpr uint64_t KEEP = 256ull << 20, OUT = 1ull << 30;
+    struct Block {
+        uint64_t bytes;
+        void* copy;  // during a fork
+    };
     std::mutex mu;
     std::multimap<uint64_t, void*> idle;
-    std::unordered_map<void*, uint64_t> out;
+    std::unordered_map<void*, Block> out;
     uint64_t idle_bytes = 0, out_bytes = 0;
     int contexts = 0;
+    bool forked = false;  // in a child: the blocks are ordinary memory, and no new ones are handed out
 };
+HostPool& host_pool();
+void before_fork() {
+    HostPool& h = host_pool();
+    h.mu.lock();
+    if (h.forked) return;
+    for (auto& b : h.out) {
+        void* p = mmap(nullptr, b.second.bytes, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS, -1, 0);
+        b.second.copy = p == MAP_FAILED ? nullptr : memcpy(p, b.first, b.second.bytes);
+    }
+}
+void after_fork_parent() {
+    HostPool& h = host_pool();
+    for (auto& b : h.out) {
+        if (b.second.copy) munmap(b.second.copy, b.second.bytes);
+        b.second.copy = nullptr;
+    }
+    h.mu.unlock();
+}
+void after_fork_child() {
+    HostPool& h = host_pool();
+    for (auto& b : h.out) {
+        if (b.second.copy)
+            (void)mremap(b.second.copy, b.second.bytes, b.second.bytes, MREMAP_MAYMOVE | MREMAP_FIXED, b.first);
+        b.second.copy = nullptr;
+    }
+    h.idle.clear();
+    h.idle_bytes = 0;
+    h.forked = true;
+    h.mu.unlock();
+}
 HostPool& host_pool() {
-    static HostPool* p = new HostPool();
+    static HostPool* p = [] {
+        (void)pthread_atfork(before_fork, after_fork_parent, after_fork_child);
+        return new HostPool();
+    }();
     return *p;
 }
 uint64_t host_block_size(uint64_t n) {
@@ -139,7 +182,7 @@ void host_pool_contexts(int d) {
     HostPool& h = host_pool();
     std::lock_guard<std::mutex> lk(h.mu);
     h.contexts += d;
-    if (h.contexts > 0) return;
+    if (h.contexts > 0 || h.forked) return;
     for (auto& b : h.idle) (void)hipHostFree(b.second);
     h.idle.clear();
     h.idle_bytes = 0;
@@ -158,7 +201,7 @@ int32_t mmhrt_host_alloc(uint64_t bytes, void** out) {
     const uint64_t n = host_block_size(bytes);
     HostPool& h = host_pool();
     std::lock_guard<std::mutex> lk(h.mu);
-    if (h.contexts == 0 || h.out_bytes + n > HostPool::OUT) return MMHRT_E_OOM;
+    if (h.forked || h.contexts == 0 || h.out_bytes + n > HostPool::OUT) return MMHRT_E_OOM;
     void* p = nullptr;
     auto it = h.idle.find(n);
     if (it != h.idle.end()) {
@@ -170,7 +213,7 @@ int32_t mmhrt_host_alloc(uint64_t bytes, void** out) {
         return MMHRT_E_OOM;
     }
     try {
-        h.out.emplace(p, n);
+        h.out.emplace(p, HostPool::Block{n, nullptr});
     } catch (const std::bad_alloc&) {
         (void)hipHostFree(p);
         return MMHRT_E_OOM;
@@ -185,9 +228,13 @@ int32_t mmhrt_host_free(void* p) {
     std::lock_guard<std::mutex> lk(h.mu);
     auto it = h.out.find(p);
     if (it == h.out.end()) return MMHRT_E_INVALID;
-    const uint64_t n = it->second;
+    const uint64_t n = it->second.bytes;
     h.out.erase(it);
     h.out_bytes -= n;
+    if (h.forked) {
+        munmap(p, n);
+        return MMHRT_OK;
+    }
     bool keep = h.contexts > 0 && h.idle_bytes + n <= HostPool::KEEP;
     if (keep) {
         try {

@@ -1,6 +1,9 @@
 """GPU: what programs may do with the page-locked arrays that results arrive in: drop them, after an error
-too, while the device is at work."""
+too, while the device is at work, and hand them to forked workers."""
 import gc
+import os
+import signal
+import time
 
 import numpy as np
 import pytest
@@ -46,3 +49,55 @@ def test_refused_download_leaves_no_copy_behind(busy):
         assert (b == 0x5A5A5A5A).all()
     f = busy.download(1920, 1080, outputs=("depth", "hit_id"))
     assert (f.hit_id >= 0).any() and np.isfinite(f.depth).all()
+
+
+def child_status(f, seconds=60):
+    """Runs f in a forked child and returns the child's wait status (f returning true: 0)."""
+    pid = os.fork()
+    if pid == 0:
+        code = 2
+        try:
+            code = 0 if f() else 1
+        finally:
+            os._exit(code)
+    end = time.monotonic() + seconds
+    while time.monotonic() < end:
+        done, status = os.waitpid(pid, os.WNOHANG)
+        if done:
+            return status
+        time.sleep(0.01)
+    os.kill(pid, signal.SIGKILL)
+    return os.waitpid(pid, 0)[1]
+
+
+def test_frames_in_forked_children(gpu_renderer):
+    """Worker processes forked from a renderer's read, write and drop its frames, as they can with any
+    array, theirs forked in turn too; the parent's frames are not touched."""
+    case("frames in forked children")
+    xyzr, rgba = scenes.random_spheres(2000, seed=4, rmin=0.02, rmax=0.06)
+    names = ("rgba8", "depth", "color", "t", "hit_id")
+    with SphereRenderer(0) as r:
+        r.set_spheres(xyzr, rgba)
+        r.build()
+        frames = [r.render(small_camera(w, h), params(w, h)) for w, h in ((64, 48), (333, 201), (64, 48))]
+        dropped = r.render(small_camera(90, 70), params(90, 70))
+        del dropped  # an idle block of the pool
+        want = [{k: getattr(f, k).copy() for k in names} for f in frames]
+
+        def equal():
+            return all((getattr(f, k).view(np.uint32) == w[k].view(np.uint32)).all() for f, w in zip(frames, want)
+                       for k in names)
+
+        def child():
+            ok = equal() and child_status(equal) == 0
+            for f in frames:
+                f.color[:] = 1.0
+            frames.clear()
+            gc.collect()
+            return ok and L.host_empty((1 << 20,), np.uint8).base is None
+
+        assert child_status(child) == 0
+        assert equal()
+        again = r.render(small_camera(64, 48), params(64, 48))
+        np.testing.assert_array_equal(again.rgba8, want[0]["rgba8"])
+        assert equal()
