@@ -225,9 +225,11 @@ MMHRT_API int32_t mmhrt_get_device_framebuffer(mmhrt_ctx ctx, mmhrt_device_frame
 MMHRT_API int32_t mmhrt_render_noalloc(mmhrt_ctx ctx, const mmhrt_camera* cam, const mmhrt_render_params* params,
                                        const mmhrt_device_framebuffer* out);
 
-/* Page-locked host memory for the calls' host outputs, from a pool of the process (freed blocks are
- * kept, up to 256 MB, until the last context is destroyed). A copy into it runs at the link's rate
- * and needs no staging and no page faults. At most 1 GB is handed out at a time (then MMHRT_E_OOM: use
+/* Page-locked host memory for the calls' host outputs, from a pool of the process. A copy into it runs at
+ * the link's rate and needs no staging and no page faults. mmhrt_host_free never waits for the device:
+ * freed blocks are kept for later calls until a device buffer grows or a context is destroyed, then up to
+ * 256 MB of them until the last context is destroyed. All blocks together take at most 1 GB (freed ones make
+ * room for other sizes while the process has one context; beyond it MMHRT_E_OOM: use
  * ordinary memory). Thread-safe; a block may outlive every context, and a child of fork() finds the blocks'
  * contents at their addresses, in memory of its own. */
 MMHRT_API int32_t mmhrt_host_alloc(uint64_t bytes, void** out);

@@ -5,6 +5,7 @@
 #include <sys/mman.h>
 
 #include <algorithm>
+#include <iterator>
 #include <map>
 #include <mutex>
 #include <new>
@@ -123,8 +124,14 @@ namespace {
 // A block is a mapping of the device's file, which a child of fork() does not inherit (a worker that
 // read a frame of its parent's died of it). So a fork copies the blocks in use into ordinary memory, which
 // the child finds at the blocks' own addresses; to the parent they are what they were.
+// Freeing page-locked memory waits for all of the device's work, that of other contexts too (a frame of
+// 300 MB dropped beside a context with ten frames queued took 139 ms, against 0.3 ms on an idle device),
+// and an array may be dropped anywhere. So a block given back only becomes idle, whatever its size; blocks
+// beyond KEEP are freed where the library waits for the device anyway (host_pool_trim). In use and idle
+// together take at most MOST; for a new size idle ones make room while there is one context, which is about
+// to wait for its own work.
 struct HostPool {
-    static constexpr uint64_t KEEP = 256ull << 20, OUT = 1ull << 30;
+    static constexpr uint64_t KEEP = 256ull << 20, MOST = 1ull << 30;
     struct Block {
         uint64_t bytes;
         void* copy;  // during a fork
@@ -178,16 +185,30 @@ uint64_t host_block_size(uint64_t n) {
     while (step * 8 < n) step *= 2;
     return (n + step - 1) / step * step;
 }
+// Idle blocks beyond `keep` bytes are taken out of the pool, the largest first, and freed outside its lock.
+void host_pool_shrink(HostPool& h, std::unique_lock<std::mutex> lk, uint64_t keep) {
+    std::multimap<uint64_t, void*> gone;
+    while (h.idle_bytes > keep) {
+        auto it = std::prev(h.idle.end());
+        h.idle_bytes -= it->first;
+        gone.insert(h.idle.extract(it));
+    }
+    lk.unlock();
+    for (auto& b : gone) (void)hipHostFree(b.second);
+}
 void host_pool_contexts(int d) {
     HostPool& h = host_pool();
-    std::lock_guard<std::mutex> lk(h.mu);
+    std::unique_lock<std::mutex> lk(h.mu);
     h.contexts += d;
-    if (h.contexts > 0 || h.forked) return;
-    for (auto& b : h.idle) (void)hipHostFree(b.second);
-    h.idle.clear();
-    h.idle_bytes = 0;
+    if (d > 0 || h.forked) return;
+    host_pool_shrink(h, std::move(lk), h.contexts > 0 ? HostPool::KEEP : 0);
 }
 }  // namespace
+void host_pool_trim() {
+    HostPool& h = host_pool();
+    std::unique_lock<std::mutex> lk(h.mu);
+    if (!h.forked && h.idle_bytes > HostPool::KEEP) host_pool_shrink(h, std::move(lk), HostPool::KEEP);
+}
 }  // namespace mmhrt
 
 using namespace mmhrt;
@@ -197,45 +218,50 @@ extern "C" {
 int32_t mmhrt_host_alloc(uint64_t bytes, void** out) {
     if (!out || bytes == 0) return MMHRT_E_INVALID;
     *out = nullptr;
-    if (bytes > HostPool::OUT) return MMHRT_E_OOM;
+    if (bytes > HostPool::MOST) return MMHRT_E_OOM;
     const uint64_t n = host_block_size(bytes);
     HostPool& h = host_pool();
-    std::lock_guard<std::mutex> lk(h.mu);
-    if (h.forked || h.contexts == 0 || h.out_bytes + n > HostPool::OUT) return MMHRT_E_OOM;
+    std::unique_lock<std::mutex> lk(h.mu);
+    if (h.forked || h.contexts == 0) return MMHRT_E_OOM;
+    // an idle block of this size or up to twice it
+    HostPool::Block blk{n, nullptr};
     void* p = nullptr;
-    auto it = h.idle.find(n);
-    if (it != h.idle.end()) {
+    auto it = h.idle.lower_bound(n);
+    if ((it == h.idle.end() || it->first > 2 * n) && h.contexts == 1 && h.out_bytes + n <= HostPool::MOST &&
+        h.out_bytes + h.idle_bytes + n > HostPool::MOST) {
+        host_pool_shrink(h, std::move(lk), HostPool::MOST - n - h.out_bytes);
+        lk = std::unique_lock<std::mutex>(h.mu);
+        it = h.idle.lower_bound(n);
+    }
+    if (it != h.idle.end() && it->first <= 2 * n) {
+        blk.bytes = it->first;
         p = it->second;
         h.idle.erase(it);
-        h.idle_bytes -= n;
+        h.idle_bytes -= blk.bytes;
+    } else if (h.out_bytes + h.idle_bytes + n > HostPool::MOST) {
+        return MMHRT_E_OOM;
     } else if (hipHostMalloc(&p, n, hipHostMallocPortable) != hipSuccess) {
         (void)hipGetLastError();
         return MMHRT_E_OOM;
     }
     try {
-        h.out.emplace(p, HostPool::Block{n, nullptr});
+        h.out.emplace(p, blk);
     } catch (const std::bad_alloc&) {
         (void)hipHostFree(p);
         return MMHRT_E_OOM;
     }
-    h.out_bytes += n;
+    h.out_bytes += blk.bytes;
     *out = p;
     return MMHRT_OK;
 }
 
 int32_t mmhrt_host_free(void* p) {
     HostPool& h = host_pool();
-    std::lock_guard<std::mutex> lk(h.mu);
+    std::unique_lock<std::mutex> lk(h.mu);
     auto it = h.out.find(p);
     if (it == h.out.end()) return MMHRT_E_INVALID;
     const uint64_t n = it->second.bytes;
-    h.out.erase(it);
-    h.out_bytes -= n;
-    if (h.forked) {
-        munmap(p, n);
-        return MMHRT_OK;
-    }
-    bool keep = h.contexts > 0 && h.idle_bytes + n <= HostPool::KEEP;
+    bool keep = !h.forked && h.contexts > 0;
     if (keep) {
         try {
             h.idle.emplace(n, p);
@@ -244,7 +270,14 @@ int32_t mmhrt_host_free(void* p) {
             keep = false;
         }
     }
-    if (!keep) (void)hipHostFree(p);
+    h.out.erase(it);
+    h.out_bytes -= n;
+    const bool forked = h.forked;
+    lk.unlock();
+    if (forked)
+        munmap(p, n);
+    else if (!keep)
+        (void)hipHostFree(p);
     return MMHRT_OK;
 }
 

@@ -206,6 +206,9 @@ int settle(mmhrt_ctx_s* c, int code);
 // to give (or they are in use)
 bool release_series(mmhrt_ctx_s* c);
 
+// api.hip: idle page-locked blocks beyond what the pool keeps are freed; for places that wait for the device
+void host_pool_trim();
+
 template <typename T>
 int ensure(mmhrt_ctx_s* c, DevBuf<T>& b, size_t n, const char* what) {
     if (b.cap >= n && b.p) return 0;
@@ -216,6 +219,7 @@ int ensure(mmhrt_ctx_s* c, DevBuf<T>& b, size_t n, const char* what) {
         b.p = nullptr;
         b.cap = 0;
         if (e != hipSuccess) return hip_fail(c, e, what);
+        host_pool_trim();
     }
     size_t bytes = (n ? n : 1) * sizeof(T);
     hipError_t e = hipMalloc((void**)&b.p, bytes);

@@ -1,5 +1,5 @@
 """GPU: what programs may do with the page-locked arrays that results arrive in: drop them, after an error
-too, while the device is at work, and hand them to forked workers."""
+too, while the device is at work, hand them to forked workers, keep as many as they like."""
 import gc
 import os
 import signal
@@ -30,6 +30,16 @@ def busy():
         long_work(r, 1)  # buffers are allocated now
         r.sync()
         yield r
+
+
+def test_sizes_change(gpu_renderer):
+    """With one context idle blocks make room for those of another size at once."""
+    case("host pool, another size")
+    small = [L.host_empty((256 << 20,), np.uint8) for _ in range(4)]
+    assert small[0].base is not None
+    del small
+    gc.collect()
+    assert L.host_empty((600 << 20,), np.uint8).base is not None
 
 
 def test_refused_download_leaves_no_copy_behind(busy):
@@ -101,3 +111,39 @@ def test_frames_in_forked_children(gpu_renderer):
         again = r.render(small_camera(64, 48), params(64, 48))
         np.testing.assert_array_equal(again.rgba8, want[0]["rgba8"])
         assert equal()
+
+
+@pytest.mark.parametrize("mb,blocks", [(300, 1), (40, 20)])
+def test_dropping_results_does_not_wait(busy, mb, blocks):
+    """Arrays of any size, and many of them, are dropped at once while another renderer's frames are
+    queued; only a renderer that must wait for its own buffers gives the memory back."""
+    case(f"drop {blocks} x {mb} MB beside a busy renderer")
+    held = [L.host_empty((mb << 20,), np.uint8) for _ in range(blocks)]
+    assert held[0].base is not None
+    long_work(busy)
+    t0 = time.perf_counter()
+    del held
+    gc.collect()
+    t1 = time.perf_counter()
+    busy.sync()
+    t2 = time.perf_counter()
+    assert t1 - t0 < 0.5 * (t2 - t1), (t1 - t0, t2 - t1)
+
+
+def test_idle_memory_is_given_back(gpu_renderer):
+    """In use and idle together the pool takes 1 GB; past that arrays are ordinary until a device buffer
+    grows, which leaves at most 256 MB idle."""
+    case("idle memory of the host pool")
+    del_me = [L.host_empty((256 << 20,), np.uint8) for _ in range(4)]
+    assert any(a.base is not None for a in del_me)
+    del del_me
+    gc.collect()
+    with SphereRenderer(0) as r:
+        xyzr, rgba = scenes.random_spheres(2000, seed=4, rmin=0.02, rmax=0.06)
+        r.set_spheres(xyzr, rgba)
+        r.build()
+        r.render_async(small_camera(64, 48), params(64, 48))
+        assert L.host_empty((600 << 20,), np.uint8).base is None
+        r.render_async(small_camera(640, 480), params(640, 480))
+        r.sync()
+        assert L.host_empty((600 << 20,), np.uint8).base is not None
