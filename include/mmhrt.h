@@ -281,7 +281,9 @@ MMHRT_API int32_t mmhrt_get_counters(mmhrt_ctx ctx, uint64_t* node_visits, uint6
  * then one persistent launch per mode (Lambert, AO) traces every job of the series; with option
  * "batch_launch" 0 each timestep's jobs are traced right after its build instead (one launch per
  * timestep, whose jobs must then share the mode; no per-timestep structures are kept). use_graph
- * captures the whole sequence into one hipGraph and launches it once. */
+ * captures the whole sequence into one hipGraph and launches it once. A finished call leaves its
+ * structures for later ones of any context, at most 1 GB of them in the process; they are freed where
+ * an allocation of a context on their device fails, and when a context is destroyed. */
 typedef struct mmhrt_job {
     uint32_t timestep;
     uint32_t reserved;

@@ -312,7 +312,6 @@ int32_t mmhrt_create(int32_t device, mmhrt_ctx* out) {
     }
     hipDeviceGetAttribute(&c->cu_count, hipDeviceAttributeMultiprocessorCount, device);
     if (c->cu_count <= 0) c->cu_count = 1;
-    if (hipDeviceTotalMem(&c->mem_total, device) != hipSuccess) (void)hipGetLastError();
     for (int i = 0; i < 12; ++i) hipEventCreate(&c->tm.ev[i]);
     c->tm.init = true;
     // the device address of this device's scratch array for mmhrt_render_noalloc; on failure that
@@ -346,7 +345,7 @@ int32_t mmhrt_destroy(mmhrt_ctx c) {
     release(c->ts_sph); release(c->ts_col); release(c->bt_col); release(c->bt_depth); release(c->bt_t);
     release(c->bt_id); release(c->bt_rgba8); release(c->batch_ctr); release(c->batch_prefix);
     release(c->batch_jobs);
-    release_series(c);
+    release_series(c->device);
     if (c->rounds_host) (void)hipHostFree(c->rounds_host);
     c->rounds_host = nullptr;
     if (c->dn) {

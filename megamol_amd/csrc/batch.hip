@@ -11,6 +11,8 @@
 #include <string.h>
 
 #include <algorithm>
+#include <mutex>
+#include <new>
 #include <vector>
 
 #include "ctx.hpp"
@@ -58,18 +60,21 @@ void frame_consts_batch(const mmhrt_camera* cam, const mmhrt_render_params* p, F
     }
 }
 
-size_t series_bytes(const mmhrt_ctx_s* c) {
-    size_t b = 0;
-    for (const auto& sl : c->ts_slots)
-        b += sl.nodes.cap * sizeof(Node) + sl.leaf.cap * 16 + sl.id.cap * 4 + sl.dim.cap + sl.box.cap * 4 + sl.rmax.cap * 4;
-    return b;
+// The per-timestep structures of finished series, kept for later ones of any context of the process (a call
+// over 8 x 500k spheres spent 3.5 of its 12.8 ms on allocating and freeing them). They take at most
+// SERIES_KEEP, whatever the number of contexts, and are freed where an allocation of any context on their
+// device fails, and when a context is destroyed.
+constexpr size_t SERIES_KEEP = 1ull << 30;
+std::mutex g_series_mu;
+std::vector<SeriesSlot>& series_idle() {  // the oldest first
+    static std::vector<SeriesSlot>* v = new std::vector<SeriesSlot>();
+    return *v;
 }
-}  // namespace
-
-namespace mmhrt {
-bool release_series(mmhrt_ctx_s* c) {
-    if (c->ts_busy || c->ts_slots.empty()) return false;
-    for (auto& sl : c->ts_slots) {
+size_t slot_bytes(const SeriesSlot& sl) {
+    return sl.nodes.cap * sizeof(Node) + sl.leaf.cap * 16 + sl.id.cap * 4 + sl.dim.cap + sl.box.cap * 4 + sl.rmax.cap * 4;
+}
+void free_slots(std::vector<SeriesSlot>& v) {
+    for (auto& sl : v) {
         release(sl.nodes);
         release(sl.leaf);
         release(sl.id);
@@ -78,8 +83,65 @@ bool release_series(mmhrt_ctx_s* c) {
         release(sl.box);
         release(sl.rmax);
     }
-    c->ts_slots.clear();
-    return true;
+    v.clear();
+}
+// A kept slot that holds n spheres and n_nodes nodes, the smallest such one, or an empty one.
+SeriesSlot take_slot(int device, size_t n_nodes, size_t n) {
+    std::lock_guard<std::mutex> lk(g_series_mu);
+    auto& idle = series_idle();
+    size_t best = idle.size();
+    for (size_t i = 0; i < idle.size(); ++i)
+        if (idle[i].device == device && idle[i].nodes.cap >= n_nodes && idle[i].leaf.cap >= n &&
+            (best == idle.size() || slot_bytes(idle[i]) < slot_bytes(idle[best])))
+            best = i;
+    SeriesSlot sl;
+    sl.device = device;
+    if (best < idle.size()) {
+        sl = idle[best];
+        idle.erase(idle.begin() + best);
+    }
+    return sl;
+}
+// The slots of a finished series (no work on them is under way) are kept, the oldest beyond SERIES_KEEP freed.
+void keep_slots(std::vector<SeriesSlot>& slots) {
+    std::vector<SeriesSlot> gone;
+    {
+        std::lock_guard<std::mutex> lk(g_series_mu);
+        auto& idle = series_idle();
+        try {
+            gone.reserve(idle.size() + slots.size());
+            idle.insert(idle.end(), slots.begin(), slots.end());
+            slots.clear();
+            size_t bytes = 0;
+            for (const auto& sl : idle) bytes += slot_bytes(sl);
+            size_t k = 0;
+            for (; bytes > SERIES_KEEP; ++k) {
+                bytes -= slot_bytes(idle[k]);
+                gone.push_back(idle[k]);
+            }
+            idle.erase(idle.begin(), idle.begin() + k);
+        } catch (const std::bad_alloc&) {
+        }
+    }
+    free_slots(gone);
+    free_slots(slots);  // (those that could not be kept)
+}
+}  // namespace
+
+namespace mmhrt {
+bool release_series(int device) {
+    std::vector<SeriesSlot> gone;
+    try {
+        std::lock_guard<std::mutex> lk(g_series_mu);
+        auto& idle = series_idle();
+        auto it = std::stable_partition(idle.begin(), idle.end(), [&](const SeriesSlot& sl) { return sl.device != device; });
+        gone.assign(it, idle.end());
+        idle.erase(it, idle.end());
+    } catch (const std::bad_alloc&) {
+    }
+    const bool any = !gone.empty();
+    free_slots(gone);
+    return any;
 }
 }  // namespace mmhrt
 
@@ -188,23 +250,24 @@ int32_t mmhrt_render_batch(mmhrt_ctx c, const mmhrt_job* jobs, uint32_t n_jobs, 
     // The builds read the timestep slices and their count; the context's own spheres, count and
     // LBVH state come back when this call returns (the tree in the buffers is then the last
     // timestep's, so the context needs a build before its next render).
-    // The per-timestep structures stay allocated for the next call while they take at most an eighth of
-    // the device's memory, and are given back where another allocation needs the room (ensure), and with
-    // the context: allocating and freeing them was 3.5 of the 12.8 ms of a call over 8 x 500k spheres.
+    std::vector<SeriesSlot> slots;  // the structures of the timesteps but the last (one launch over all)
     struct Restore {
         mmhrt_ctx_s* c;
         uint64_t n;
+        std::vector<SeriesSlot>& slots;
+        bool done;
         ~Restore() {
             c->sph_cur = nullptr;
             c->n = n;
             c->built = false;
             c->info_valid = false;
-            c->ts_busy = false;
-            if (series_bytes(c) > c->mem_total / 8) release_series(c);
+            if (done)
+                keep_slots(slots);
+            else
+                free_slots(slots);  // (hipFree waits for work on them)
         }
-    } restore{c, c->n};
+    } restore{c, c->n, slots, false};
     c->built = false;
-    c->ts_busy = true;
     // every buffer the per-timestep build and trace touch is allocated before any capture
     c->sph_cur = c->ts_sph.p;
     c->n = c->ts_n;
@@ -226,9 +289,10 @@ int32_t mmhrt_render_batch(mmhrt_ctx c, const mmhrt_job* jobs, uint32_t n_jobs, 
         // sized for this series (the context's own buffers may be larger, from an earlier scene)
         const uint64_t n = c->ts_n;
         const size_t n_nodes = tl ? (size_t)c->pkd_L - 1 : (size_t)(n > 1 ? n - 1 : 1);
-        if (c->ts_slots.size() < T - 1) c->ts_slots.resize(T - 1);
+        slots.reserve(T - 1);
         for (uint32_t t = 0; t + 1 < T; ++t) {
-            SeriesSlot& sl = c->ts_slots[t];
+            slots.push_back(take_slot(c->device, n_nodes, n));
+            SeriesSlot& sl = slots[t];
             if ((e = ensure(c, sl.nodes, n_nodes, "series nodes"))) return e;
             if ((e = ensure(c, sl.leaf, n, "series leaf spheres"))) return e;
             if ((e = ensure(c, sl.info, 1, "series scene info"))) return e;
@@ -243,7 +307,7 @@ int32_t mmhrt_render_batch(mmhrt_ctx c, const mmhrt_job* jobs, uint32_t n_jobs, 
     auto bind = [&](uint32_t t) {
         if (!one) return;
         if (t + 1 < T) {
-            SeriesSlot& sl = c->ts_slots[t];
+            SeriesSlot& sl = slots[t];
             std::swap(c->nodes, sl.nodes);
             std::swap(c->leaf_sph, sl.leaf);
             std::swap(c->info, sl.info);
@@ -254,7 +318,7 @@ int32_t mmhrt_render_batch(mmhrt_ctx c, const mmhrt_job* jobs, uint32_t n_jobs, 
             }
         }
         const uint32_t g = t / period;
-        if (g + 1 < G) std::swap(c->leaf_id, c->ts_slots[g].id);
+        if (g + 1 < G) std::swap(c->leaf_id, slots[g].id);
     };
     // job table and tile prefixes (the jobs of a launch are contiguous, each launch's prefix
     // array starts at 0)
@@ -349,6 +413,7 @@ int32_t mmhrt_render_batch(mmhrt_ctx c, const mmhrt_job* jobs, uint32_t n_jobs, 
     if (rgba8_out) he = hipMemcpy(rgba8_out, c->bt_rgba8.p, total_px * 4, hipMemcpyDeviceToHost);
     if (he == hipSuccess && depth_out) he = hipMemcpy(depth_out, c->bt_depth.p, total_px * 4, hipMemcpyDeviceToHost);
     if (he != hipSuccess) return hip_fail(c, he, "render_batch download");
+    restore.done = true;
     return MMHRT_OK;
 }
 

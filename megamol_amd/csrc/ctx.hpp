@@ -52,6 +52,7 @@ struct DevBuf {
 // treelets, the split axes, treelet boxes and radii; `id` holds the leaf order of one rebuild (its
 // refits share it).
 struct SeriesSlot {
+    int device = 0;
     DevBuf<Node> nodes;
     DevBuf<float4> leaf;
     DevBuf<uint32_t> id;
@@ -73,7 +74,6 @@ struct mmhrt_ctx_s {
     std::string err;
     std::string noalloc_err;  // why mmhrt_render_noalloc cannot run on this device ("" = it can)
     int cu_count = 0;
-    size_t mem_total = 0;  // bytes of device memory
 
     // scene (original particle order)
     uint64_t n = 0;
@@ -179,8 +179,6 @@ struct mmhrt_ctx_s {
     mmhrt::DevBuf<int32_t> bt_id;
     mmhrt::DevBuf<uint32_t> bt_rgba8, batch_ctr, batch_prefix;
     mmhrt::DevBuf<uint8_t> batch_jobs;
-    std::vector<mmhrt::SeriesSlot> ts_slots;  // per timestep but the last (one-launch series), kept between calls
-    bool ts_busy = false;                     // a series is being built and traced
 
     // learned denoiser (created on first use)
     mmhrt::dn::Denoiser* dn = nullptr;
@@ -202,9 +200,9 @@ int hip_fail(mmhrt_ctx_s* c, hipError_t e, const char* what);
 // the caller may free or reuse that memory once the call is over. Returns code.
 int settle(mmhrt_ctx_s* c, int code);
 
-// batch.hip: the structures that a series keeps between calls are given back; false if there were none
-// to give (or they are in use)
-bool release_series(mmhrt_ctx_s* c);
+// batch.hip: the structures on this device that finished series left for later ones are freed; false if
+// there were none
+bool release_series(int device);
 
 // api.hip: idle page-locked blocks beyond what the pool keeps are freed; for places that wait for the device
 void host_pool_trim();
@@ -223,7 +221,7 @@ int ensure(mmhrt_ctx_s* c, DevBuf<T>& b, size_t n, const char* what) {
     }
     size_t bytes = (n ? n : 1) * sizeof(T);
     hipError_t e = hipMalloc((void**)&b.p, bytes);
-    if (e != hipSuccess && release_series(c)) {  // the kept structures make room for what is needed now
+    if (e != hipSuccess && release_series(c->device)) {  // the kept structures make room for what is needed now
         (void)hipGetLastError();
         e = hipMalloc((void**)&b.p, bytes);
     }
