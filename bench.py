@@ -183,7 +183,7 @@ def run_build_sweep(r, args):
             r.set_option(k, v)
             rows.append({"options": {k: v}, **measure()})
             log(f"build {k}={v}: {rows[-1]}")
-            r.set_option(k, defaults[k])
+            r.set_option(k, -1 if k in ("sort_ri", "build_span") else defaults[k])  # (-1: as without a request)
     print(json.dumps({"build_sweep": rows, "spheres": r.info()[0], "bits": args.bits}), flush=True)
 
 

@@ -338,14 +338,15 @@ MMHRT_API int32_t mmhrt_denoiser_train_step(mmhrt_ctx ctx, const uint16_t* feats
  * (leaves per LBVH chunk workgroup: 1024, 512 or 256), "build_ls" (level-synchronous chunk
  * pass, default 1; 0: one climbing thread per leaf), "build_grid" (test hook: at most this many
  * persistent chunk workgroups, 0 = as many as fit), "sort_ri" (radix sort keys per thread per
- * tile: 8, 16 or 32, default 16, which takes 8 up to 2^19 spheres and one workgroup's sort up to 2^14), "sort_onesweep" (single-pass radix passes with look-back, default 0),
+ * tile: 8, 16 or 32; -1, the default: 16, 8 up to 2^19 spheres and one workgroup's sort up to 2^14; "used_sort_ri" is
+ * what the last build took, 0 for one workgroup's sort), "sort_onesweep" (single-pass radix passes with look-back, default 0),
  * "sort_digit" (radix digit width: 8, the default, or 0 for wide digits: three 10-bit passes over
  * 30-bit keys, six 11-bit passes over 63-bit keys),
  * "leaf_pairs" (default 1: nodes over two leaves are not stored, their parents reference the
  * pair; 0: every node is stored), "build_tail" (straddler worklist size from which one
  * workgroup finishes the tree, default 512; used when "build_span" is 0), "build_span" (straddlers
- * merged by one workgroup per span of this many chunks before the tail, default 256, at most 64 up to
- * 8192 chunks; 0: kernel rounds), "build_wave" (chunk pass: once a round would merge at most this many splits, the
+ * merged by one workgroup per span of this many chunks before the tail; -1, the default: 256, 64 up to
+ * 8192 chunks; 0: kernel rounds; "used_build_span" is what the last build took), "build_wave" (chunk pass: once a round would merge at most this many splits, the
  * rest of the chunk climbs without rounds, one lane per split; default 64, one wavefront; up to
  * the chunk size; 0: rounds to the top),
  * "accel" (structure the next build makes: 0 LBVH, the default; 1 treelet P-k-d trees, about one

@@ -739,6 +739,8 @@ static int64_t* option_slot(mmhrt_ctx c, const char* key) {
     if (k == "batch_launch") return &c->opt_batch_launch;
     if (k == "stack_overflow") return &c->stack_overflow;
     if (k == "pair_visits") return &c->pair_visits;
+    if (k == "used_sort_ri") return &c->used_sort_ri;
+    if (k == "used_build_span") return &c->used_build_span;
     if (k == "leaf_fetches") return &c->leaf_fetches;
     return nullptr;
 }
@@ -747,6 +749,11 @@ int32_t mmhrt_set_option(mmhrt_ctx c, const char* key, int64_t value) {
     if (!c) return MMHRT_E_INVALID;
     int64_t* s = option_slot(c, key);
     if (!s) return fail(c, MMHRT_E_INVALID, std::string("set_option: unknown key ") + (key ? key : "(null)"));
+    // these two adapt to the scene until a value is asked for; a negative one goes back to that
+    if (s == &c->opt_sort_ri || s == &c->opt_build_span) {
+        (s == &c->opt_sort_ri ? c->sort_ri_set : c->build_span_set) = value >= 0;
+        if (value < 0) value = s == &c->opt_sort_ri ? 16 : 256;
+    }
     *s = value;
     return MMHRT_OK;
 }

@@ -158,6 +158,8 @@ struct mmhrt_ctx_s {
     int64_t opt_build_wave = 64;    // chunk pass: from this many merges on, lanes climb instead of rounds (0: never)
     int64_t opt_sort_xcd = 1;       // radix scatter: each XCD takes one contiguous range of tiles (0: round robin)
     int64_t opt_build_span = 256;   // straddlers: one workgroup per span of this many chunks, then the tail (0: rounds)
+    bool sort_ri_set = false, build_span_set = false;  // asked for: taken as they are, not adapted to the scene's size
+    int64_t used_sort_ri = 0, used_build_span = 0;     // of the last build
     int64_t opt_fail_alloc = 0;     // test hook: the k-th device allocation from now fails with E_OOM (0: none)
     int64_t opt_accel = 0;          // structure the next build makes: 0 LBVH, 1 treelet P-k-d trees
     int64_t opt_treelet = 1024;     // spheres per treelet of the P-k-d structure: 256, 512 or 1024

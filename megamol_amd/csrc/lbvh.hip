@@ -1917,8 +1917,11 @@ int morton_sort(mmhrt_ctx_s* c, K* ka, K* kb, uint32_t* va, uint32_t* vb, uint32
                 bool reserve_only) {
     // tiles of 16 keys per thread (the default) halve where they would leave CUs idle: 250k spheres (62
     // tiles of 16) build in 170 us with them, in 157 us with tiles of 8; 1M in 255 and 258 us
-    if (c->opt_sort_ri == 8 || (c->opt_sort_ri == 16 && n <= (1u << 19))) return morton_sort_d<K, 8>(c, ka, kb, va, vb, vfinal, n, reserve_only);
-    if (c->opt_sort_ri == 32 && sizeof(K) == 4) return morton_sort_d<K, 32>(c, ka, kb, va, vb, vfinal, n, reserve_only);
+    const int64_t ri = c->sort_ri_set || n > (1u << 19) ? c->opt_sort_ri : 8;
+    c->used_sort_ri = ri == 8 ? 8 : ri == 32 && sizeof(K) == 4 ? 32 : 16;
+    if (c->used_sort_ri == 8) return morton_sort_d<K, 8>(c, ka, kb, va, vb, vfinal, n, reserve_only);
+    if constexpr (sizeof(K) == 4)
+        if (c->used_sort_ri == 32) return morton_sort_d<K, 32>(c, ka, kb, va, vb, vfinal, n, reserve_only);
     return morton_sort_d<K, 16>(c, ka, kb, va, vb, vfinal, n, reserve_only);
 }
 
@@ -1965,8 +1968,9 @@ int hierarchy(mmhrt_ctx_s* c, const K* keys, const uint32_t* ids, bool reserve_o
     // with spans of 256, 242, 235, 234, 233, 243 us with 128, 64, 32, 16, 8; 4M refit in 310 us, then 300,
     // 295, 299, 322, 387; 50M (48.8k chunks) in 1.60 ms of boxes with 128 against 1.53 with 256
     const int64_t span_chunks = !bounds_stored ? std::max<int64_t>(c->opt_build_span, (nchunks + 255) / 256)
-                                : nchunks <= 8192 ? std::min<int64_t>(c->opt_build_span, 64)
-                                                  : c->opt_build_span;
+                                : c->build_span_set || nchunks > 8192 ? c->opt_build_span
+                                                                      : 64;
+    c->used_build_span = c->opt_build_span > 0 ? span_chunks : 0;
     const int64_t span = span_chunks * (int64_t)bc;
     const uint64_t spans = c->opt_build_span > 0 ? (n + span - 1) / span : 0;
     const size_t xcap = 4 * spans + 64;
@@ -2114,9 +2118,10 @@ template <typename K>
 static int bounds_and_sort(mmhrt_ctx_s* c, K* ka, K* kb, uint32_t* ids, bool reserve_only) {
     const uint64_t n = c->n;
     if (int e = reserve_reduction(c)) return e;
-    const bool plain = c->opt_sort_digit != 0 && c->opt_sort_onesweep == 0 && c->opt_sort_ri == 16;
+    const bool plain = c->opt_sort_digit != 0 && c->opt_sort_onesweep == 0 && !c->sort_ri_set;
     if (plain && n <= small_sort_max<K>()) {
         if (reserve_only) return 0;
+        c->used_sort_ri = 0;
         rec(c, 1);
         rec(c, 2);
         const PassInit init = pass_init(c);
