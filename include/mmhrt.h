@@ -345,8 +345,8 @@ MMHRT_API int32_t mmhrt_denoiser_train_step(mmhrt_ctx ctx, const uint16_t* feats
  * "leaf_pairs" (default 1: nodes over two leaves are not stored, their parents reference the
  * pair; 0: every node is stored), "build_tail" (straddler worklist size from which one
  * workgroup finishes the tree, default 512; used when "build_span" is 0), "build_span" (straddlers
- * merged by one workgroup per span of this many chunks before the tail; -1, the default: 256, 64 up to
- * 8192 chunks; 0: kernel rounds; "used_build_span" is what the last build took), "build_wave" (chunk pass: once a round would merge at most this many splits, the
+ * merged by one workgroup per span of this many chunks before the tail; -1, the default: 256, and
+ * 64 from 257 to 8192 chunks; 0: kernel rounds; "used_build_span" is what the last build took), "build_wave" (chunk pass: once a round would merge at most this many splits, the
  * rest of the chunk climbs without rounds, one lane per split; default 64, one wavefront; up to
  * the chunk size; 0: rounds to the top),
  * "accel" (structure the next build makes: 0 LBVH, the default; 1 treelet P-k-d trees, about one

@@ -1963,13 +1963,16 @@ int hierarchy(mmhrt_ctx_s* c, const K* keys, const uint32_t* ids, bool reserve_o
     // most three per span: its right boundary from the chunk pass, its two boundary splits).
     // Without flags2 at most 256 spans: every span's workgroup then scans the chunk pass's
     // whole list, so larger scenes take longer spans rather than more of them
-    // Where those make few spans they take 64 chunks at most, which trades levels of a span's workgroup
-    // for levels of the top's and runs more spans side by side: 1M spheres (977 chunks) build in 254 us
-    // with spans of 256, 242, 235, 234, 233, 243 us with 128, 64, 32, 16, 8; 4M refit in 310 us, then 300,
-    // 295, 299, 322, 387; 50M (48.8k chunks) in 1.60 ms of boxes with 128 against 1.53 with 256
+    // Without a request: one span, and no pass over exports after it, up to 256 chunks; spans of 64 chunks
+    // up to 8192, which trade levels of a span's workgroup for levels of the top's and run more spans side
+    // by side. Refits of 66, 98, 147, 196, 225 chunks take 77, 78, 87, 92, 97 us with one span and 93, 96,
+    // 102, 101, 103 us with spans of 64; 258 and 391 chunks 103 and 122 us with one, 108 and 113 with spans
+    // of 64, 121 and 126 with spans of 256. 1M spheres (977 chunks) build in 254 us with spans of 256, 242,
+    // 235, 234, 233, 243 us with 128, 64, 32, 16, 8; 4M refit in 310 us, then 300, 295, 299, 322, 387;
+    // 50M (48.8k chunks) in 1.60 ms of boxes with 128 against 1.53 with 256
     const int64_t span_chunks = !bounds_stored ? std::max<int64_t>(c->opt_build_span, (nchunks + 255) / 256)
-                                : c->build_span_set || nchunks > 8192 ? c->opt_build_span
-                                                                      : 64;
+                                : c->build_span_set || nchunks <= 256 || nchunks > 8192 ? c->opt_build_span
+                                                                                        : 64;
     c->used_build_span = c->opt_build_span > 0 ? span_chunks : 0;
     const int64_t span = span_chunks * (int64_t)bc;
     const uint64_t spans = c->opt_build_span > 0 ? (n + span - 1) / span : 0;
