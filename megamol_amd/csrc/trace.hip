@@ -955,10 +955,13 @@ __device__ void shade_pixel(const TraceArgs& A, uint32_t px, uint32_t py, float 
 // ms; 60M clustered at 4K: 6.7 against 5.7; 10k spheres at 320x240: 92 against 80 us): bound by the
 // vector memory unit's address rate (busy 60-90 %), then by VALU issue (50-70 %).
 // Small frames (W = 5) are held to 102 VGPRs, with hardly a spill: their wavefronts have one or two tiles
-// each and the longest rays are the kernel's time. One sample, 1.5 tiles per wavefront (816x600), scenes
-// of 100k, 1M, 4M spheres: AO 238, 282, 310 -> 210, 255, 295 us, Lambert 189, 229, 266 -> 173, 198, 230 and
-// 4 bounces 0.51, 0.52, 0.56 -> 0.45, 0.48, 0.54 ms (640x480 0 to 12 % off, 320x240 the same); at 2.1 tiles
-// (960x720) 4 and 8 bounces take 5 to 22 % longer, at 1280x720 a Lambert frame 4 %.
+// each and the longest rays are the kernel's time. One sample, W = 5 against 7 at 0.2 to 3.5 tiles per
+// wavefront (5 scenes of 100k to 4M spheres, uniform, FCC and clusters; Lambert, AO, 1, 4 and 8 bounces): up to
+// 1.5 tiles 0 to 20 % off and at most 2 % longer (as two runs differ), at 1.65 up to 14 % off but 4 bounces over FCC spheres 4 %
+// longer, at 1.8 13 % off to 5 % longer, at 1.95 and 2.1 uniform scenes of 1M and more 2 to 23 % longer in
+// every mode. So the line is at 1.5, in all modes. It counts the 20 wavefronts a CU holds at W = 5: with
+// fewer (blocks_per_cu 2 and 4, mmhrt_render_noalloc) both take the same time within 3 %, or W = 5 up to
+// 10 % less.
 template <int S, int MODE, bool COUNT, bool STEAL, bool TL = false, int W = TL ? 5 : 7>
 __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(W, 8))) void k_trace(TraceArgs A) {
     __shared__ int2 lds_stack[LaneStack<S>::N * TB];
@@ -1396,7 +1399,7 @@ template <int S, int MODE>
 void launch2(const TraceArgs& A, const Grid& g, bool steal, bool count) {
     if (count)
         launch3<S, MODE, true>(A, g, steal);
-    else if (steal && A.fc.spp == 1 && A.n_tiles <= 30 * g.cus)  // 1.5 for each of 20 wavefronts per CU
+    else if (steal && A.fc.spp == 1 && A.n_tiles <= 30 * g.cus)  // 1.5 for each of 20 wavefronts per CU (figures at k_trace)
         launch_resident<k_trace<S, MODE, false, true, false, 5>>(g, A);
     else
         launch3<S, MODE, false>(A, g, steal);
@@ -1435,11 +1438,12 @@ constexpr int TL_STACK = 10 + SPILL_DIST;
 // well enough: k_tl_cost counts them in steps of four (one lane per tile, boxes of the top tree only),
 // k_tl_order sorts the tiles by it, and the work queues hand out the first tiles of the order before the
 // others. 8M clustered spheres at 1280x720: trace 5.2 -> 4.4 ms, for 0.09 ms of counting and 0.015 of
-// sorting. For 2 to 8 tiles per wavefront: at 1280x720 (2.8) it takes 0 to 13 % off frames of 50k to 4M
-// spheres, uniform or clustered, at 1080p (6.3) up to 16 % off, at worst 2 % more (2M clustered, 11.1 ->
-// 11.4 ms: neighbouring tiles no longer share a cache), but at 800x600 (1.5) uniform scenes take up
-// to 9 % longer (1M: 2.15 -> 2.35 ms, the dear tiles all run at once). Four wavefronts for each of
-// the dearest 1/64 to 1/8 of the tiles took 4 to 25 % longer, wavefront priority by age 1 %.
+// sorting. For 2 to 8 tiles per wavefront. Ordered against as they lie, Lambert and AO over 6 scenes of 100k
+// to 4M spheres: clusters take 3 to 26 % less at every ratio from 1 to 12, most at 2.8 to 4.5. Uniform and
+// FCC scenes take up to 14 % longer at 1, 8 % at 1.65, 11 % at 1.8 (AO 9, 7 and 2 %); at 2.05, 2.2 and 2.4
+// Lambert frames still take up to 8, 6 and 3 % longer, AO frames 1 % longer to 16 % less; from 2.8 to 9
+// nothing takes more than 2 % longer, at 12 AO frames 2 % with half of the gain. Four wavefronts for
+// each of the dearest 1/64 to 1/8 of the tiles took 4 to 25 % longer, wavefront priority by age 1 %.
 constexpr int TL_TOP = 24;  // stack entries of a walk over the top tree (at most 22 levels)
 __global__ __launch_bounds__(TB) void k_tl_cost(TraceArgs A, uint32_t* cost) {
     __shared__ int2 lds_stack[TL_TOP * TB];
