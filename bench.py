@@ -59,7 +59,7 @@ def dram_traffic(workload_key, path=DRAM_PROFILE, field="dram_bytes_per_launch")
 
 def trace_kernel_label(r, spp, mode):
     """Name of the traversal kernel the library dispatches for this frame (mirrors render_frame)."""
-    sl = (r.get_option("sample_lanes") and r.get_option("refill") == 0 and spp > 1
+    sl = (r.get_option("sample_lanes") and r.get_option("refill") <= 0 and spp > 1
           and ((spp <= 64 and spp & (spp - 1) == 0) or spp % 64 == 0))
     name = "k_trace_sl" if sl else "k_trace"
     return f"{name} ({mode}, {spp} spp)"
@@ -70,10 +70,10 @@ def trace_kernel_label(r, spp, mode):
 # AO frame with the feature buffer.
 ABLATION = {
     "64spp": [
-        ("sample lanes, work stealing, LDS stack 16 words (library default), 8x8 tiles", {"stack_lds": 16, "refill": 0}),
-        ("LDS stack 8 words", {"stack_lds": 8, "refill": 0}),
-        ("LDS stack 24 words", {"stack_lds": 24, "refill": 0}),
-        ("LDS stack 32 words", {"stack_lds": 32, "refill": 0}),
+        ("sample lanes, work stealing, 10 stack entries in LDS (library default), 8x8 tiles", {"stack_lds": 16, "refill": 0}),
+        ("6 stack entries in LDS", {"stack_lds": 8, "refill": 0}),
+        ("14 stack entries in LDS", {"stack_lds": 24, "refill": 0}),
+        ("18 stack entries in LDS", {"stack_lds": 32, "refill": 0}),
         ("4x16 tiles", {"stack_lds": 16, "refill": 0, "tile_w": 4}),
         ("lane per pixel (samples in a loop)", {"stack_lds": 16, "refill": 0, "sample_lanes": 0}),
         ("lane per pixel, static tile order (no work stealing)",
@@ -85,13 +85,13 @@ ABLATION = {
          {"stack_lds": 16, "refill": 0, "leaf_pairs": 1}),
     ],
     "1spp": [
-        ("lane per pixel, work stealing, LDS stack 16 words, 8x8 tiles, no compaction (library default)",
+        ("lane per pixel, work stealing, 10 stack entries in LDS, 8x8 tiles, no compaction (library default)",
          {"stack_lds": 16, "refill": 0}),
         ("static tile order (no work stealing)", {"stack_lds": 16, "refill": 0, "persistent": 0}),
         ("ballot compaction (refill at 16 idle lanes)", {"stack_lds": 16, "refill": 16}),
         ("ballot compaction (refill at 32 idle lanes)", {"stack_lds": 16, "refill": 32}),
-        ("LDS stack 8 words", {"stack_lds": 8, "refill": 0}),
-        ("LDS stack 32 words", {"stack_lds": 32, "refill": 0}),
+        ("6 stack entries in LDS", {"stack_lds": 8, "refill": 0}),
+        ("18 stack entries in LDS", {"stack_lds": 32, "refill": 0}),
         ("4 workgroups per CU", {"stack_lds": 16, "refill": 0, "blocks_per_cu": 4}),
         ("tree without leaf pairs", {"stack_lds": 16, "refill": 0, "leaf_pairs": 0}),
     ],
@@ -806,22 +806,21 @@ def main():
     frame()
     visits, tests, rays = r.counters()
     overflow = r.get_option("stack_overflow")
-    pair_visits, leaf_fetches = r.get_option("pair_visits"), r.get_option("leaf_fetches")
+    pair_visits = r.get_option("pair_visits")
     r.set_option("count_visits", 0)
     fr = r.download(args.width, args.height, outputs=("hit_id",))
     hit_px = int((fr.hit_id >= 0).sum())
     P = args.width * args.height
     hit_samples = rays - P * args.spp if mode == L.MODE_AO else hit_px * args.spp
-    # a stored node is 64 bytes, a leaf pair's two spheres 32, a leaf child's sphere 16; shading
-    # reads each hit sphere (16) and the frame writes 32 bytes per pixel
-    algo_bytes = (64 * (visits - pair_visits) + 32 * pair_visits + 16 * leaf_fetches
-                  + 16 * max(hit_samples, 0) + 32 * P)
+    # a stored node is 64 bytes, a leaf reference's two spheres 32; shading reads each hit sphere (16)
+    # and the frame writes 32 bytes per pixel
+    algo_bytes = 64 * (visits - pair_visits) + 32 * pair_visits + 16 * max(hit_samples, 0) + 32 * P
     achieved = algo_bytes / (trace_ms * 1e-3) / 1e9
     kernel_name = trace_kernel_label(r, args.spp, args.mode)
     traffic = (dram_traffic(f"cells {args.cells}, {args.width}x{args.height}, spp {args.spp}, mode {args.mode}")
                if args.config == "fcc" else None)
     mrays = rays / (ms * 1e-3) / 1e6
-    log(f"visits {visits} (leaf pairs {pair_visits}) tests {tests} leaf fetches {leaf_fetches} rays {rays} "
+    log(f"visits {visits} (leaf pairs {pair_visits}) tests {tests} rays {rays} "
         f"overflow {overflow} hit px {hit_px}")
     split = None
     if mode == L.MODE_AO:

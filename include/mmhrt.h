@@ -270,7 +270,7 @@ MMHRT_API int32_t mmhrt_get_timings(mmhrt_ctx ctx, float* times_ms, int32_t n);
  * "count_visits"): node visits, sphere tests, rays traced. Also refreshes the options
  * "stack_overflow" (1 if a traversal stack ever exceeded its capacity; 0 expected),
  * "pair_visits" (the node visits that were leaf references: two 16-byte spheres read instead of a
- * 64-byte node) and "leaf_fetches" (spheres read apart from visits: none by the current kernels).
+ * 64-byte node) and "leaf_fetches" (spheres read apart from visits: always 0).
  * A visit that a whole wavefront makes together is counted once per active lane. */
 MMHRT_API int32_t mmhrt_get_counters(mmhrt_ctx ctx, uint64_t* node_visits, uint64_t* sphere_tests, uint64_t* rays);
 
@@ -359,7 +359,7 @@ MMHRT_API int32_t mmhrt_denoiser_train_step(mmhrt_ctx ctx, const uint16_t* feats
  * "fail_alloc" (test hook: the k-th device allocation from now fails with MMHRT_E_OOM, as a real
  * failure would, and the option returns to 0; 0, the default, injects nothing).
  * Diagnostics: "count_visits" (0/1) and, read-only in effect, "stack_overflow", "pair_visits",
- * "leaf_fetches" (refreshed by mmhrt_get_counters), "sort_fault", and "leaf_pair_count" (get
+ * "leaf_fetches" (refreshed by mmhrt_get_counters), "used_sort_ri" and "used_build_span", "sort_fault", and "leaf_pair_count" (get
  * only: the leaf pairs of the current tree, counted on the device from its sorted keys). */
 MMHRT_API int32_t mmhrt_set_option(mmhrt_ctx ctx, const char* key, int64_t value);
 MMHRT_API int32_t mmhrt_get_option(mmhrt_ctx ctx, const char* key, int64_t* value);

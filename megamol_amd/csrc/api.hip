@@ -704,7 +704,6 @@ int32_t mmhrt_get_counters(mmhrt_ctx c, uint64_t* visits, uint64_t* tests, uint6
     if (rays) *rays = r;
     c->stack_overflow = h[1];
     memcpy(&c->pair_visits, h + 8, 8);
-    memcpy(&c->leaf_fetches, h + 10, 8);
     return MMHRT_OK;
 }
 

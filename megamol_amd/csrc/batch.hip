@@ -276,7 +276,7 @@ int32_t mmhrt_render_batch(mmhrt_ctx c, const mmhrt_job* jobs, uint32_t n_jobs, 
     if ((e = tl ? build_pkd(c, morton_bits, true) : build_lbvh(c, morton_bits, true))) return e;
     {
         unsigned grid = (unsigned)std::max<int64_t>(1, c->cu_count * c->opt_blocks_per_cu);
-        if ((e = ensure(c, c->spill, (size_t)grid * 256 * 120, "traversal spill"))) return e;
+        if ((e = ensure(c, c->spill, (size_t)grid * 256 * TRACE_SPILL_PER_LANE, "traversal spill"))) return e;
     }
     // One launch reads every timestep's structure, so each timestep but the last builds into a
     // slot of its own (the last one into the context's buffers), and each rebuild but the last

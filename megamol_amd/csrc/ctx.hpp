@@ -167,7 +167,7 @@ struct mmhrt_ctx_s {
     int64_t refits_since_build = 0;
     int64_t stack_overflow = 0;  // set by mmhrt_get_counters from the trace kernel's flag
     int64_t pair_visits = 0;     // set by mmhrt_get_counters: visits of leaf pairs (of the node visits)
-    int64_t leaf_fetches = 0;    // set by mmhrt_get_counters: sphere loads of leaf children of stored nodes
+    int64_t leaf_fetches = 0;    // option kept for callers: no kernel reads spheres apart from its visits
 
     // batched time series: all timesteps resident, one hipGraph for the whole sequence
     mmhrt::DevBuf<float4> ts_sph;      // timesteps x n spheres
@@ -281,7 +281,7 @@ int build_pkd(mmhrt_ctx_s* c, int bits, bool reserve_only = false);
 constexpr int TRACE_SPILL_PER_LANE = 120;
 constexpr uint32_t TRACE_QUEUE = 32;                       // first word of the 8 work queue counters
 constexpr uint32_t TRACE_QUEUE_STRIDE = 32;                // words between them (a cache line each)
-constexpr uint32_t TRACE_CTR_WORDS = TRACE_QUEUE + 8 * TRACE_QUEUE_STRIDE;  // overflow flag, 5 u64 counters, queues
+constexpr uint32_t TRACE_CTR_WORDS = TRACE_QUEUE + 8 * TRACE_QUEUE_STRIDE;  // overflow flag, 4 u64 counters, queues
 struct FrameOutputs {
     float4* color;
     float* depth;

@@ -1877,18 +1877,18 @@ int morton_sort_t(mmhrt_ctx_s* c, K* ka, K* kb, uint32_t* va, uint32_t* vb, uint
         } else {
             hipLaunchKernelGGL(k_col_sums, dim3(groups, ND / 256), dim3(256), 0, c->stream, hist, tiles,
                                c->scan_tmp.p, (uint32_t)ND);
-        }
-        if (ND == 256 && tiles <= COL_FEW) {
-        } else if (ND == 256) {
-            hipLaunchKernelGGL(k_col_scan, dim3(4), dim3(1024), 0, c->stream, c->scan_tmp.p, groups);
-            hipLaunchKernelGGL(k_col_offsets<true>, dim3(groups), dim3(256), 0, c->stream, hist, tiles, groups,
-                               c->scan_tmp.p, offs, (uint32_t)ND);
-        } else {
-            hipLaunchKernelGGL(k_col_top, dim3(ND / 256), dim3(256), 0, c->stream, c->scan_tmp.p, groups,
-                               (uint32_t)ND);
-            hipLaunchKernelGGL(k_col_digits, dim3(1), dim3(256), 0, c->stream, c->scan_tmp.p, groups, (uint32_t)ND);
-            hipLaunchKernelGGL(k_col_offsets<false>, dim3(groups, ND / 256), dim3(256), 0, c->stream, hist, tiles,
-                               groups, c->scan_tmp.p, offs, (uint32_t)ND);
+            if (ND == 256) {
+                hipLaunchKernelGGL(k_col_scan, dim3(4), dim3(1024), 0, c->stream, c->scan_tmp.p, groups);
+                hipLaunchKernelGGL(k_col_offsets<true>, dim3(groups), dim3(256), 0, c->stream, hist, tiles, groups,
+                                   c->scan_tmp.p, offs, (uint32_t)ND);
+            } else {
+                hipLaunchKernelGGL(k_col_top, dim3(ND / 256), dim3(256), 0, c->stream, c->scan_tmp.p, groups,
+                                   (uint32_t)ND);
+                hipLaunchKernelGGL(k_col_digits, dim3(1), dim3(256), 0, c->stream, c->scan_tmp.p, groups,
+                                   (uint32_t)ND);
+                hipLaunchKernelGGL(k_col_offsets<false>, dim3(groups, ND / 256), dim3(256), 0, c->stream, hist, tiles,
+                                   groups, c->scan_tmp.p, offs, (uint32_t)ND);
+            }
         }
         const bool xcd = c->opt_sort_xcd != 0;
         hipLaunchKernelGGL((k_radix_scatter<K, RI, DB>), dim3(xcd ? 8 * ((tiles + 7) / 8) : tiles), dim3(RB), 0,

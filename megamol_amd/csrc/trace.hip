@@ -34,7 +34,7 @@ struct TraceArgs {
     const SceneInfo* info;
     int32_t* spill;
     uint32_t spill_stride;  // lanes in the grid
-    uint32_t* ctr;          // [1] overflow flag, [2..11] u64 counters, from TRACE_QUEUE on the work queues
+    uint32_t* ctr;          // [1] overflow flag, [2..9] u64 counters, from TRACE_QUEUE on the work queues
     uint32_t n_tiles, tiles_x;
     uint32_t sub_log2;      // k_trace_sl: a unit of work is 1 / (1 << sub_log2) of a tile's passes
     uint32_t tw_log2;  // pixel tile = (1 << tw_log2) x (64 >> tw_log2), one wavefront
@@ -228,7 +228,7 @@ __device__ __forceinline__ float slab(const RayPre& r, float lx, float ly, float
 }
 
 struct Count {
-    uint64_t visits = 0, tests = 0, rays = 0, pair_visits = 0, leaf_fetches = 0;
+    uint64_t visits = 0, tests = 0, rays = 0, pair_visits = 0;
 };
 
 // Traversal of the LBVH by one lane, in two alternating phases. The inner phase visits stored
@@ -991,7 +991,6 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(W, 8))) void
         atomicAdd(reinterpret_cast<unsigned long long*>(A.ctr + 4), (unsigned long long)cnt.tests);
         atomicAdd(reinterpret_cast<unsigned long long*>(A.ctr + 6), (unsigned long long)cnt.rays);
         atomicAdd(reinterpret_cast<unsigned long long*>(A.ctr + 8), (unsigned long long)cnt.pair_visits);
-        atomicAdd(reinterpret_cast<unsigned long long*>(A.ctr + 10), (unsigned long long)cnt.leaf_fetches);
     }
 }
 
@@ -1174,7 +1173,6 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(TL ? 5 : 7, 
         atomicAdd(reinterpret_cast<unsigned long long*>(A.ctr + 4), (unsigned long long)cnt.tests);
         atomicAdd(reinterpret_cast<unsigned long long*>(A.ctr + 6), (unsigned long long)cnt.rays);
         atomicAdd(reinterpret_cast<unsigned long long*>(A.ctr + 8), (unsigned long long)cnt.pair_visits);
-        atomicAdd(reinterpret_cast<unsigned long long*>(A.ctr + 10), (unsigned long long)cnt.leaf_fetches);
     }
 }
 
@@ -1362,7 +1360,6 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(5, 8))) void
         atomicAdd(reinterpret_cast<unsigned long long*>(A.ctr + 4), (unsigned long long)cnt.tests);
         atomicAdd(reinterpret_cast<unsigned long long*>(A.ctr + 6), (unsigned long long)cnt.rays);
         atomicAdd(reinterpret_cast<unsigned long long*>(A.ctr + 8), (unsigned long long)cnt.pair_visits);
-        atomicAdd(reinterpret_cast<unsigned long long*>(A.ctr + 10), (unsigned long long)cnt.leaf_fetches);
     }
 }
 
@@ -1774,7 +1771,7 @@ int render_frame(mmhrt_ctx_s* c, const FrameConsts& fc) {
 
 // The frame into the given device outputs: the persistent grid is capped at `lanes`, whose
 // traversal stacks spill into `spill` (lanes x TRACE_SPILL_PER_LANE words, lane-interleaved);
-// `ctr` (TRACE_CTR_WORDS words) takes the tile counter, the overflow flag and the instrumentation
+// `ctr` (TRACE_CTR_WORDS words) takes the overflow flag, the instrumentation counters and the work queues'
 // counters and is cleared here by a fill kernel (safe under graph capture). `order` (two words per
 // tile, or null) takes the order of a treelet frame's tiles. Allocates nothing.
 int render_frame_into(mmhrt_ctx_s* c, const FrameConsts& fc, const FrameOutputs& out, uint32_t* ctr, int32_t* spill,
