@@ -953,7 +953,7 @@ __device__ void shade_pixel(const TraceArgs& A, uint32_t px, uint32_t py, float 
 // 801x600, 1 sample) went from 1.65 to 0.71 ms, with the work queues to 0.61 ms. At 1 sample it now
 // beats the refill kernel, which had been the default there (50M spheres, 1080p AO: 0.88 against 0.70
 // ms; 60M clustered at 4K: 6.7 against 5.7; 10k spheres at 320x240: 92 against 80 us): bound by the
-// vector memory unit's address rate (busy 60-90 %), then by VALU issue (50-70 %).
+// vector memory unit's address rate (busy 43-81 % of the time) and by lanes that wait (23-41 % active).
 // Small frames (W = 5) are held to 102 VGPRs, with hardly a spill: their wavefronts have one or two tiles
 // each and the longest rays are the kernel's time. One sample, W = 5 against 7 at 0.2 to 3.5 tiles per
 // wavefront (5 scenes of 100k to 4M spheres, uniform, FCC and clusters; Lambert, AO, 1, 4 and 8 bounces): up to
